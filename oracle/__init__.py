@@ -33,8 +33,8 @@ REF_TREE = Path("/root/reference")
 
 def build() -> Path:
     subprocess.run(["make", "-s", "-C", str(HERE)], check=True)
-    # the reference's own OBJ loader, when its tree is here (oracle/_ref)
-    if REF_TREE.exists():
+    # the reference's own OBJ loader and SAH builder, when its tree is here (oracle/_ref)
+    if (REF_TREE / "src" / "rt" / "obj-loader.cpp").exists():
         subprocess.run(["make", "-s", "-C", str(HERE), "-f", "Makefile.ref", f"REF={REF_TREE}"], check=True,
                        capture_output=True)
     return LIB
