@@ -22,20 +22,18 @@ constexpr int BS = 256;
 constexpr int SORT_ITEMS = 16;               // the smallest tile (sizes the look-back words)
 constexpr int SORT_TILE = BS * SORT_ITEMS;
 constexpr int BOUNDS_GRID = 512;
-constexpr uint32_t FAT_LEAF = 16;
-constexpr int HIER_TOP = 8;    // levels 0..8 (<= 256 nodes) emitted by one block
-constexpr int REFIT_TOP = 10;  // levels 10..0 (<= 1024 nodes) refit by one block
+constexpr int TREE_TILE = 1024;              // tree phase: sorted positions per tile
+constexpr uint32_t NONE = 0xffffffffu;
 
 // Counter slots in scene->tickets.
 constexpr int TK_BOUNDS = 0;
 constexpr int TK_SORT = 1;    // up to 8 passes (4-bit digits)
-constexpr int TK_LEVEL = 16;  // up to 64 levels
+constexpr int TK_RANK = 16;
 constexpr int TK_COUNT = 80;
 
 // Layout of scene->levels (uint32): [d] = first node of level d,
 // [64 + d] = node count of level d, [128] = total node count.
-// [129] = number of fat leaves (more than FAT_LEAF triangles) in scene->fat.
-constexpr int LV_OFF = 0, LV_CNT = 64, LV_TOTAL = 128, LV_FAT = 129, LV_WORDS = 192;
+constexpr int LV_OFF = 0, LV_CNT = 64, LV_TOTAL = 128, LV_WORDS = 192;
 
 // ------------------------------------------------------------- helpers --
 __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t x, uint32_t lane) {
@@ -66,24 +64,21 @@ __device__ __forceinline__ uint32_t block_excl_scan(uint32_t x, uint32_t* s_w, u
 
 // -------------------------------------------------------------- kernels --
 __global__ __launch_bounds__(BS) void k_build_init(uint32_t* zero_a, uint32_t na, uint32_t* zero_b, uint32_t nb,
-                                                   uint32_t* zero_c, uint32_t nc, uint32_t* levels, uint32_t* bstart,
-                                                   uint32_t* bend, uint32_t* parent, uint32_t T, int set_root) {
+                                                   uint32_t* zero_c, uint32_t nc, uint32_t* zero_d, uint32_t nd,
+                                                   uint32_t* levels, uint32_t* parent) {
     uint32_t stride = gridDim.x * BS;
     for (uint32_t i = blockIdx.x * BS + threadIdx.x; i < na; i += stride) zero_a[i] = 0;
     for (uint32_t i = blockIdx.x * BS + threadIdx.x; i < nb; i += stride) zero_b[i] = 0;
     for (uint32_t i = blockIdx.x * BS + threadIdx.x; i < nc; i += stride) zero_c[i] = 0;
-    if (set_root && blockIdx.x == 0) {
+    for (uint32_t i = blockIdx.x * BS + threadIdx.x; i < nd; i += stride) zero_d[i] = 0;
+    if (blockIdx.x == 0) {
         // every word is written once, by one thread, with its final value:
         // the root's count and the node total are 1, the rest 0 (a zeroing
         // pass followed by a store of the root words from another wave would
         // race with it)
         for (uint32_t i = threadIdx.x; i < LV_WORDS; i += BS)
             levels[i] = (i == (uint32_t)(LV_CNT + 0) || i == (uint32_t)LV_TOTAL) ? 1u : 0u;
-        if (threadIdx.x == 0) {
-            bstart[0] = 0;
-            bend[0] = T;
-            parent[0] = 0;
-        }
+        if (threadIdx.x == 0) parent[0] = 0;
     }
 }
 
@@ -373,8 +368,8 @@ __global__ __launch_bounds__(BS) void k_rearrange(const uint32_t* __restrict__ p
     tri[3 * (size_t)i + 2] = make_float4(pc.x, pc.y, pc.z, __uint_as_float(c));
 }
 
-// Triangle records from the current index buffer, identity order (refit
-// path, Q14 of src/rt/bvh-builder.cpp:779-817).
+// Triangle records from the current index buffer, identity order (the SAH
+// build).
 __global__ __launch_bounds__(BS) void k_tri_records(const uint32_t* __restrict__ idx, const float4* __restrict__ pos,
                                                     float4* __restrict__ tri, uint32_t T) {
     uint32_t i = blockIdx.x * BS + threadIdx.x;
@@ -387,312 +382,536 @@ __global__ __launch_bounds__(BS) void k_tri_records(const uint32_t* __restrict__
     }
 }
 
-// One iteration of process_task (src/kernel/bvh-builder.cl:582-671) over the
-// nodes of level d, in order.  Children of the k-th splitting node of the
-// level go to off_next + 2k (ordered compaction by decoupled look-back),
-// which is the order in-order work-groups of the reference produce.
-// Binary radix tree over the sorted codes (Karras 2012, "Maximizing
-// parallelism in the construction of BVHs, octrees and k-d trees"), keys
-// made unique by their position.  For internal node i it stores the other
-// end j of its range and the split gamma (left = [min, gamma], right =
-// [gamma+1, max]).  The reference splits a range [s, e) with differing end
-// codes at the highest differing bit, at the first index with that bit set
-// (find_middle, src/kernel/bvh-builder.cl:484-552): the same split as the
-// radix-tree node whose range is [s, e-1], and that node's index is s or e-1.
-__device__ __forceinline__ int rt_delta(const uint32_t* __restrict__ codes, int T, int i, int j) {
-    if (j < 0 || j >= T) return -1;
-    const uint32_t x = codes[i] ^ codes[j];
-    return x ? __builtin_clz(x) : 32 + __builtin_clz((uint32_t)(i ^ j));
+// ------------------------------------------------------------ tree phase --
+// The reference splits a range [l, r] of sorted positions whose first and
+// last codes differ, and which holds more than min_leaf + 2 triangles, at the
+// highest differing bit, after the last position s without that bit
+// (find_middle, src/kernel/bvh-builder.cl:484-552), and numbers the children
+// level by level in the order of their parents (process_task, :582-671).
+// Instead of one launch per level, every inner node is found by its split s,
+// which no other node shares:
+//   its range is that of the codes that agree with code[s] above the bit in
+//     which code[s] and code[s + 1] differ (k_spans);
+//   its parent is the split at l - 1 or at r, whichever's codes agree in more
+//     bits, and its level the number of its ancestors, from bit masks that a
+//     scan carries (k_spans);
+//   the nodes of one level lie in the order of their splits, so its rank among
+//     all inner nodes in (level, split) order, a stable counting sort by level,
+//     gives its children's numbers 1 + 2 rank and 2 + 2 rank (k_ranks), and
+//     with its parent's rank its own;
+//   the box of a node is the union of the triangle boxes of its range, in
+//     any order (k_boxes, k_cross).
+// A build was bound by its launches (55, a few microseconds each) and, when
+// large, by the chains of dependent reads in each level's tiles; now it has 16
+// launches and no chain longer than one search.  Whole builds, back to back,
+// before and now: 65k triangles 258 and 116 us, 8M triangles 2197 and 1601 us;
+// refit of 1M 145 and 111 us.
+
+// Split s of the nodes: {l, r, flags | level << 2, -}, then (k_boxes) {l, r,
+// node, children}.  Flags: bit 0 the left child is a leaf, bit 1 the right.
+constexpr uint32_t SPAN_LEFT = 0x40000000u, SPAN_RIGHT = 0x80000000u, SPAN_NUM = 0x3fffffffu;
+
+// Ancestors as masks.  D(k) is the number of leading bits in which code[k] and
+// code[k + 1] agree.  Split k is an ancestor of split s iff D(k) is below every
+// D from s up to k, and the ancestors of a node have different D, so the
+// level is the number of bits of two masks: the D that are new minima walking
+// left from s, and walking right, below D(s).  Appending a D to a walk drops the
+// mask's bits from D up and sets bit D; such maps compose to maps of the same
+// form (min, mask), so one scan per direction gives every split's masks.
+struct Walk {
+    uint32_t least, mask;  // least D met (32: none), new minima
+};
+__device__ __forceinline__ uint32_t bits_below(uint32_t n) { return n >= 32u ? 0xffffffffu : (1u << n) - 1u; }
+// The walk over `far`, then the nearer `near`.
+__device__ __forceinline__ Walk walk_on(Walk far, Walk near) {
+    return Walk{far.least < near.least ? far.least : near.least, (far.mask & bits_below(near.least)) | near.mask};
 }
 
-__global__ __launch_bounds__(BS) void k_radix_tree(const uint32_t* __restrict__ codes, uint32_t* __restrict__ kj,
-                                                   uint32_t* __restrict__ kg, int T) {
-    const int i = (int)(blockIdx.x * BS + threadIdx.x);
-    if (i >= T - 1) return;
-    const int d = rt_delta(codes, T, i, i + 1) - rt_delta(codes, T, i, i - 1) > 0 ? 1 : -1;
-    const int dmin = rt_delta(codes, T, i, i - d);
-    int lmax = 2;
-    while (rt_delta(codes, T, i, i + lmax * d) > dmin) lmax <<= 1;
-    int l = 0;
-    for (int t = lmax >> 1; t >= 1; t >>= 1)
-        if (rt_delta(codes, T, i, i + (l + t) * d) > dmin) l += t;
-    const int j = i + l * d;
-    const int dnode = rt_delta(codes, T, i, j);
-    int sp = 0;
-    for (int t = l;;) {
-        t = (t + 1) >> 1;
-        if (rt_delta(codes, T, i, i + (sp + t) * d) > dnode) sp += t;
-        if (t <= 1) break;
+// First position of [0, at] with a code >= want, given codes[at] >= want: four
+// ways a step, so the chain of dependent reads is log4 of the range.
+__device__ __forceinline__ int first_from(const uint32_t* __restrict__ codes, int at, uint32_t want) {
+    int lo = -1, hi = at;  // codes[lo] < want <= codes[hi]
+    while (hi - lo > 1) {
+        const int q = (hi - lo) >> 2, m1 = lo + (q ? q : 1), m2 = lo + ((hi - lo) >> 1), m3 = hi - (q ? q : 1);
+        const bool g1 = codes[m1] >= want, g2 = codes[m2] >= want, g3 = codes[m3] >= want;
+        const int l = g1 ? lo : (g2 ? m1 : (g3 ? m2 : m3));
+        hi = g1 ? m1 : (g2 ? m2 : (g3 ? m3 : hi));
+        lo = l;
     }
-    const int gamma = i + sp * d + (d < 0 ? -1 : 0);
-    kj[i] = (uint32_t)j;
-    kg[i] = (uint32_t)gamma;
+    return hi;
+}
+// Last position of [at, T) with a code <= want, given codes[at] <= want.
+__device__ __forceinline__ int last_up_to(const uint32_t* __restrict__ codes, int at, int T, uint32_t want) {
+    int lo = at, hi = T;  // codes[lo] <= want < codes[hi]
+    while (hi - lo > 1) {
+        const int q = (hi - lo) >> 2, m1 = lo + (q ? q : 1), m2 = lo + ((hi - lo) >> 1), m3 = hi - (q ? q : 1);
+        const bool g1 = codes[m1] > want, g2 = codes[m2] > want, g3 = codes[m3] > want;
+        const int l = g1 ? lo : (g2 ? m1 : (g3 ? m2 : m3));
+        hi = g1 ? m1 : (g2 ? m2 : (g3 ? m3 : hi));
+        lo = l;
+    }
+    return lo;
 }
 
-// build_leaf_bbox (src/kernel/bvh-builder.cl:262-288) for a leaf of at most
-// FAT_LEAF triangles, by one thread: the vertices of four triangles are
-// loaded before any is folded in (a short leaf costs a few memory round
-// trips, not one per vertex).  Min/max is exact in any order.
-__device__ __forceinline__ void leaf_bounds(const float4* __restrict__ tri, float4* __restrict__ node, uint32_t n,
-                                            uint32_t a, uint32_t cnt) {
-    v3 lo = xyz(tri[3 * (size_t)a]), hi = lo;
-    const uint32_t end = a + cnt;
-    for (uint32_t t = a; t < end; t += 4) {
-        float4 p[12];
-#pragma unroll
-        for (int q = 0; q < 12; ++q) {
-            const uint32_t tq = t + (uint32_t)(q / 3) < end ? t + (uint32_t)(q / 3) : a;
-            p[q] = tri[3 * (size_t)tq + (q % 3)];
+// Ranges, child kinds, parents and levels; one split per thread.  The codes of
+// the tile are in LDS, where a range's ends are found in doubling steps from
+// its split.  A range that leaves the tile contains the tile's first or last
+// code, so its end there depends only on how many leading bits it shares with
+// that code: 33 values per edge, found by 33 lanes side by side, the only
+// searches in global memory (their chain of dependent reads bounds small
+// builds).  The edge's walk mask has the bits where two neighbouring values
+// differ, and the parent is on the side whose walk has the larger D below
+// the node's own.
+__global__ __launch_bounds__(TREE_TILE) void k_spans(const uint32_t* __restrict__ codes, uint4* __restrict__ span,
+                                                     uint32_t* __restrict__ par, uint32_t* __restrict__ level, int T,
+                                                     uint32_t min_leaf) {
+    constexpr int WAVES = TREE_TILE / RTX_WAVE;
+    __shared__ uint32_t s_c[TREE_TILE + 1];
+    __shared__ Walk s_w[2][WAVES];
+    __shared__ int s_end[2][33];
+    __shared__ uint32_t s_edge[2];
+    const int tid = (int)threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int base = (int)blockIdx.x * TREE_TILE, s = base + tid;
+    const int last = base + TREE_TILE <= T ? base + TREE_TILE - 1 : T - 1;
+    s_c[tid] = s < T ? codes[s] : 0u;
+    if (tid == 0) s_c[TREE_TILE] = base + TREE_TILE < T ? codes[base + TREE_TILE] : 0u;
+    __syncthreads();
+    if (w < 2) {
+        int end = 0;
+        if (lane < 33) {
+            const uint32_t rest = lane == 32 ? 0u : 0xffffffffu >> lane;  // the bits not shared
+            end = w == 0 ? first_from(codes, base, s_c[0] & ~rest)
+                         : last_up_to(codes, last, T, s_c[last - base] | rest);
+            s_end[w][lane] = end;
         }
-#pragma unroll
-        for (int q = 0; q < 12; ++q) {
-            lo = vmin(lo, xyz(p[q]));
-            hi = vmax(hi, xyz(p[q]));
+        const int next = __shfl_down(end, 1, RTX_WAVE);
+        const uint32_t m = (uint32_t)ballot(lane < 32 && next != end);
+        if (lane == 0) s_edge[w] = m;
+    }
+    const bool pair = s < T - 1;
+    const uint32_t c0 = s_c[tid], c1 = pair ? s_c[tid + 1] : c0, x = c0 ^ c1;
+    const uint32_t D = x ? (uint32_t)__builtin_clz(x) : 32u;
+    // scans: the walk over the wave's splits left of this one (up), right of it
+    // (down; the tile's last split counts as beyond the edge)
+    Walk up{D, x ? 1u << D : 0u}, down = s < last ? up : Walk{32u, 0u};
+    for (int off = 1; off < RTX_WAVE; off <<= 1) {
+        const Walk u{(uint32_t)__shfl_up((int)up.least, off, RTX_WAVE), (uint32_t)__shfl_up((int)up.mask, off, RTX_WAVE)};
+        const Walk v{(uint32_t)__shfl_down((int)down.least, off, RTX_WAVE),
+                     (uint32_t)__shfl_down((int)down.mask, off, RTX_WAVE)};
+        if (lane >= off) up = walk_on(u, up);
+        if (lane + off < RTX_WAVE) down = walk_on(v, down);
+    }
+    if (lane == 63) s_w[0][w] = up;
+    if (lane == 0) s_w[1][w] = down;
+    up = Walk{(uint32_t)__shfl_up((int)up.least, 1, RTX_WAVE), (uint32_t)__shfl_up((int)up.mask, 1, RTX_WAVE)};
+    down = Walk{(uint32_t)__shfl_down((int)down.least, 1, RTX_WAVE), (uint32_t)__shfl_down((int)down.mask, 1, RTX_WAVE)};
+    if (lane == 0) up = Walk{32u, 0u};
+    if (lane == 63) down = Walk{32u, 0u};
+    // the range inside the tile
+    const uint32_t rest = 0xffffffffu >> (D & 31u), low = c0 & ~rest, high = c0 | rest;
+    int l = tid, r = tid + 1;
+    if (x) {
+        int st = 1;
+        while (l - st >= 0 && s_c[l - st] >= low) {
+            l -= st;
+            st <<= 1;
+        }
+        for (st >>= 1; st; st >>= 1)
+            if (l - st >= 0 && s_c[l - st] >= low) l -= st;
+        st = 1;
+        const int n = last - base + 1;
+        while (r + st < n && s_c[r + st] <= high) {
+            r += st;
+            st <<= 1;
+        }
+        for (st >>= 1; st; st >>= 1)
+            if (r + st < n && s_c[r + st] <= high) r += st;
+    }
+    __syncthreads();
+    if (s >= T) return;
+    uint32_t p = NONE, n = NONE;
+    if (x) {
+        l = l == 0 ? s_end[0][D] : base + l;
+        r = r >= last - base ? s_end[1][D] : base + r;
+        // inner: more than min_leaf + 2 triangles (the codes differ by construction)
+        if ((uint32_t)(r - l + 1) - 2u > min_leaf) {
+            // all codes of a child equal: within the tile its end codes, beyond it
+            // the run of the edge's code
+            const bool same_l = l >= base ? s_c[l - base] == c0 : (s_c[0] == c0 && s_end[0][32] <= l);
+            const bool same_r = r <= last   ? s_c[r - base] == c1
+                                : s == last ? codes[r] == c1
+                                            : (s_c[last - base] == c1 && s_end[1][32] >= r);
+            const bool leaf_l = !((uint32_t)(s - l + 1) - 2u > min_leaf && !same_l);
+            const bool leaf_r = !((uint32_t)(r - s) - 2u > min_leaf && !same_r);
+            Walk wl{32u, s_edge[0]}, wr{32u, s_edge[1]};
+            for (int k = 0; k < w; ++k) wl = walk_on(wl, s_w[0][k]);
+            for (int k = WAVES - 1; k > w; --k) wr = walk_on(wr, s_w[1][k]);
+            const uint32_t ml = walk_on(wl, up).mask & bits_below(D), mr = walk_on(wr, down).mask & bits_below(D);
+            p = (ml | mr) == 0u ? (uint32_t)s : (ml > mr ? (uint32_t)(l - 1) : (uint32_t)r);  // the root: itself
+            n = (uint32_t)__builtin_popcount(ml | mr);
+            span[s] = make_uint4((uint32_t)l, (uint32_t)r, (leaf_l ? 1u : 0u) | (leaf_r ? 2u : 0u) | (n << 2), 0u);
         }
     }
-    node[2 * (size_t)n] = make_float4(lo.x, lo.y, lo.z, __uint_as_float(a));
-    node[2 * (size_t)n + 1] = make_float4(hi.x, hi.y, hi.z, __uint_as_float(cnt));
+    par[s] = p;
+    level[s] = n;
 }
 
-// Leaves of more than FAT_LEAF triangles (long runs of equal codes, up to
-// hundreds of triangles) are listed during emission and bounded here, one
-// wave per leaf, every lane folding four vertices per round.
-__global__ __launch_bounds__(BS) void k_fat_leaves(const float4* __restrict__ tri, float4* __restrict__ node,
-                                                   const uint32_t* __restrict__ fat, const uint32_t* __restrict__ levels) {
-    const uint32_t nfat = levels[LV_FAT];
-    const uint32_t lane = threadIdx.x & 63;
-    const uint32_t wpb = BS / RTX_WAVE;
-    for (uint32_t i = blockIdx.x * wpb + (threadIdx.x >> 6); i < nfat; i += gridDim.x * wpb) {
-        const uint32_t n = fat[i];
-        const uint32_t a = __float_as_uint(node[2 * (size_t)n].w), cnt = __float_as_uint(node[2 * (size_t)n + 1].w);
-        const size_t v0 = 3 * (size_t)a, v1 = 3 * (size_t)(a + cnt);
-        float q[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
-        for (size_t v = v0 + lane; v < v1; v += 4 * RTX_WAVE) {
-            float4 p[4];
+// The rank of every split among those of its level (the level in `rel` is
+// replaced by it): in-tile by wave ballots, across tiles by one look-back per
+// level, as a radix-sort pass ranks digits.  The last tile writes the level
+// table.
+template <int RANK_ITEMS>
+__global__ __launch_bounds__(BS) void k_ranks(uint32_t* __restrict__ rel, uint32_t* status, uint32_t* ticket,
+                                              uint32_t* __restrict__ levels, uint32_t T, uint32_t ntiles) {
+    __shared__ uint32_t s_wcnt[BS / RTX_WAVE][64];
+    __shared__ uint32_t s_pref[64];
+    __shared__ uint32_t s_tile;
+    const uint32_t tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    if (tid == 0) s_tile = atomicAdd(ticket, 1u);
+    s_wcnt[w][lane] = 0;
+    __syncthreads();
+    const uint32_t tile = s_tile, base = tile * (BS * RANK_ITEMS);
+    uint32_t d[RANK_ITEMS], r[RANK_ITEMS];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) p[j] = tri[v + j * RTX_WAVE < v1 ? v + j * RTX_WAVE : v];
+    for (int j = 0; j < RANK_ITEMS; ++j) {
+        const uint32_t s = base + (w * RANK_ITEMS + j) * RTX_WAVE + lane;
+        d[j] = s < T ? rel[s] : NONE;
+    }
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                q[0] = fminf(q[0], p[j].x); q[1] = fminf(q[1], p[j].y); q[2] = fminf(q[2], p[j].z);
-                q[3] = fmaxf(q[3], p[j].x); q[4] = fmaxf(q[4], p[j].y); q[5] = fmaxf(q[5], p[j].z);
+    for (int j = 0; j < RANK_ITEMS; ++j) {
+        const bool ok = d[j] != NONE;
+        uint64_t peers = ballot(ok);
+#pragma unroll
+        for (int b = 0; b < 6; ++b) {
+            const bool bit = (d[j] >> b) & 1u;
+            const uint64_t bal = ballot(bit);
+            peers &= bit ? bal : ~bal;
+        }
+        const uint32_t below = lanes_below(peers);
+        const uint32_t basec = ok ? s_wcnt[w][d[j]] : 0u;
+        r[j] = basec + below;
+        if (ok && below == 0) s_wcnt[w][d[j]] = basec + (uint32_t)__builtin_popcountll(peers);
+    }
+    __syncthreads();
+    if (tid < 64) {
+        uint32_t tot = 0;
+#pragma unroll
+        for (int i = 0; i < BS / RTX_WAVE; ++i) {
+            const uint32_t c = s_wcnt[i][tid];
+            s_wcnt[i][tid] = tot;
+            tot += c;
+        }
+        const uint32_t prefix = lookback_thread(status + tid, tile, tot, 64u);
+        s_pref[tid] = prefix;
+        if (tile == ntiles - 1) {
+            const uint32_t all = prefix + tot, inc = wave_incl_scan(all, tid);
+            if (tid < 63) {
+                levels[LV_OFF + tid + 1] = 1u + 2u * (inc - all);
+                levels[LV_CNT + tid + 1] = 2u * all;
+            } else {
+                levels[LV_TOTAL] = 1u + 2u * inc;
             }
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < RANK_ITEMS; ++j) {
+        const uint32_t s = base + (w * RANK_ITEMS + j) * RTX_WAVE + lane;
+        if (d[j] != NONE) rel[s] = s_pref[d[j]] + s_wcnt[w][d[j]] + r[j];
+    }
+}
+
+// Triangles from which the ranks use tiles of 4096 splits instead of 1024: the
+// look-back over many tiles then costs more than a tile's longer ranking (8M
+// splits 55 against 113 us; at 65k the short tiles take 6.3 us).
+constexpr uint32_t RANK_WIDE = 1u << 19;
+
+struct Box {
+    v3 lo, hi;
+};
+// NaN is the identity: min and max drop it.
+__device__ __forceinline__ Box no_box() {
+    const float n = __builtin_nanf("");
+    return Box{mk3(n, n, n), mk3(n, n, n)};
+}
+__device__ __forceinline__ Box join(const Box& a, const Box& b) { return Box{vmin(a.lo, b.lo), vmax(a.hi, b.hi)}; }
+__device__ __forceinline__ void put_node(float4* __restrict__ node, uint32_t n, const Box& b, uint32_t w0,
+                                         uint32_t w1) {
+    node[2 * (size_t)n] = make_float4(b.lo.x, b.lo.y, b.lo.z, __uint_as_float(w0));
+    node[2 * (size_t)n + 1] = make_float4(b.hi.x, b.hi.y, b.hi.z, __uint_as_float(w1));
+}
+
+// What k_boxes leaves for the ranges that cross tiles (at most 32 nested
+// nodes cross one tile edge): per tile its box, and the boxes of its ends that
+// such a range takes from it, by their first or last position.
+constexpr uint32_t TILE_ENDS = 32;
+struct TreeTiles {
+    float4* box;      // 2 per tile: {lo, number of tails}{hi, number of heads}
+    float4* tails;    // TILE_ENDS x 2 per tile: {lo, first position}{hi, -}: that position to the tile's end
+    float4* heads;    // TILE_ENDS x 2 per tile: the tile's start to that position
+    uint4* cross;     // TILE_CROSS per tile: crossing nodes {first, last, node, children or NONE for a leaf}
+    uint32_t* ncross;  // per tile
+};
+// Crossing nodes and leaves whose split is in one tile: at most 32 nested
+// nodes and a leaf per tile edge.
+constexpr uint32_t TILE_CROSS = 2 * (TILE_ENDS + 1);
+constexpr size_t TILE_BYTES = (2 + 4 * TILE_ENDS) * sizeof(float4) + TILE_CROSS * sizeof(uint4) + 4;
+
+struct TreeArgs {
+    const uint32_t* __restrict__ idx;
+    const float4* __restrict__ pos;
+    float4* __restrict__ tri;
+    uint4* __restrict__ span;
+    const uint32_t* __restrict__ par;
+    const uint32_t* __restrict__ rel;
+    float4* __restrict__ node;
+    uint32_t* __restrict__ parent;
+    uint32_t* levels;
+    TreeTiles tiles;
+    uint32_t T;
+};
+
+// Boxes of every node whose range lies in one tile, and what the others take
+// from the tile.  Round k has the union of every window of 2^k positions in
+// LDS; min and max are idempotent, so the box of a range of 2^k to 2^(k+1) - 1
+// positions is the union of its first and its last window, and a node costs
+// two windows whatever its size and needs no other node's box.  The ranges are
+// listed by their round first, so that a round's are taken by dense lanes.
+// Build: also the node numbers from the ranks, and the parent array; REFIT:
+// the numbers are kept in the spans, and the triangle records are gathered
+// again.  Bound by LDS and barrier latency at few tiles (17 us at 65k), by
+// the record, span and node traffic at many (8M: 254 us for 0.9 GB).
+constexpr int BOX_THREADS = 512, BOX_ITEMS = TREE_TILE / BOX_THREADS, BOX_ROUNDS = 11;
+template <bool REFIT>
+__global__ __launch_bounds__(BOX_THREADS) void k_boxes(TreeArgs A) {
+    __shared__ float s_m[6][TREE_TILE];
+    __shared__ uint4 s_span[TREE_TILE];
+    __shared__ uint16_t s_list[2 * TREE_TILE + 2 * TILE_ENDS];
+    __shared__ uint32_t s_off[64];
+    __shared__ uint32_t s_cnt[BOX_ROUNDS], s_at[BOX_ROUNDS + 1];
+    __shared__ uint32_t s_tails, s_heads, s_cross;
+    const uint32_t tid = threadIdx.x, base = blockIdx.x * TREE_TILE;
+    const uint32_t valid = A.T - base < (uint32_t)TREE_TILE ? A.T - base : (uint32_t)TREE_TILE;
+    const uint32_t last = base + valid - 1u;  // the tile's last position
+    if (tid == 0) s_tails = s_heads = s_cross = 0;
+    if (tid < BOX_ROUNDS) s_cnt[tid] = 0;
+    if (!REFIT && tid < 64) s_off[tid] = A.levels[LV_OFF + tid];
+    const bool one_leaf = !REFIT && A.levels[LV_TOTAL] == 1u;
+    Box m[BOX_ITEMS];
+    auto put = [&](uint32_t p, const Box& b) {
+        s_m[0][p] = b.lo.x, s_m[1][p] = b.lo.y, s_m[2][p] = b.lo.z;
+        s_m[3][p] = b.hi.x, s_m[4][p] = b.hi.y, s_m[5][p] = b.hi.z;
+    };
+    auto get = [&](uint32_t p) {
+        return Box{mk3(s_m[0][p], s_m[1][p], s_m[2][p]), mk3(s_m[3][p], s_m[4][p], s_m[5][p])};
+    };
+#pragma unroll
+    for (int j = 0; j < BOX_ITEMS; ++j) {
+        const uint32_t p = j * BOX_THREADS + tid, i = base + p;
+        m[j] = no_box();
+        if (p < valid) {
+            float4 v[3];
+            if (REFIT) {
+#pragma unroll
+                for (int k = 0; k < 3; ++k) {
+                    const uint32_t a = A.idx[3 * (size_t)i + k];
+                    const float4 q = A.pos[a];
+                    v[k] = make_float4(q.x, q.y, q.z, __uint_as_float(a));
+                    A.tri[3 * (size_t)i + k] = v[k];
+                }
+            } else {
+#pragma unroll
+                for (int k = 0; k < 3; ++k) v[k] = A.tri[3 * (size_t)i + k];
+            }
+            m[j].lo = vmin(vmin(xyz(v[0]), xyz(v[1])), xyz(v[2]));
+            m[j].hi = vmax(vmax(xyz(v[0]), xyz(v[1])), xyz(v[2]));
+        }
+        put(p, m[j]);
+    }
+    __syncthreads();
+    // The ranges that the split at tile position p asks for: 0 its node, 1 and
+    // 2 its leaf children, 3 the tile's end after it, 4 the tile's start up to
+    // it.  False where there is none.
+    auto ask = [&](const uint4& q, uint32_t p, int kind, uint32_t& a, uint32_t& b) -> bool {
+        const uint32_t s = base + p;
+        if (q.z == NONE) return false;
+        if (kind == 0) {
+            a = q.x;
+            b = q.y;
+            return true;
+        }
+        if (q.w == NONE) return false;  // the root is a leaf
+        if (kind == 1) {
+            a = q.x;
+            b = s;
+            return (q.w & SPAN_LEFT) != 0u;
+        }
+        if (kind == 2) {
+            a = s + 1u;
+            b = q.y;
+            return (q.w & SPAN_RIGHT) != 0u;
+        }
+        if (kind == 3) {
+            a = s + 1u;
+            b = last;
+            return q.y > last && s < last;
+        }
+        a = base;
+        b = s;
+        return q.x < base && s < last;
+    };
+    uint32_t slot[BOX_ITEMS][5];  // round << 16 | place in the round's list; NONE: not listed
+#pragma unroll
+    for (int j = 0; j < BOX_ITEMS; ++j) {
+        const uint32_t p = j * BOX_THREADS + tid, s = base + p;
+        uint4 q = make_uint4(0, 0, NONE, 0);  // {l, r, node, children}; node NONE: no node splits here
+        if (s < A.T) {
+            if (REFIT) {
+                q = A.span[s];
+            } else {
+                const uint32_t up = A.par[s];
+                if (up != NONE) {
+                    q = A.span[s];
+                    const uint32_t d = q.z >> 2, c = s_off[d + 1u] + 2u * A.rel[s];
+                    const uint32_t n = up == s ? 0u : s_off[d] + 2u * A.rel[up] + (s > up ? 1u : 0u);
+                    q = make_uint4(q.x, q.y, n, c | ((q.z & 1u) ? SPAN_LEFT : 0u) | ((q.z & 2u) ? SPAN_RIGHT : 0u));
+                    A.parent[c] = n;
+                    A.parent[c + 1u] = n;
+                } else if (one_leaf && s == A.T - 1u) {
+                    q = make_uint4(0u, s, 0u, NONE);  // the root is a leaf
+                }
+                A.span[s] = q;
+            }
+        }
+        s_span[p] = q;
+#pragma unroll
+        for (int kind = 0; kind < 5; ++kind) {
+            uint32_t a, b;
+            slot[j][kind] = NONE;
+            if (!ask(q, p, kind, a, b)) continue;
+            if (kind < 3 && (a < base || b > last)) {
+                const uint32_t k = atomicAdd(&s_cross, 1u), c = q.w & SPAN_NUM;
+                if (k < TILE_CROSS)
+                    A.tiles.cross[(size_t)blockIdx.x * TILE_CROSS + k] =
+                        make_uint4(a, b, kind == 0 ? q.z : c + (uint32_t)kind - 1u,
+                                   kind == 0 && q.w != NONE ? c : NONE);
+            } else {
+                const uint32_t k = 31u - (uint32_t)__builtin_clz(b - a + 1u);
+                slot[j][kind] = (k << 16) | atomicAdd(&s_cnt[k], 1u);
+            }
+        }
+    }
+    __syncthreads();
+    if (tid == 0) {
+        uint32_t at = 0;
+        for (int k = 0; k < BOX_ROUNDS; ++k) {
+            s_at[k] = at;
+            at += s_cnt[k];
+        }
+        s_at[BOX_ROUNDS] = at;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < BOX_ITEMS; ++j)
+#pragma unroll
+        for (int kind = 0; kind < 5; ++kind)
+            if (slot[j][kind] != NONE)
+                s_list[s_at[slot[j][kind] >> 16] + (slot[j][kind] & 0xffffu)] =
+                    (uint16_t)((kind << 10) | (j * BOX_THREADS + tid));
+    float4* const tails = A.tiles.tails + (size_t)blockIdx.x * 2 * TILE_ENDS;
+    float4* const heads = A.tiles.heads + (size_t)blockIdx.x * 2 * TILE_ENDS;
+    __syncthreads();
+    for (int k = 0; k < BOX_ROUNDS; ++k) {
+        const uint32_t len = 1u << k;
+        for (uint32_t i = s_at[k] + tid; i < s_at[k + 1]; i += BOX_THREADS) {
+            const uint32_t p = s_list[i] & (TREE_TILE - 1u);
+            const int kind = (int)(s_list[i] >> 10);
+            const uint4 q = s_span[p];
+            uint32_t a = 0, b = 0;
+            ask(q, p, kind, a, b);
+            const Box box = join(get(a - base), get(b + 1u - len - base));
+            const uint32_t c = q.w & SPAN_NUM;
+            if (kind == 0) {
+                if (q.w == NONE)
+                    put_node(A.node, 0u, box, 0u, A.T);
+                else
+                    put_node(A.node, q.z, box, c, 0u);
+            } else if (kind < 3) {
+                put_node(A.node, c + (uint32_t)kind - 1u, box, a, b - a + 1u);
+            } else if (kind == 3) {
+                const uint32_t t = atomicAdd(&s_tails, 1u);
+                if (t < TILE_ENDS) put_node(tails, t, box, a, 0u);
+            } else {
+                const uint32_t t = atomicAdd(&s_heads, 1u);
+                if (t < TILE_ENDS) put_node(heads, t, box, b, 0u);
+            }
+        }
+        if (k == BOX_ROUNDS - 1) break;
+        // windows of 2^(k+1): mine and the one 2^k further on
+#pragma unroll
+        for (int j = 0; j < BOX_ITEMS; ++j) {
+            const uint32_t p = j * BOX_THREADS + tid + len;
+            if (p < (uint32_t)TREE_TILE) m[j] = join(m[j], get(p));
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < BOX_ITEMS; ++j) put(j * BOX_THREADS + tid, m[j]);
+        __syncthreads();
+    }
+    __syncthreads();
+    // the last window at position 0 covers the tile
+    if (tid == 0) {
+        put_node(A.tiles.box, blockIdx.x, m[0], s_tails, s_heads);
+        A.tiles.ncross[blockIdx.x] = s_cross;
+    }
+}
+
+// Boxes of the nodes whose range crosses tiles, one wave each: the tail of
+// the first tile, the boxes of the tiles between, the head of the last.
+__global__ __launch_bounds__(BS) void k_cross(float4* __restrict__ node, TreeTiles tiles, uint32_t T) {
+    const uint32_t lane = threadIdx.x & 63, n = tiles.ncross[blockIdx.x];
+    for (uint32_t k = threadIdx.x >> 6; k < n; k += BS / RTX_WAVE) {
+        const uint4 q = tiles.cross[(size_t)blockIdx.x * TILE_CROSS + k];
+        const uint32_t ta = q.x / TREE_TILE, tb = q.y / TREE_TILE;
+        Box b = no_box();
+        for (uint32_t t = ta + 1u + lane; t < tb; t += RTX_WAVE)
+            b = join(b, Box{xyz(tiles.box[2 * (size_t)t]), xyz(tiles.box[2 * (size_t)t + 1])});
+        // lanes 0..31: the entries of the first tile's tails; 32..63: the last tile's heads
+        const bool first = lane < TILE_ENDS;
+        const uint32_t t = first ? ta : tb, i = lane & (TILE_ENDS - 1u);
+        const bool whole = first ? q.x % TREE_TILE == 0u : (q.y + 1u == T || (q.y + 1u) % TREE_TILE == 0u);
+        const float4 b0 = tiles.box[2 * (size_t)t], b1 = tiles.box[2 * (size_t)t + 1];
+        if (first && ta == tb) {
+            // a leaf that starts its tile, listed by the tile before (its parent's
+            // split is that tile's last position): a head only
+        } else if (whole) {
+            b = join(b, Box{xyz(b0), xyz(b1)});
+        } else if (i < __float_as_uint(first ? b0.w : b1.w)) {
+            const float4* p = (first ? tiles.tails : tiles.heads) + 2 * ((size_t)t * TILE_ENDS + i);
+            const float4 p0 = p[0], p1 = p[1];
+            if (__float_as_uint(p0.w) == (first ? q.x : q.y)) b = join(b, Box{xyz(p0), xyz(p1)});
         }
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) {
-#pragma unroll
-            for (int k = 0; k < 3; ++k) q[k] = fminf(q[k], __shfl_xor(q[k], off, RTX_WAVE));
-#pragma unroll
-            for (int k = 3; k < 6; ++k) q[k] = fmaxf(q[k], __shfl_xor(q[k], off, RTX_WAVE));
+            const Box o{mk3(__shfl_xor(b.lo.x, off, RTX_WAVE), __shfl_xor(b.lo.y, off, RTX_WAVE),
+                            __shfl_xor(b.lo.z, off, RTX_WAVE)),
+                        mk3(__shfl_xor(b.hi.x, off, RTX_WAVE), __shfl_xor(b.hi.y, off, RTX_WAVE),
+                            __shfl_xor(b.hi.z, off, RTX_WAVE))};
+            b = join(b, o);
         }
-        if (lane == 0) {
-            node[2 * (size_t)n] = make_float4(q[0], q[1], q[2], __uint_as_float(a));
-            node[2 * (size_t)n + 1] = make_float4(q[3], q[4], q[5], __uint_as_float(cnt));
-        }
+        if (lane == 0) put_node(node, q.z, b, q.w == NONE ? q.x : q.w, q.w == NONE ? q.y - q.x + 1u : 0u);
     }
 }
 
-struct HierArgs {
-    const uint32_t* __restrict__ codes;
-    const uint32_t* __restrict__ kj;  // radix tree: other end of node i's range
-    const uint32_t* __restrict__ kg;  // radix tree: split of node i
-    uint32_t* __restrict__ bstart;
-    uint32_t* __restrict__ bend;
-    float4* __restrict__ node;
-    uint32_t* __restrict__ parent;
-    const float4* __restrict__ tri;
-    uint32_t* levels;
-    uint32_t* __restrict__ fat_list;
-    uint32_t T;
-    int min_leaf;
-};
-
-// One tile (BS consecutive nodes) of level d, by the whole block; the tile's
-// exclusive prefix of splitting nodes comes from the look-back over the
-// level's tiles (status).  Ends with a block barrier.
-__device__ __forceinline__ void hier_tile(const HierArgs& A, uint32_t* status, int d, bool force_leaf, uint32_t off,
-                                          uint32_t cnt, uint32_t tile, uint32_t ntiles, uint32_t* s_w,
-                                          uint32_t* s_prefix) {
-    const uint32_t tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const uint32_t k = tile * BS + tid;
-    const bool active = k < cnt;
-    const uint32_t n = off + k;
-    uint32_t start = 0, end = 0, split = 0;
-    if (active) {
-        start = A.bstart[n];
-        end = A.bend[n];
-        // Leaf iff count <= min_leaf + 2 (unsigned test, so a single triangle
-        // falls through) or the first and last codes are equal: find_middle
-        // advances its level while first and last share the level's bit, so it
-        // ends at their highest differing bit, and runs out of bits only when
-        // the codes are equal (every node's level bit is above all bits in
-        // which its codes differ).
-        if (!force_leaf && end - start - 2u > (uint32_t)A.min_leaf && A.codes[start] != A.codes[end - 1]) {
-            const uint32_t last = end - 1;
-            const uint32_t other = (last <= A.T - 2u) ? last : start;
-            split = (A.kj[start] == last ? A.kg[start] : A.kg[other]) + 1u;
-        }
-    }
-    const bool is_split = split != 0;
-    const uint64_t bal = ballot(is_split);
-    const uint32_t excl = lanes_below(bal);
-    if (lane == 0) s_w[w] = (uint32_t)__builtin_popcountll(bal);
-    __syncthreads();
-    uint32_t wofs = 0, agg = 0;
-#pragma unroll
-    for (int i = 0; i < BS / RTX_WAVE; ++i) {
-        wofs += (i < (int)w) ? s_w[i] : 0u;
-        agg += s_w[i];
-    }
-    if (w == 0) {
-        const uint32_t prefix = lookback_wave(status, tile, agg, 1u);
-        if (lane == 0) *s_prefix = prefix;
-        if (lane == 0 && tile == ntiles - 1) {
-            const uint32_t total = prefix + agg;
-            A.levels[LV_OFF + d + 1] = off + cnt;
-            A.levels[LV_CNT + d + 1] = 2u * total;
-            A.levels[LV_TOTAL] = off + cnt + 2u * total;
-        }
-    }
-    __syncthreads();
-    // Leaves of more than FAT_LEAF triangles go to the fat list (bounded by
-    // k_fat_leaves, one wave each); the node gets its range now.
-    const bool fat = active && !is_split && end - start > FAT_LEAF;
-    const uint64_t fm = ballot(fat);
-    if (fm) {
-        uint32_t fbase = 0;
-        if (lane == (uint32_t)__builtin_ctzll(fm))
-            fbase = atomicAdd(&A.levels[LV_FAT], (uint32_t)__builtin_popcountll(fm));
-        fbase = __shfl(fbase, __builtin_ctzll(fm), RTX_WAVE);
-        if (fat) {
-            A.fat_list[fbase + lanes_below(fm)] = n;
-            A.node[2 * (size_t)n] = make_float4(0.f, 0.f, 0.f, __uint_as_float(start));
-            A.node[2 * (size_t)n + 1] = make_float4(0.f, 0.f, 0.f, __uint_as_float(end - start));
-        }
-    }
-    if (active && is_split) {
-        const uint32_t rank = *s_prefix + wofs + excl;
-        const uint32_t c = off + cnt + 2u * rank;
-        A.bstart[c] = start;
-        A.bend[c] = split;
-        A.bstart[c + 1] = split;
-        A.bend[c + 1] = end;
-        A.parent[c] = n;
-        A.parent[c + 1] = n;
-        uint32_t* node_u32 = reinterpret_cast<uint32_t*>(A.node);
-        node_u32[8 * (size_t)n + 3] = c;
-        node_u32[8 * (size_t)n + 7] = 0u;
-    } else if (active && !fat) {
-        // build_leaf_bbox (src/kernel/bvh-builder.cl:262-288) for this leaf
-        leaf_bounds(A.tri, A.node, n, start, end - start);
-    }
-    __syncthreads();
-}
-
-// Levels 0..dtop (at most 2^d <= BS nodes each, one tile) by one block, one
-// level after the other: the top of the tree costs one launch, not dtop+1.
-__global__ __launch_bounds__(BS) void k_hier_top(HierArgs A, uint32_t* status, uint32_t status_stride, int dtop,
-                                                 int depth) {
-    __shared__ uint32_t s_prefix;
-    __shared__ uint32_t s_w[BS / RTX_WAVE];
-    for (int d = 0; d <= dtop; ++d) {
-        const uint32_t off = A.levels[LV_OFF + d], cnt = A.levels[LV_CNT + d];
-        if (cnt == 0) {
-            if (threadIdx.x == 0) {
-                A.levels[LV_OFF + d + 1] = off;
-                A.levels[LV_CNT + d + 1] = 0;
-            }
-            __syncthreads();
-            continue;
-        }
-        hier_tile(A, status + (size_t)d * status_stride, d, d == depth, off, cnt, 0u, 1u, s_w, &s_prefix);
-    }
-}
-
-// One iteration of process_task (src/kernel/bvh-builder.cl:582-671) over the
-// nodes of level d, in order.  Children of the k-th splitting node of the
-// level go to off_next + 2k (ordered compaction by decoupled look-back),
-// which is the order in-order work-groups of the reference produce.  Blocks
-// are persistent: each takes tile tickets until the level is done.
-__global__ __launch_bounds__(BS) void k_hier_level(HierArgs A, uint32_t* status, uint32_t* ticket, int d,
-                                                   int force_leaf) {
-    __shared__ uint32_t s_tile, s_prefix;
-    __shared__ uint32_t s_w[BS / RTX_WAVE];
-    const uint32_t off = A.levels[LV_OFF + d];
-    const uint32_t cnt = A.levels[LV_CNT + d];
-    if (cnt == 0) {
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
-            A.levels[LV_OFF + d + 1] = off;
-            A.levels[LV_CNT + d + 1] = 0;
-        }
-        return;
-    }
-    const uint32_t ntiles = (cnt + BS - 1) / BS;
-    if (blockIdx.x >= ntiles) return;  // only blocks with work take tickets
-    for (;;) {
-        if (threadIdx.x == 0) s_tile = atomicAdd(ticket, 1u);
-        __syncthreads();
-        const uint32_t tile = s_tile;
-        if (tile >= ntiles) return;
-        hier_tile(A, status, d, force_leaf != 0, off, cnt, tile, ntiles, s_w, &s_prefix);
-    }
-}
-
-// build_node_bbox (src/kernel/bvh-builder.cl:290-311) for the internal nodes
-// of level d: union of the two children (computed by the launch for level
-// d+1, or as leaves), plus the near-child delta right.lo - left.lo used by
-// traversal.  One launch per level, deepest first, as the reference's host
-// loop (src/rt/bvh-builder.cpp:683-695).
-__global__ __launch_bounds__(BS) void k_refit_level(float4* __restrict__ node, float4* __restrict__ delta,
-                                                    const uint32_t* __restrict__ levels, int d) {
-    const uint32_t off = levels[LV_OFF + d], cnt = levels[LV_CNT + d];
-    for (uint32_t k = blockIdx.x * BS + threadIdx.x; k < cnt; k += gridDim.x * BS) {
-        uint32_t n = off + k;
-        float4 f0 = node[2 * (size_t)n], f1 = node[2 * (size_t)n + 1];
-        if (__float_as_uint(f1.w) != 0u) continue;  // leaf: bounded at emission
-        uint32_t l = __float_as_uint(f0.w);
-        float4 L0 = node[2 * (size_t)l], L1 = node[2 * (size_t)l + 1];
-        float4 R0 = node[2 * (size_t)l + 2], R1 = node[2 * (size_t)l + 3];
-        v3 plo = vmin(xyz(L0), xyz(R0));
-        v3 phi = vmax(xyz(L1), xyz(R1));
-        node[2 * (size_t)n] = make_float4(plo.x, plo.y, plo.z, f0.w);
-        node[2 * (size_t)n + 1] = make_float4(phi.x, phi.y, phi.z, f1.w);
-        v3 dl = xyz(R0) - xyz(L0);
-        delta[n] = make_float4(dl.x, dl.y, dl.z, 0.f);
-    }
-}
-
-// Internal-node AABBs of levels dhi..0 (at most 2^d nodes each) by one
-// block, deepest first.
-__global__ __launch_bounds__(BS) void k_refit_top(float4* __restrict__ node, float4* __restrict__ delta,
-                                                  const uint32_t* __restrict__ levels, int dhi) {
-    for (int d = dhi; d >= 0; --d) {
-        const uint32_t off = levels[LV_OFF + d], cnt = levels[LV_CNT + d];
-        for (uint32_t k = threadIdx.x; k < cnt; k += BS) {
-            const uint32_t n = off + k;
-            const float4 f0 = node[2 * (size_t)n], f1 = node[2 * (size_t)n + 1];
-            if (__float_as_uint(f1.w) != 0u) continue;
-            const uint32_t l = __float_as_uint(f0.w);
-            const float4 L0 = node[2 * (size_t)l], L1 = node[2 * (size_t)l + 1];
-            const float4 R0 = node[2 * (size_t)l + 2], R1 = node[2 * (size_t)l + 3];
-            const v3 plo = vmin(xyz(L0), xyz(R0));
-            const v3 phi = vmax(xyz(L1), xyz(R1));
-            node[2 * (size_t)n] = make_float4(plo.x, plo.y, plo.z, f0.w);
-            node[2 * (size_t)n + 1] = make_float4(phi.x, phi.y, phi.z, f1.w);
-            const v3 dl = xyz(R0) - xyz(L0);
-            delta[n] = make_float4(dl.x, dl.y, dl.z, 0.f);
-        }
-        __syncthreads();
-    }
-}
-
-// Leaf AABBs of an existing topology (refit path).
-__global__ __launch_bounds__(BS) void k_leaf_bounds(const float4* __restrict__ tri, float4* __restrict__ node,
-                                                    const uint32_t* __restrict__ levels) {
+// The near-child differences right.lo - left.lo of the inner nodes.
+__global__ __launch_bounds__(BS) void k_deltas(const float4* __restrict__ node, float4* __restrict__ delta,
+                                               const uint32_t* __restrict__ levels) {
     const uint32_t N = levels[LV_TOTAL];
     for (uint32_t n = blockIdx.x * BS + threadIdx.x; n < N; n += gridDim.x * BS) {
-        float4 f0 = node[2 * (size_t)n], f1 = node[2 * (size_t)n + 1];
-        uint32_t cnt = __float_as_uint(f1.w);
-        if (cnt && cnt <= FAT_LEAF) leaf_bounds(tri, node, n, __float_as_uint(f0.w), cnt);
+        const uint32_t l = __float_as_uint(node[2 * (size_t)n].w), cnt = __float_as_uint(node[2 * (size_t)n + 1].w);
+        if (cnt) continue;
+        const v3 dl = xyz(node[2 * (size_t)l + 2]) - xyz(node[2 * (size_t)l]);
+        delta[n] = make_float4(dl.x, dl.y, dl.z, 0.f);
     }
 }
 
@@ -704,13 +923,12 @@ static int32_t lbvh_alloc(rtx_scene* s, uint32_t T, int depth) {
     size_t ncap = 2 * (size_t)T;
     uint32_t passes = (uint32_t)(depth + 7) / 8;
     uint32_t sort_tiles = rtx_div_up(T, SORT_TILE);
-    uint32_t hier_tiles = rtx_div_up(T, BS);
+    const size_t tree_tiles = rtx_div_up(T, TREE_TILE);
     int32_t e = 0;
     if ((e = s->b().node.reserve(c, ncap * 32 + 64))) return e;
     if ((e = s->b().delta.reserve(c, ncap * 16))) return e;
     if ((e = s->b().parent.reserve(c, ncap * 4))) return e;
-    if ((e = s->b().bstart.reserve(c, ncap * 4))) return e;
-    if ((e = s->b().bend.reserve(c, ncap * 4))) return e;
+    if ((e = s->b().span.reserve(c, (size_t)T * 16))) return e;
     if ((e = s->b().tri.reserve(c, (size_t)T * 48))) return e;
     if ((e = s->b().codes.reserve(c, (size_t)T * 4))) return e;
     if ((e = s->b().perm.reserve(c, (size_t)T * 4))) return e;
@@ -723,8 +941,8 @@ static int32_t lbvh_alloc(rtx_scene* s, uint32_t T, int depth) {
     if ((e = s->b().tickets.reserve(c, TK_COUNT * 4))) return e;
     if ((e = s->b().sort_hist.reserve(c, 4 * 256 * 4))) return e;
     if ((e = s->b().sort_status.reserve(c, (size_t)passes * sort_tiles * 256 * 4))) return e;
-    if ((e = s->b().hier_status.reserve(c, (size_t)(depth + 1) * hier_tiles * 4))) return e;
-    if ((e = s->b().fat.reserve(c, ((size_t)T / (FAT_LEAF + 1) + 1) * 4))) return e;
+    if ((e = s->b().rank_status.reserve(c, tree_tiles * 64 * 4))) return e;
+    if ((e = s->b().tree_tiles.reserve(c, tree_tiles * TILE_BYTES))) return e;
     return 0;
 }
 
@@ -732,44 +950,51 @@ static int32_t lbvh_alloc(rtx_scene* s, uint32_t T, int depth) {
 // scene's buffer set holds it for rtx_lbvh_build; the allocation-free build
 // carves it from a fixed array instead.
 struct BuildScratch {
-    uint32_t *bstart, *bend;        // per-node triangle range during emission
-    uint32_t *keys_alt, *vals_alt;  // radix ping-pong, then the radix-tree arrays
+    uint32_t *keys_alt, *vals_alt;  // radix ping-pong, then the splits' parents and ranks
     float4* centroid;
     float* partials;
-    uint32_t *sort_hist, *sort_status, *tickets, *hier_status;
+    uint32_t *sort_hist, *sort_status, *tickets, *rank_status;
+    void* tree_tiles;
 };
 
 static BuildScratch scratch_of(BuildSet& b) {
-    return BuildScratch{b.bstart.as<uint32_t>(),   b.bend.as<uint32_t>(),        b.keys_alt.as<uint32_t>(),
-                        b.vals_alt.as<uint32_t>(), b.centroid.as<float4>(),      b.partials.as<float>(),
-                        b.sort_hist.as<uint32_t>(), b.sort_status.as<uint32_t>(), b.tickets.as<uint32_t>(),
-                        b.hier_status.as<uint32_t>()};
+    return BuildScratch{b.keys_alt.as<uint32_t>(),  b.vals_alt.as<uint32_t>(),    b.centroid.as<float4>(),
+                        b.partials.as<float>(),     b.sort_hist.as<uint32_t>(),   b.sort_status.as<uint32_t>(),
+                        b.tickets.as<uint32_t>(),   b.rank_status.as<uint32_t>(), b.tree_tiles.p};
 }
 
-static void fat_leaf_bounds(rtx_scene* s, hipStream_t st, rtx_ctx* pc) {
-    ProfScope ps(pc, st, "lbvh_fat_leaves");
-    uint32_t g = rtx_div_up((uint64_t)s->T / (FAT_LEAF + 1) + 1, BS / RTX_WAVE);
-    hipLaunchKernelGGL(k_fat_leaves, dim3(g > 1024 ? 1024 : g), dim3(BS), 0, st, s->b().tri.as<float4>(), s->nodes(),
-                       s->b().fat.as<uint32_t>(), s->b().levels.as<uint32_t>());
+static TreeArgs tree_args(rtx_scene* s, const BuildScratch& W) {
+    const size_t tiles = rtx_div_up(s->T, TREE_TILE);
+    float4* f = static_cast<float4*>(W.tree_tiles);
+    uint4* const cross = reinterpret_cast<uint4*>(f + (2 + 4 * TILE_ENDS) * tiles);
+    TreeTiles t{f, f + 2 * tiles, f + (2 + 2 * TILE_ENDS) * tiles, cross,
+                reinterpret_cast<uint32_t*>(cross + (size_t)TILE_CROSS * tiles)};
+    return TreeArgs{s->idx.as<uint32_t>(), s->pos.as<float4>(),      s->b().tri.as<float4>(),
+                    s->b().span.as<uint4>(), W.keys_alt,             W.vals_alt,
+                    s->nodes(),            s->b().parent.as<uint32_t>(), s->b().levels.as<uint32_t>(),
+                    t,                     s->T};
 }
 
-// Internal-node AABBs, deepest level first (levels depth-1 .. 0; level
-// `depth` holds only leaves).
-static void refit_internal(rtx_scene* s, hipStream_t st, int depth, rtx_ctx* pc) {
+// Boxes of all nodes (REFIT: of the kept topology, from the current
+// positions), then the near-child differences.
+template <bool REFIT>
+static void tree_boxes(rtx_scene* s, hipStream_t st, const BuildScratch& W, rtx_ctx* pc) {
+    const TreeArgs A = tree_args(s, W);
+    const uint32_t tiles = rtx_div_up(s->T, TREE_TILE);
     const uint32_t gmax = (uint32_t)s->ctx->cus * (uint32_t)s->ctx->tune.build_grid;
-    for (int d = depth - 1; d > REFIT_TOP; --d) {
-        ProfScope ps(pc, st, "lbvh_refit_level");
-        uint64_t maxn = d < 32 ? (1ull << d) : (uint64_t)s->T;
-        if (maxn > 2ull * s->T) maxn = 2ull * s->T;
-        uint32_t g = rtx_div_up(maxn, BS);
-        hipLaunchKernelGGL(k_refit_level, dim3(g > gmax ? gmax : g), dim3(BS), 0, st, s->nodes(),
-                           s->b().delta.as<float4>(), s->b().levels.as<uint32_t>(), d);
+    {
+        ProfScope ps(pc, st, "lbvh_boxes");
+        hipLaunchKernelGGL((k_boxes<REFIT>), dim3(tiles), dim3(BOX_THREADS), 0, st, A);
     }
-    const int dhi = depth - 1 < REFIT_TOP ? depth - 1 : REFIT_TOP;
-    if (dhi >= 0) {
-        ProfScope ps(pc, st, "lbvh_refit_top");
-        hipLaunchKernelGGL(k_refit_top, dim3(1), dim3(BS), 0, st, s->nodes(), s->b().delta.as<float4>(),
-                           s->b().levels.as<uint32_t>(), dhi);
+    {
+        ProfScope ps(pc, st, "lbvh_cross");
+        hipLaunchKernelGGL(k_cross, dim3(tiles), dim3(BS), 0, st, s->nodes(), A.tiles, s->T);
+    }
+    {
+        ProfScope ps(pc, st, "lbvh_deltas");
+        const uint32_t g = rtx_div_up(s->T, BS);
+        hipLaunchKernelGGL(k_deltas, dim3(g > gmax ? gmax : g), dim3(BS), 0, st, s->nodes(),
+                           s->b().delta.as<float4>(), s->b().levels.as<uint32_t>());
     }
 }
 
@@ -799,21 +1024,16 @@ static bool build_sort_phase(rtx_scene* s, int depth, hipStream_t st, const Buil
     const int rb = (int)s->ctx->tune.sort_bits, items = (int)s->ctx->tune.sort_items;
     const int passes = (depth + rb - 1) / rb;
     const uint32_t sort_tiles = rtx_div_up(T, (uint64_t)BS * items);
-    const uint32_t hier_tiles = rtx_div_up(T, BS);
     uint32_t* tickets = W.tickets;
-    uint32_t* levels = s->b().levels.as<uint32_t>();
     {
         ProfScope ps(pc, st, "lbvh_init");
-        uint32_t nb = (uint32_t)(passes * (size_t)sort_tiles << rb);
-        uint32_t nc = (uint32_t)((size_t)(depth + 1) * hier_tiles);
+        const uint32_t nb = (uint32_t)(passes * (size_t)sort_tiles << rb);
+        const uint32_t nc = rtx_div_up(T, TREE_TILE) * 64u;
         uint32_t grid = rtx_div_up((uint64_t)(nb > nc ? nb : nc), BS);
-        grid = grid < 1 ? 1 : (grid > 2048 ? 2048 : grid);
-        // zero: tickets + histograms (contiguous? no: separate buffers)
+        grid = grid < 4 ? 4 : (grid > 2048 ? 2048 : grid);
         hipLaunchKernelGGL(k_build_init, dim3(grid), dim3(BS), 0, st, tickets, (uint32_t)TK_COUNT, W.sort_status, nb,
-                           W.hier_status, nc, levels, W.bstart, W.bend, s->b().parent.as<uint32_t>(), T, 1);
-        hipLaunchKernelGGL(k_build_init, dim3(1), dim3(BS), 0, st, W.sort_hist, 4u * 256u,
-                           (uint32_t*)nullptr, 0u, (uint32_t*)nullptr, 0u, levels, (uint32_t*)nullptr,
-                           (uint32_t*)nullptr, (uint32_t*)nullptr, T, 0);
+                           W.rank_status, nc, W.sort_hist, 4u * 256u, s->b().levels.as<uint32_t>(),
+                           s->b().parent.as<uint32_t>());
     }
     {
         ProfScope ps(pc, st, "lbvh_prim_bounds");
@@ -872,43 +1092,30 @@ static bool build_sort_phase(rtx_scene* s, int depth, hipStream_t st, const Buil
     return in_alt;
 }
 
-// Tree phase: radix tree, level-ordered hierarchy, fat-leaf bounds and the
-// bottom-up refit.  It reads only the buffer set's own sorted codes and
-// triangle records, so it can run beside the next build's sort phase when
-// that one writes another set.
-static void build_tree_phase(rtx_scene* s, int depth, int min_leaf, hipStream_t st, const BuildScratch& W,
-                             rtx_ctx* pc) {
-    const uint32_t T = s->T;
-    const uint32_t hier_tiles = rtx_div_up(T, BS);
-    uint32_t* tickets = W.tickets;
-    uint32_t* levels = s->b().levels.as<uint32_t>();
+// Tree phase: ranges, levels and ranks of the splits, then the nodes with
+// their boxes.  It reads only the buffer set's own sorted codes and triangle
+// records, so it can run beside the next build's sort phase when that one
+// writes another set.
+static void build_tree_phase(rtx_scene* s, int min_leaf, hipStream_t st, const BuildScratch& W, rtx_ctx* pc) {
+    const uint32_t T = s->T, tiles = rtx_div_up(T, TREE_TILE);
     {
-        ProfScope ps(pc, st, "lbvh_radix_tree");
-        // radix-tree arrays reuse the sort's alternate buffers
-        hipLaunchKernelGGL(k_radix_tree, dim3(rtx_div_up(T, BS)), dim3(BS), 0, st, s->b().codes.as<uint32_t>(),
-                           W.keys_alt, W.vals_alt, (int)T);
+        ProfScope ps(pc, st, "lbvh_spans");
+        hipLaunchKernelGGL(k_spans, dim3(tiles), dim3(TREE_TILE), 0, st, s->b().codes.as<uint32_t>(),
+                           s->b().span.as<uint4>(), W.keys_alt, W.vals_alt, (int)T, (uint32_t)min_leaf);
     }
     {
-        HierArgs A{s->b().codes.as<uint32_t>(), W.keys_alt, W.vals_alt, W.bstart, W.bend, s->nodes(),
-                   s->b().parent.as<uint32_t>(), s->b().tri.as<float4>(), levels, s->b().fat.as<uint32_t>(), T,
-                   min_leaf};
-        const int dtop = depth < HIER_TOP ? depth : HIER_TOP;
-        {
-            ProfScope ps(pc, st, "lbvh_hier_top");
-            hipLaunchKernelGGL(k_hier_top, dim3(1), dim3(BS), 0, st, A, W.hier_status, hier_tiles, dtop, depth);
-        }
-        const uint32_t gmax = (uint32_t)s->ctx->cus * (uint32_t)s->ctx->tune.build_grid;
-        for (int d = dtop + 1; d <= depth; ++d) {
-            ProfScope ps(pc, st, "lbvh_hier_level");
-            uint64_t maxn = d < 32 ? (1ull << d) : (uint64_t)T;
-            if (maxn > 2ull * T) maxn = 2ull * T;
-            uint32_t grid = rtx_div_up(maxn, BS);
-            hipLaunchKernelGGL(k_hier_level, dim3(grid > gmax ? gmax : grid), dim3(BS), 0, st, A,
-                               W.hier_status + (size_t)d * hier_tiles, tickets + TK_LEVEL + d, d, d == depth ? 1 : 0);
-        }
+        ProfScope ps(pc, st, "lbvh_ranks");
+        // short tiles while the look-back is short, else fewer of them
+#define RTX_RANKS(I)                                                                                                \
+    hipLaunchKernelGGL((k_ranks<I>), dim3(rtx_div_up(T, BS * I)), dim3(BS), 0, st, W.vals_alt, W.rank_status,      \
+                       W.tickets + TK_RANK, s->b().levels.as<uint32_t>(), T, rtx_div_up(T, BS * I))
+        if (T < RANK_WIDE)
+            RTX_RANKS(4);
+        else
+            RTX_RANKS(16);
+#undef RTX_RANKS
     }
-    fat_leaf_bounds(s, st, pc);
-    refit_internal(s, st, depth, pc);
+    tree_boxes<false>(s, st, W, pc);
 }
 
 // Sorted codes and permutation left in the scratch's alternates by an odd
@@ -929,7 +1136,7 @@ int32_t rtx_lbvh_build(rtx_scene* s, const rtx_lbvh_params* p, void* stream) {
     {
         ProfScope whole(s->ctx, st, "LBVH_BUILD");
         settle_sorted(s, build_sort_phase(s, depth, st, scratch_of(s->b()), s->ctx));
-        build_tree_phase(s, depth, min_leaf, st, scratch_of(s->b()), s->ctx);
+        build_tree_phase(s, min_leaf, st, scratch_of(s->b()), s->ctx);
     }
     RTX_CHECK_HIP(hipGetLastError());
     s->built = true;
@@ -948,7 +1155,7 @@ int32_t rtx_lbvh_build_split(rtx_scene* s, const rtx_lbvh_params* p, hipStream_t
     settle_sorted(s, build_sort_phase(s, depth, sort_stream, scratch_of(s->b()), s->ctx));
     RTX_CHECK_HIP(hipEventRecord(sorted, sort_stream));
     RTX_CHECK_HIP(hipStreamWaitEvent(tree_stream, sorted, 0));
-    build_tree_phase(s, depth, min_leaf, tree_stream, scratch_of(s->b()), s->ctx);
+    build_tree_phase(s, min_leaf, tree_stream, scratch_of(s->b()), s->ctx);
     RTX_CHECK_HIP(hipGetLastError());
     s->built = true;
     s->sah = false;
@@ -970,18 +1177,19 @@ namespace {
 constexpr size_t al256(size_t b) { return (b + 255) & ~(size_t)255; }
 constexpr size_t NA_T = RTX_LBVH_NOALLOC_MAX_TRIS;
 constexpr size_t NA_SORT_TILES = (NA_T + SORT_TILE - 1) / SORT_TILE;
-constexpr size_t NA_HIER_TILES = (NA_T + BS - 1) / BS;
-constexpr size_t NA_BYTES = 2 * al256(2 * NA_T * 4)                  // bstart, bend
-                          + 2 * al256(NA_T * 4)                      // keys_alt, vals_alt
-                          + al256(NA_T * 16)                         // centroid
-                          + al256((size_t)BOUNDS_GRID * 6 * 4)       // partials
-                          + al256(4 * 256 * 4)                       // sort_hist
-                          + al256(4 * NA_SORT_TILES * 256 * 4)       // sort_status
-                          + al256((size_t)TK_COUNT * 4)              // tickets
-                          + al256(33 * NA_HIER_TILES * 4);           // hier_status
+constexpr size_t NA_TREE_TILES = (NA_T + TREE_TILE - 1) / TREE_TILE;
+constexpr size_t NA_USED = 2 * al256(NA_T * 4)                      // keys_alt, vals_alt
+                         + al256(NA_T * 16)                         // centroid
+                         + al256((size_t)BOUNDS_GRID * 6 * 4)       // partials
+                         + al256(4 * 256 * 4)                       // sort_hist
+                         + al256(4 * NA_SORT_TILES * 256 * 4)       // sort_status
+                         + al256((size_t)TK_COUNT * 4)              // tickets
+                         + al256(NA_TREE_TILES * 64 * 4)            // rank_status
+                         + al256(NA_TREE_TILES * TILE_BYTES);       // tree_tiles
+constexpr size_t NA_BYTES = RTX_LBVH_NOALLOC_SCRATCH_BYTES;
 }  // namespace
 
-static_assert(NA_BYTES == RTX_LBVH_NOALLOC_SCRATCH_BYTES, "include/rtx.h states the scratch size");
+static_assert(NA_USED <= NA_BYTES, "the scratch holds every part");
 
 static __device__ __align__(256) unsigned char scratch[NA_BYTES];
 
@@ -1006,10 +1214,8 @@ static BuildScratch carve_scratch(void* base, uint32_t T) {
         p += al256(bytes);
         return q;
     };
-    const size_t sort_tiles = rtx_div_up(T, SORT_TILE), hier_tiles = rtx_div_up(T, BS);
+    const size_t sort_tiles = rtx_div_up(T, SORT_TILE), tree_tiles = rtx_div_up(T, TREE_TILE);
     BuildScratch W;
-    W.bstart = reinterpret_cast<uint32_t*>(take(2 * (size_t)T * 4));
-    W.bend = reinterpret_cast<uint32_t*>(take(2 * (size_t)T * 4));
     W.keys_alt = reinterpret_cast<uint32_t*>(take((size_t)T * 4));
     W.vals_alt = reinterpret_cast<uint32_t*>(take((size_t)T * 4));
     W.centroid = reinterpret_cast<float4*>(take((size_t)T * 16));
@@ -1017,7 +1223,8 @@ static BuildScratch carve_scratch(void* base, uint32_t T) {
     W.sort_hist = reinterpret_cast<uint32_t*>(take(4 * 256 * 4));
     W.sort_status = reinterpret_cast<uint32_t*>(take(4 * sort_tiles * 256 * 4));
     W.tickets = reinterpret_cast<uint32_t*>(take((size_t)TK_COUNT * 4));
-    W.hier_status = reinterpret_cast<uint32_t*>(take(33 * hier_tiles * 4));
+    W.rank_status = reinterpret_cast<uint32_t*>(take(tree_tiles * 64 * 4));
+    W.tree_tiles = take(tree_tiles * TILE_BYTES);
     return W;
 }
 
@@ -1043,7 +1250,7 @@ int32_t rtx_lbvh_build_noalloc(rtx_scene* s, const rtx_lbvh_params* p, void* str
     BuildSet& b = s->b();
     RTX_REQUIRE(b.node.bytes >= ncap * 32 + 64 && b.delta.bytes >= ncap * 16 && b.parent.bytes >= ncap * 4 &&
                     b.tri.bytes >= T * 48 && b.codes.bytes >= T * 4 && b.perm.bytes >= T * 4 && b.gbox.bytes >= 32 &&
-                    b.levels.bytes >= LV_WORDS * 4 && b.fat.bytes >= (T / (FAT_LEAF + 1) + 1) * 4,
+                    b.levels.bytes >= LV_WORDS * 4 && b.span.bytes >= T * 16,
                 RTX_ESTATE,
                 "rtx_lbvh_build_noalloc: the scene's tree buffers are not reserved for its triangle count "
                 "(run rtx_lbvh_build once first)");
@@ -1054,7 +1261,7 @@ int32_t rtx_lbvh_build_noalloc(rtx_scene* s, const rtx_lbvh_params* p, void* str
         hipLaunchKernelGGL(k_copy_pairs, dim3(g > 4096 ? 4096 : g), dim3(BS), 0, st, W.keys_alt, W.vals_alt,
                            b.codes.as<uint32_t>(), b.perm.as<uint32_t>(), (uint32_t)T);
     }
-    build_tree_phase(s, depth, min_leaf, st, W, nullptr);
+    build_tree_phase(s, min_leaf, st, W, nullptr);
     RTX_CHECK_HIP(hipGetLastError());
     s->built = true;
     s->sah = false;
@@ -1148,21 +1355,7 @@ int32_t rtx_lbvh_refit(rtx_scene* s, void* stream) {
     RTX_REQUIRE(s->built, RTX_ESTATE, "rtx_lbvh_refit: no BVH built");
     RTX_REQUIRE(!s->sah, RTX_ESTATE, "rtx_lbvh_refit: the tree is an SAH tree (refit follows LBVH levels)");
     hipStream_t st = s->ctx->pick(stream);
-    const uint32_t T = s->T;
-    {
-        ProfScope ps(s->ctx, st, "lbvh_tri_records");
-        hipLaunchKernelGGL(k_tri_records, dim3(rtx_div_up(T, BS)), dim3(BS), 0, st, s->idx.as<uint32_t>(),
-                           s->pos.as<float4>(), s->b().tri.as<float4>(), T);
-    }
-    {
-        ProfScope ps(s->ctx, st, "lbvh_leaf_bounds");
-        uint32_t ncap = (uint32_t)(2 * (size_t)T);
-        uint32_t g = rtx_div_up(ncap, BS);
-        hipLaunchKernelGGL(k_leaf_bounds, dim3(g > 4096 ? 4096 : g), dim3(BS), 0, st, s->b().tri.as<float4>(),
-                           s->nodes(), s->b().levels.as<uint32_t>());
-    }
-    fat_leaf_bounds(s, st, s->ctx);
-    refit_internal(s, st, s->depth, s->ctx);
+    tree_boxes<true>(s, st, scratch_of(s->b()), s->ctx);
     RTX_CHECK_HIP(hipGetLastError());
     return RTX_OK;
 }

@@ -70,7 +70,7 @@ struct rtx_tuning {
     int64_t xcds = 1;           // ray chunks = L2 domains (MI355X: 8 XCDs); 1 = plain grid order
     int64_t sort_bits = 8;      // LBVH radix sort digit width: 8 or 4 bits a pass
     int64_t sort_items = 16;    // LBVH radix sort: pairs per thread of a tile (16 or 32)
-    int64_t build_grid = 8;     // LBVH hierarchy and refit levels: persistent blocks per CU (1..16)
+    int64_t build_grid = 8;     // LBVH near-child difference pass: blocks per CU at most (1..16)
     int64_t stack_lds = 32;     // traversal stack entries per lane kept in LDS: 8, 16 or 32 (all)
     int64_t shadow_order = 0;   // 1: shadow rays visit children in the reference's near-child order everywhere;
                                 // 0: in index order (no delta fetch) wherever the order cannot change the result
@@ -123,22 +123,22 @@ struct BuildSet {
     DevBuf gbox;        // 6 x int32 ordered-float keys
     DevBuf levels;      // uint32: [0..64) level offsets, [64..128) level counts, [128] node count
     // build scratch
-    DevBuf bstart, bend;          // per-node build state: triangle range
+    DevBuf span;                  // per split: its node's range, number and children (kept for refit)
     DevBuf keys_alt, vals_alt;    // radix ping-pong
     DevBuf centroid, partials;    // per-triangle centroids, per-block AABB partials
     DevBuf sort_hist;             // [4][256] digit histograms -> exclusive offsets
     DevBuf sort_status;           // look-back words, per pass x tile x digit
     DevBuf tickets;               // tile tickets for every ordered kernel
-    DevBuf hier_status;           // look-back words, per level x tile
-    DevBuf fat;                   // node ids of the leaves bounded by one wave each (kept for refit)
+    DevBuf rank_status;           // look-back words of the ranks, per tile x level
+    DevBuf tree_tiles;            // tile boxes and crossing nodes of the box kernels
     // Node i lives at byte 32 + 32 i of `node`: left children have odd ids, so
     // every sibling pair (i, i + 1) fills one 64-byte aligned chunk.
     float4* nodes() const { return reinterpret_cast<float4*>(static_cast<char*>(node.p) + 32); }
     template <class F>
     void each(F f) {
         DevBuf* all[] = {&node,     &delta,    &parent,   &tri,       &codes,       &perm,    &gbox,
-                         &levels,   &bstart,   &bend,     &keys_alt,  &vals_alt,    &centroid, &partials,
-                         &sort_hist, &sort_status, &tickets, &hier_status, &fat};
+                         &levels,   &span,     &keys_alt, &vals_alt,  &centroid,    &partials, &sort_hist,
+                         &sort_status, &tickets, &rank_status, &tree_tiles};
         for (DevBuf* d : all) f(*d);
     }
 };
