@@ -597,7 +597,7 @@ def build_stage_rooflines(kernels, T, nodes):
     stages = {
         "prim_bounds_morton": (("lbvh_prim_bounds", "lbvh_morton"), 76.0 * T),
         "permutation": (("lbvh_rearrange",), 36.0 * T),
-        "refit": (("lbvh_boxes", "lbvh_cross", "lbvh_deltas"), 28.0 * T + 32.0 * nl + 80.0 * ni),
+        "refit": (("lbvh_boxes", "lbvh_cross", "lbvh_pairs"), 28.0 * T + 32.0 * nl + 80.0 * ni),
         "sort_all_passes": (("lbvh_sort_pass",), 16.0 * T * 4),
         # the same passes against 4 + 16 P_s B per element (one key read for
         # the digit histograms, then key and value read and written per pass)

@@ -213,7 +213,7 @@ uint64_t rtx_mem_in_use(rtx_ctx* ctx);
  *                    30-bit codes) or 4 (8 passes, longer scatter runs).
  *   "sort_items":    LBVH radix sort pairs per thread of a tile: 16 (default)
  *                    or 32.
- *   "build_grid":    LBVH near-child difference pass: blocks per CU at most
+ *   "build_grid":    LBVH pass over the child pairs: blocks per CU at most
  *                    (1..16, default 8).
  * All settings give identical results. */
 int32_t rtx_tune_set(rtx_ctx* ctx, const char* key, int64_t value);

@@ -355,7 +355,7 @@ uint64_t rtx_scene_device_bytes(const rtx_scene* sc) {
     uint64_t b = 0;
     for (const DevBuf* d : all) b += d->p ? d->bytes : 0;
     for (auto& set : s->sets) set.each([&](DevBuf& d) { b += d.p ? d.bytes : 0; });
-    for (const auto& c : s->rc) b += c.node.bytes + c.delta.bytes + c.tri.bytes + c.nrm.bytes + c.matmap.bytes;
+    for (const auto& c : s->rc) b += c.node.bytes + c.delta.bytes + c.tri.bytes + c.nrm.bytes + c.matmap.bytes + c.wide.bytes;
     return b;
 }
 
@@ -372,6 +372,7 @@ int32_t rtx_scene_destroy(rtx_scene* s) {
         c.tri.release();
         c.nrm.release();
         c.matmap.release();
+        c.wide.release();
     }
     for (DevBuf* b : all) b->release();
     delete s;

@@ -15,6 +15,7 @@
 #include "devmath.hpp"
 #include "lookback.hpp"
 #include "rtx_impl.hpp"
+#include "wide.hpp"
 
 namespace {
 
@@ -903,21 +904,72 @@ __global__ __launch_bounds__(BS) void k_cross(float4* __restrict__ node, TreeTil
     }
 }
 
-// The near-child differences right.lo - left.lo of the inner nodes.
-__global__ __launch_bounds__(BS) void k_deltas(const float4* __restrict__ node, float4* __restrict__ delta,
-                                               const uint32_t* __restrict__ levels) {
-    const uint32_t N = levels[LV_TOTAL];
-    for (uint32_t n = blockIdx.x * BS + threadIdx.x; n < N; n += gridDim.x * BS) {
-        const uint32_t l = __float_as_uint(node[2 * (size_t)n].w), cnt = __float_as_uint(node[2 * (size_t)n + 1].w);
-        if (cnt) continue;
-        const v3 dl = xyz(node[2 * (size_t)l + 2]) - xyz(node[2 * (size_t)l]);
-        delta[n] = make_float4(dl.x, dl.y, dl.z, 0.f);
+// One pass over the child pairs (pair k: nodes 1 + 2k and 2 + 2k), four lanes
+// each: the near-child difference right.lo - left.lo of their parent and, where
+// the parent is at an even level, its wide record (wide.hpp), number k, one
+// slot per lane.  by_level: the tree is level-ordered and its level table gives
+// a node's level; else the level is the length of its parent chain.  Reads and
+// writes run through the arrays in order (HBM bound: 1M triangles 25 us for
+// 110 MB, 13 of them the differences alone).
+__global__ __launch_bounds__(BS) void k_pairs(const float4* __restrict__ node, const uint32_t* __restrict__ parent,
+                                              float4* __restrict__ delta, float4* __restrict__ wide,
+                                              const uint32_t* __restrict__ levels, int by_level) {
+    __shared__ uint32_t s_off[64];
+    const uint32_t pairs = (levels[LV_TOTAL] - 1u) >> 1, q = threadIdx.x & 3u;
+    if (threadIdx.x < 64) s_off[threadIdx.x] = levels[LV_CNT + threadIdx.x] ? levels[LV_OFF + threadIdx.x] : NONE;
+    __syncthreads();
+    for (uint32_t k = (blockIdx.x * BS + threadIdx.x) >> 2; k < pairs; k += gridDim.x * (BS / 4)) {
+        const uint32_t c = 1u + 2u * k + (q >> 1), n = parent[c];
+        const float4 f0 = node[2 * (size_t)c], f1 = node[2 * (size_t)c + 1];
+        const v3 right = mk3(__shfl_down(f0.x, 2, 4), __shfl_down(f0.y, 2, 4), __shfl_down(f0.z, 2, 4));
+        if (q == 0u) {
+            const v3 dl = right - xyz(f0);
+            delta[n] = make_float4(dl.x, dl.y, dl.z, 0.f);
+        }
+        if (!wide) continue;
+        int d = 0;  // the parent's level
+        if (by_level) {
+            while (d + 2 < 64 && s_off[d + 2] <= c) ++d;
+        } else {
+            for (uint32_t p = n; p; p = parent[p]) ++d;
+        }
+        if (d & 1) continue;
+        const uint32_t a = __float_as_uint(f0.w), cnt = __float_as_uint(f1.w);
+        float4 g0 = f0, g1 = f1;
+        uint32_t ref;
+        if (cnt == 0u) {
+            const uint32_t g = a + (q & 1u);
+            g0 = node[2 * (size_t)g];
+            g1 = node[2 * (size_t)g + 1];
+            const uint32_t ga = __float_as_uint(g0.w), gc = __float_as_uint(g1.w);
+            ref = wide_ref(g, ga, gc);
+            // an inner child at level 31 below this slot's node at level 30
+            if (d == 28 && gc == 0u &&
+                (__float_as_uint(node[2 * (size_t)ga + 1].w) == 0u || __float_as_uint(node[2 * (size_t)ga + 3].w) == 0u))
+                ref |= WIDE_DEEP;
+        } else if ((q & 1u) == 0u) {
+            ref = wide_ref(c, a, cnt);
+        } else {
+            ref = WIDE_EMPTY;
+            g0 = g1 = make_float4(INFINITY, INFINITY, INFINITY, 0.f);
+        }
+        float4* out = wide + 8 * (size_t)k + 2 * q;
+        out[0] = make_float4(g0.x, g0.y, g0.z, __uint_as_float(ref));
+        out[1] = make_float4(g1.x, g1.y, g1.z, 0.f);
     }
 }
 
 }  // namespace
 
 // ------------------------------------------------------------------ host --
+static void write_pairs(rtx_scene* s, hipStream_t st, bool by_level, rtx_ctx* pc) {
+    ProfScope ps(pc, st, "lbvh_pairs");
+    const uint32_t g = rtx_div_up(2ull * s->T, BS), gmax = (uint32_t)s->ctx->cus * (uint32_t)s->ctx->tune.build_grid;
+    hipLaunchKernelGGL(k_pairs, dim3(g > gmax ? gmax : g), dim3(BS), 0, st, s->nodes(), s->b().parent.as<uint32_t>(),
+                       s->b().delta.as<float4>(), s->T <= WIDE_MAX_TRIS ? s->b().wide.as<float4>() : nullptr,
+                       s->b().levels.as<uint32_t>(), by_level ? 1 : 0);
+}
+
 static int32_t lbvh_alloc(rtx_scene* s, uint32_t T, int depth) {
     rtx_ctx* c = s->ctx;
     size_t ncap = 2 * (size_t)T;
@@ -928,6 +980,7 @@ static int32_t lbvh_alloc(rtx_scene* s, uint32_t T, int depth) {
     if ((e = s->b().node.reserve(c, ncap * 32 + 64))) return e;
     if ((e = s->b().delta.reserve(c, ncap * 16))) return e;
     if ((e = s->b().parent.reserve(c, ncap * 4))) return e;
+    if (T <= WIDE_MAX_TRIS && (e = s->b().wide.reserve(c, (size_t)T * 128))) return e;
     if ((e = s->b().span.reserve(c, (size_t)T * 16))) return e;
     if ((e = s->b().tri.reserve(c, (size_t)T * 48))) return e;
     if ((e = s->b().codes.reserve(c, (size_t)T * 4))) return e;
@@ -976,12 +1029,11 @@ static TreeArgs tree_args(rtx_scene* s, const BuildScratch& W) {
 }
 
 // Boxes of all nodes (REFIT: of the kept topology, from the current
-// positions), then the near-child differences.
+// positions), then the child pairs' differences and wide records.
 template <bool REFIT>
 static void tree_boxes(rtx_scene* s, hipStream_t st, const BuildScratch& W, rtx_ctx* pc) {
     const TreeArgs A = tree_args(s, W);
     const uint32_t tiles = rtx_div_up(s->T, TREE_TILE);
-    const uint32_t gmax = (uint32_t)s->ctx->cus * (uint32_t)s->ctx->tune.build_grid;
     {
         ProfScope ps(pc, st, "lbvh_boxes");
         hipLaunchKernelGGL((k_boxes<REFIT>), dim3(tiles), dim3(BOX_THREADS), 0, st, A);
@@ -990,12 +1042,7 @@ static void tree_boxes(rtx_scene* s, hipStream_t st, const BuildScratch& W, rtx_
         ProfScope ps(pc, st, "lbvh_cross");
         hipLaunchKernelGGL(k_cross, dim3(tiles), dim3(BS), 0, st, s->nodes(), A.tiles, s->T);
     }
-    {
-        ProfScope ps(pc, st, "lbvh_deltas");
-        const uint32_t g = rtx_div_up(s->T, BS);
-        hipLaunchKernelGGL(k_deltas, dim3(g > gmax ? gmax : g), dim3(BS), 0, st, s->nodes(),
-                           s->b().delta.as<float4>(), s->b().levels.as<uint32_t>());
-    }
+    write_pairs(s, st, true, pc);
 }
 
 // Depth and leaf size of a build, clamped as the reference's RendererConfig
@@ -1249,6 +1296,7 @@ int32_t rtx_lbvh_build_noalloc(rtx_scene* s, const rtx_lbvh_params* p, void* str
     const size_t T = s->T, ncap = 2 * T;
     BuildSet& b = s->b();
     RTX_REQUIRE(b.node.bytes >= ncap * 32 + 64 && b.delta.bytes >= ncap * 16 && b.parent.bytes >= ncap * 4 &&
+                    (T > WIDE_MAX_TRIS || b.wide.bytes >= T * 128) &&
                     b.tri.bytes >= T * 48 && b.codes.bytes >= T * 4 && b.perm.bytes >= T * 4 && b.gbox.bytes >= 32 &&
                     b.levels.bytes >= LV_WORDS * 4 && b.span.bytes >= T * 16,
                 RTX_ESTATE,
@@ -1340,6 +1388,7 @@ int32_t rtx_sah_build(rtx_scene* s, void* stream) {
     RTX_CHECK_HIP(hipMemcpy(b.levels.p, lv.data(), LV_WORDS * 4, hipMemcpyHostToDevice));
     hipLaunchKernelGGL(k_tri_records, dim3(rtx_div_up(T, BS)), dim3(BS), 0, st, s->idx.as<uint32_t>(),
                        s->pos.as<float4>(), b.tri.as<float4>(), T);
+    write_pairs(s, st, false, s->ctx);
     RTX_CHECK_HIP(hipGetLastError());
     RTX_CHECK_HIP(hipStreamSynchronize(st));
     s->built = true;

@@ -18,9 +18,9 @@ __global__ void k_zero_u64(unsigned long long* p, int n) {
 }
 // Device copy of up to 5 u32 arrays (the render copy of a scene), grid-stride.
 struct CopySegs {
-    uint32_t* dst[5];
-    const uint32_t* src[5];
-    uint64_t n[5];
+    uint32_t* dst[6];
+    const uint32_t* src[6];
+    uint64_t n[6];
     int count;
 };
 __global__ __launch_bounds__(256) void k_copy_segs(CopySegs c) {
@@ -48,7 +48,8 @@ int32_t rtx_reserve_render_copy(rtx_scene* s, int k, bool shading_only) {
         return e;
     if (shading_only) return RTX_OK;
     if ((e = rc.node.reserve(s->ctx, s->b().node.bytes)) || (e = rc.delta.reserve(s->ctx, s->b().delta.bytes)) ||
-        (e = rc.tri.reserve(s->ctx, (uint64_t)s->T * 48)))
+        (e = rc.tri.reserve(s->ctx, (uint64_t)s->T * 48)) ||
+        (s->b().wide.p && (e = rc.wide.reserve(s->ctx, s->b().wide.bytes))))
         return e;
     return RTX_OK;
 }
@@ -64,11 +65,12 @@ int32_t rtx_refresh_render_copy(rtx_scene* s, int k, hipStream_t st, bool shadin
 // material ids) into rc, on `st`.
 int32_t rtx_copy_render_state(rtx_scene* s, rtx_scene::RenderCopy& rc, hipStream_t st, bool shading_only) {
     int32_t e;
-    DevBuf* src[5] = {&s->nrm, &s->matmap, &s->b().node, &s->b().delta, &s->b().tri};
-    DevBuf* dst[5] = {&rc.nrm, &rc.matmap, &rc.node, &rc.delta, &rc.tri};
-    const uint64_t bytes[5] = {(uint64_t)s->V * 16, (uint64_t)s->T * 4, s->b().node.bytes, s->b().delta.bytes,
-                               (uint64_t)s->T * 48};
-    const int n = shading_only ? 2 : 5;
+    DevBuf* src[6] = {&s->nrm, &s->matmap, &s->b().node, &s->b().delta, &s->b().tri, &s->b().wide};
+    DevBuf* dst[6] = {&rc.nrm, &rc.matmap, &rc.node, &rc.delta, &rc.tri, &rc.wide};
+    const uint64_t bytes[6] = {(uint64_t)s->V * 16, (uint64_t)s->T * 4, s->b().node.bytes, s->b().delta.bytes,
+                               (uint64_t)s->T * 48, s->b().wide.bytes};
+    const int n = shading_only ? 2 : s->b().wide.p ? 6 : 5;
+    if (!shading_only && n < 6) rc.wide.release();
     CopySegs c{};
     for (int j = 0; j < n; ++j) {
         RTX_REQUIRE(src[j]->p && src[j]->bytes >= bytes[j], RTX_ESTATE, "render copy: scene not built");

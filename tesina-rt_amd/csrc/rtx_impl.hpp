@@ -70,7 +70,7 @@ struct rtx_tuning {
     int64_t xcds = 1;           // ray chunks = L2 domains (MI355X: 8 XCDs); 1 = plain grid order
     int64_t sort_bits = 8;      // LBVH radix sort digit width: 8 or 4 bits a pass
     int64_t sort_items = 16;    // LBVH radix sort: pairs per thread of a tile (16 or 32)
-    int64_t build_grid = 8;     // LBVH near-child difference pass: blocks per CU at most (1..16)
+    int64_t build_grid = 8;     // LBVH pass over the child pairs (k_pairs): blocks per CU at most (1..16)
     int64_t stack_lds = 32;     // traversal stack entries per lane kept in LDS: 8, 16 or 32 (all)
     int64_t shadow_order = 0;   // 1: shadow rays visit children in the reference's near-child order everywhere;
                                 // 0: in index order (no delta fetch) wherever the order cannot change the result
@@ -120,6 +120,7 @@ struct ProfScope {
 // triangle records, sorted codes) and its scratch.
 struct BuildSet {
     DevBuf node, delta, parent, tri, codes, perm;
+    DevBuf wide;        // wide records (wide.hpp); none for trees of more than WIDE_MAX_TRIS triangles
     DevBuf gbox;        // 6 x int32 ordered-float keys
     DevBuf levels;      // uint32: [0..64) level offsets, [64..128) level counts, [128] node count
     // build scratch
@@ -136,7 +137,7 @@ struct BuildSet {
     float4* nodes() const { return reinterpret_cast<float4*>(static_cast<char*>(node.p) + 32); }
     template <class F>
     void each(F f) {
-        DevBuf* all[] = {&node,     &delta,    &parent,   &tri,       &codes,       &perm,    &gbox,
+        DevBuf* all[] = {&node,     &delta,    &parent,   &tri,       &codes,       &perm,    &wide,     &gbox,
                          &levels,   &span,     &keys_alt, &vals_alt,  &centroid,    &partials, &sort_hist,
                          &sort_status, &tickets, &rank_status, &tree_tiles};
         for (DevBuf* d : all) f(*d);
@@ -169,7 +170,7 @@ struct rtx_scene {
     // render from copies).  use_copy selects one for the launches being
     // enqueued (-1: the build's own buffers).
     struct RenderCopy {
-        DevBuf node, delta, tri, nrm, matmap;
+        DevBuf node, delta, tri, nrm, matmap, wide;
     };
     static constexpr int COPIES = 8;
     RenderCopy rc[COPIES];
@@ -218,13 +219,14 @@ struct SceneView {
     const float4* nrm;
     const int32_t* matmap;
     const uint32_t* parent;  // node parents (the stackless walk); null for a render copy
+    const float4* wide;      // wide records; null where the tree has none
 };
 inline SceneView scene_view(const rtx_scene* s) {
     if (s->ext) {
         const rtx_scene::RenderCopy& c = s->ext->copy;
         return SceneView{reinterpret_cast<const float4*>(static_cast<const char*>(c.node.p) + 32),
                          c.delta.as<float4>(), c.tri.as<float4>(), c.nrm.as<float4>(), c.matmap.as<int32_t>(),
-                         nullptr};
+                         nullptr, c.wide.as<float4>()};
     }
     if (s->use_set >= 0) {
         const BuildSet& b = s->sets[s->use_set];
@@ -232,16 +234,16 @@ inline SceneView scene_view(const rtx_scene* s) {
         return SceneView{b.nodes(), b.delta.as<float4>(), b.tri.as<float4>(),
                          c ? s->rc[s->use_copy].nrm.as<float4>() : s->nrm.as<float4>(),
                          c ? s->rc[s->use_copy].matmap.as<int32_t>() : s->matmap.as<int32_t>(),
-                         b.parent.as<uint32_t>()};
+                         b.parent.as<uint32_t>(), b.wide.as<float4>()};
     }
     if (s->use_copy >= 0) {
         const rtx_scene::RenderCopy& c = s->rc[s->use_copy];
         return SceneView{reinterpret_cast<const float4*>(static_cast<const char*>(c.node.p) + 32),
                          c.delta.as<float4>(), c.tri.as<float4>(), c.nrm.as<float4>(), c.matmap.as<int32_t>(),
-                         nullptr};
+                         nullptr, c.wide.as<float4>()};
     }
     return SceneView{s->nodes(), s->b().delta.as<float4>(), s->b().tri.as<float4>(), s->nrm.as<float4>(),
-                     s->matmap.as<int32_t>(), s->b().parent.as<uint32_t>()};
+                     s->matmap.as<int32_t>(), s->b().parent.as<uint32_t>(), s->b().wide.as<float4>()};
 }
 
 struct rtx_rays {
@@ -404,6 +406,7 @@ struct WfSeg {
     // scene (resident, built)
     const float4* node;
     const float4* delta;
+    const float4* wide;  // null where the scene has no wide records (the step then uses no WF_WIDE launch)
     const float4* tri;
     const float4* nrm;
     const float2* uv;
@@ -469,6 +472,8 @@ enum {
 // secondary.hip).  `any_*` says whether some segment needs the stage.
 void rtx_wf_init(const WfSeg* segs, uint32_t nseg, uint32_t* ctr, hipStream_t st);
 void rtx_wf_raygen(const WfSeg* segs, uint32_t nseg, uint64_t pixels, int cus, hipStream_t st);
+// var: a traversal form (trace_variant 0 to 2), or WF_WIDE: the wide walk.
+constexpr int WF_WIDE = -1;
 // sched 1: persistent waves over per-XCD queues; 0: one chunk per wave in
 // launch order over a grid of `max_chunks` (an upper bound of the chunks).
 void rtx_wf_trace(const WfSeg* segs, uint32_t nseg, uint32_t* ctr, int var, int tb, int sr, uint32_t coop,

@@ -21,6 +21,7 @@
 #include "rtx_impl.hpp"
 #include "stack.hpp"
 #include "wavefront.hpp"
+#include "wide.hpp"
 
 namespace {
 
@@ -659,6 +660,348 @@ __device__ bool traverse_any_ns(const float4* __restrict__ node, const float4* _
     return false;
 }
 
+// ------------------------------------------------------- wide walk -------
+// Four lanes per ray over the wide records (wide.hpp): each lane tests one
+// slot, so a step costs one 128-byte line and one box test of latency for two
+// levels of the tree, and a wave holds 16 rays instead of waiting for the
+// slowest of 64.
+//
+// Equality with the node-by-node walk.  The reference visits leaves in a
+// fixed depth-first order of the ray (near child first by
+// dot(dir, right.lo - left.lo) > 0) and tests a leaf whose box, and whose
+// ancestors' boxes, pass the slab test at the tMax of their visit.  The box
+// differences that order the children are those of the slots (a left child's
+// lo is the minimum of its children's), so the order is the same.  A box's
+// entry distance t0 is kept with its stack entry and compared with the
+// current tMax when the entry is popped, which is the slab test at that time
+// (the exit side was tested at the push, and tMax only shrinks).  The boxes of
+// the odd levels in between are not tested: float subtraction, multiplication,
+// min and max are monotone, so a box inside another has the later entry and
+// the earlier exit and passes only where the outer box passes.
+// Two kinds of rays are walked node by node instead (exact_*): those with an
+// axis whose 1/dir is infinite (0 * inf is NaN, which min and max drop, and
+// the argument fails), and those that pass a WIDE_DEEP node, below which the
+// reference's stack count can reach MAX_LEVELS.
+
+// Value of lane (lane ^ 1), (lane ^ 2) of the group of four, or of its lane 0.
+constexpr int QX1 = 0xB1, QX2 = 0x4E, QFIRST = 0x00;
+template <int CTRL>
+__device__ __forceinline__ int quad_i(int x) {
+    return __builtin_amdgcn_mov_dpp(x, CTRL, 0xf, 0xf, true);
+}
+template <int CTRL>
+__device__ __forceinline__ float quad_f(float x) {
+    return __int_as_float(quad_i<CTRL>(__float_as_int(x)));
+}
+template <int CTRL>
+__device__ __forceinline__ v3 quad_v(v3 a) {
+    return mk3(quad_f<CTRL>(a.x), quad_f<CTRL>(a.y), quad_f<CTRL>(a.z));
+}
+
+// Ray constants of the wide walk: a skipped axis (RayC::ax etc. false) has a
+// NaN reciprocal, which min and max drop like the skip.  The origin,
+// direction and tMin are those of the ray.
+struct WideRay {
+    v3 o, d, inv;
+    float tmin;
+};
+__device__ __forceinline__ WideRay wide_ray(const RayC& r) {
+    const float skip = __builtin_nanf("");
+    return WideRay{r.o, r.d, mk3(r.ax ? r.inv.x : skip, r.ay ? r.inv.y : skip, r.az ? r.inv.z : skip), r.tmin};
+}
+__device__ __forceinline__ bool wide_odd(const RayC& r) { return isinf(r.inv.x) || isinf(r.inv.y) || isinf(r.inv.z); }
+
+// slab() with the entry distance.
+__device__ __forceinline__ bool wide_slab(float4 lo4, float4 hi4, const WideRay& r, float tmax, float& t0) {
+    const v3 tl = (xyz(lo4) - r.o) * r.inv, th = (xyz(hi4) - r.o) * r.inv;
+    const v3 tM = vmax(tl, th), tm = vmin(tl, th);
+    t0 = fmaxf(fmaxf(fmaxf(r.tmin, tm.x), tm.y), tm.z);
+    const float t1 = fminf(fminf(fminf(tmax, tM.x), tM.y), tM.z);
+    return t0 <= t1;
+}
+
+// Stack of a group in LDS: entry lv of the block's groups side by side.
+template <int GROUPS>
+struct WideStack {
+    uint2* e;
+    __device__ __forceinline__ void put(int lv, uint32_t ref, float t0) {
+        e[lv * GROUPS] = make_uint2(ref, __float_as_uint(t0));
+    }
+    __device__ __forceinline__ uint2 get(int lv) const { return e[lv * GROUPS]; }
+};
+
+// Orders the pushes of a group's lanes before the pops of its other lanes (one
+// wave: no instruction, only the compiler is held).
+__device__ __forceinline__ void wide_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// A step's outcome on a lane: whether its slot's box passes, its entry
+// distance, how many of the passing slots are visited after it, and how many
+// pass in all.  ORDERED: in the ray's child order, else in slot order.
+struct WideStep {
+    bool pass;
+    float t0;
+    int after, total;
+};
+template <bool ORDERED>
+__device__ __forceinline__ WideStep wide_step(float4 f0, float4 f1, const WideRay& r, float tmax, uint32_t q) {
+    WideStep s;
+    s.pass = wide_slab(f0, f1, r, tmax, s.t0) && __float_as_uint(f0.w) != WIDE_EMPTY;
+    bool first = (q & 1u) == 0u, first_pair = (q & 2u) == 0u;
+    if (ORDERED) {
+        // dot(d, right.lo - left.lo) on the right lane, its exact negation on the left
+        const v3 lo = xyz(f0), sib = quad_v<QX1>(lo);
+        const float din = dot(r.d, lo - sib);
+        first = first ? din < 0.f : !(din > 0.f);
+        const v3 plo = vmin(lo, sib);
+        const float dout = dot(r.d, plo - quad_v<QX2>(plo));
+        first_pair = first_pair ? dout < 0.f : !(dout > 0.f);
+    }
+    const int me = s.pass ? 1 : 0;
+    const int sib = quad_i<QX1>(me), pair = me + sib, other = quad_i<QX2>(pair);
+    s.total = pair + other;
+    s.after = (first_pair ? other : 0) + (first ? sib : 0);
+    return s;
+}
+
+// The triangles of leaf entry `e`.
+__device__ __forceinline__ void wide_leaf(const float4* __restrict__ node, uint32_t e, uint32_t& first,
+                                          uint32_t& cnt) {
+    cnt = (e >> 27) & 15u;
+    first = e & WIDE_LOW;
+    if (cnt == 0u) {
+        const float4* p = node + 2 * (size_t)first;
+        first = __float_as_uint(p[0].w);
+        cnt = __float_as_uint(p[1].w);
+    }
+}
+
+// The root's entry, when its box passes.
+__device__ __forceinline__ bool wide_root(const float4* __restrict__ node, const WideRay& r, float tmax, uint32_t& ref,
+                                          float& t0) {
+    const float4 f0 = node[0], f1 = node[1];
+    ref = wide_ref(0u, __float_as_uint(f0.w), __float_as_uint(f1.w));
+    return wide_slab(f0, f1, r, tmax, t0);
+}
+
+// Closest hit of the group's ray; called by the whole wave, `start` the same
+// on the four lanes.  best is kept equal on them.  Leaves are tested four
+// triangles at a time, one per lane, leaves of at least `coop` triangles by
+// the whole wave.  True: the ray has to be walked by exact_closest instead.
+template <int GROUPS>
+__device__ __forceinline__ bool wide_closest(const float4* __restrict__ node, const float4* __restrict__ wide,
+                                             const float4* __restrict__ tri, const WideRay& r, Closest& best,
+                                             WideStack<GROUPS> stk, uint32_t coop, bool start) {
+    const uint32_t q = lane_id() & 3u;
+    int level = 0;
+    bool redo = false;
+    if (start) {
+        uint32_t ref;
+        float t0;
+        if (wide_root(node, r, best.t, ref, t0)) {
+            stk.put(0, ref, t0);
+            level = 1;
+        }
+    }
+    while (ballot(level > 0)) {
+        wide_sync();
+        uint32_t la = 0, lcnt = 0;
+        if (level > 0) {
+            const uint2 e = stk.get(--level);
+            if (__uint_as_float(e.y) <= best.t) {
+                // the slot or the group's first four triangles: one round trip
+                // whichever a group needs
+                const bool leaf = (e.x & WIDE_LEAF) != 0u;
+                uint32_t first = 0, cnt = 0;
+                const char* p = reinterpret_cast<const char*>(wide) + ((e.x << 7) | (q << 5));
+                if (leaf) {
+                    wide_leaf(node, e.x, first, cnt);
+                    p = reinterpret_cast<const char*>(tri) + 48 * (size_t)(first + (q < cnt ? q : 0u));
+                }
+                const float4* p4 = reinterpret_cast<const float4*>(p);
+                float4 f0 = p4[0], f1 = p4[1], f2 = make_float4(0.f, 0.f, 0.f, 0.f);
+                if (leaf) f2 = p4[2];
+                if (!leaf) {
+                    if (e.x & WIDE_DEEP) {
+                        redo = true;
+                        level = 0;
+                    } else {
+                        const WideStep s = wide_step<true>(f0, f1, r, best.t, q);
+                        if (s.pass) stk.put(level + s.after, __float_as_uint(f0.w), s.t0);
+                        level += s.total;
+                    }
+                } else if (cnt >= coop) {
+                    la = first;
+                    lcnt = cnt;
+                } else {
+                    for (uint32_t b = 0;;) {
+                        const uint32_t i = b + q;
+                        float tt, u, v;
+                        const bool h =
+                            tri_hit_v(f0, f1, f2, r.o, r.d, &tt, &u, &v) && i < cnt && tt <= best.t && tt >= r.tmin;
+                        if (ballot(h)) {
+                            // the smallest t and, among equal ones, the latest triangle: what the
+                            // in-order loop with its `t <= best` update keeps
+                            int id = h ? (int)(first + i) : -1;
+                            tt = h ? tt : INFINITY;
+#pragma unroll
+                            for (int x = 0; x < 2; ++x) {
+                                const float ot = x ? quad_f<QX2>(tt) : quad_f<QX1>(tt);
+                                const float ou = x ? quad_f<QX2>(u) : quad_f<QX1>(u);
+                                const float ov = x ? quad_f<QX2>(v) : quad_f<QX1>(v);
+                                const int oi = x ? quad_i<QX2>(id) : quad_i<QX1>(id);
+                                const bool take = ot < tt || (ot == tt && oi > id);
+                                tt = take ? ot : tt;
+                                u = take ? ou : u;
+                                v = take ? ov : v;
+                                id = take ? oi : id;
+                            }
+                            if (id >= 0) best = Closest{tt, u, v, id};
+                        }
+                        b += 4;
+                        if (b >= cnt) break;
+                        const float4* t4 = tri + 3 * (size_t)(first + (b + q < cnt ? b + q : 0u));
+                        f0 = t4[0];
+                        f1 = t4[1];
+                        f2 = t4[2];
+                    }
+                }
+            }
+        }
+        if (ballot(lcnt != 0u)) {
+            RayC rc;
+            rc.o = r.o;
+            rc.d = r.d;
+            rc.tmin = r.tmin;
+            coop_closest(tri, la, q == 0u ? lcnt : 0u, rc, best, ~0ull);
+            best.t = quad_f<QFIRST>(best.t);
+            best.u = quad_f<QFIRST>(best.u);
+            best.v = quad_f<QFIRST>(best.v);
+            best.id = quad_i<QFIRST>(best.id);
+        }
+    }
+    return redo;
+}
+
+// Any hit with tMin < t < tMax.  ORDERED where the order can matter (trees of
+// 32 levels); `redo` as above.
+template <bool ORDERED, int GROUPS>
+__device__ __forceinline__ bool wide_any(const float4* __restrict__ node, const float4* __restrict__ wide,
+                                         const float4* __restrict__ tri, const WideRay& r, float tmax,
+                                         WideStack<GROUPS> stk, uint32_t coop, bool start, bool& redo) {
+    const uint32_t q = lane_id() & 3u;
+    int level = 0;
+    bool found = false;
+    if (start) {
+        uint32_t ref;
+        float t0;
+        if (wide_root(node, r, tmax, ref, t0)) {
+            stk.put(0, ref, t0);
+            level = 1;
+        }
+    }
+    while (ballot(level > 0)) {
+        wide_sync();
+        uint32_t la = 0, lcnt = 0;
+        if (level > 0) {
+            const uint32_t e = stk.get(--level).x;
+            const bool leaf = (e & WIDE_LEAF) != 0u;
+            uint32_t first = 0, cnt = 0;
+            const char* p = reinterpret_cast<const char*>(wide) + ((e << 7) | (q << 5));
+            if (leaf) {
+                wide_leaf(node, e, first, cnt);
+                p = reinterpret_cast<const char*>(tri) + 48 * (size_t)(first + (q < cnt ? q : 0u));
+            }
+            const float4* p4 = reinterpret_cast<const float4*>(p);
+            float4 f0 = p4[0], f1 = p4[1], f2 = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (leaf) f2 = p4[2];
+            if (!leaf) {
+                if (ORDERED && (e & WIDE_DEEP)) {
+                    redo = true;
+                    level = 0;
+                } else {
+                    const WideStep s = wide_step<ORDERED>(f0, f1, r, tmax, q);
+                    if (s.pass) stk.put(level + s.after, __float_as_uint(f0.w), s.t0);
+                    level += s.total;
+                }
+            } else if (cnt >= coop) {
+                la = first;
+                lcnt = cnt;
+            } else {
+                int h = 0;
+                for (uint32_t b = 0;;) {
+                    float tt, u, v;
+                    if (tri_hit_v(f0, f1, f2, r.o, r.d, &tt, &u, &v) && b + q < cnt && tt < tmax && tt > r.tmin) h = 1;
+                    b += 4;
+                    if (b >= cnt) break;
+                    const float4* t4 = tri + 3 * (size_t)(first + (b + q < cnt ? b + q : 0u));
+                    f0 = t4[0];
+                    f1 = t4[1];
+                    f2 = t4[2];
+                }
+                h |= quad_i<QX1>(h);
+                h |= quad_i<QX2>(h);
+                if (h) {
+                    found = true;
+                    level = 0;
+                }
+            }
+        }
+        if (ballot(lcnt != 0u)) {
+            RayC rc;
+            rc.o = r.o;
+            rc.d = r.d;
+            rc.tmin = r.tmin;
+            const int h = coop_any(tri, la, q == 0u ? lcnt : 0u, rc, tmax, ~0ull) ? 1 : 0;
+            if (quad_i<QFIRST>(h)) {
+                found = true;
+                level = 0;
+            }
+        }
+    }
+    return found;
+}
+
+// The reference's walk, node by node, for the rays the wide walk leaves: the
+// steps of traverse_closest_node / traverse_any_node (near child first, pops
+// only below MAX_LEVELS) with the leaf loop a triangle at a time, the same on
+// the four lanes of a group.  Few rays come here, so it is kept small.
+template <bool ANY, int GROUPS>
+__device__ __forceinline__ bool exact_walk(const float4* __restrict__ node, const float4* __restrict__ delta,
+                                           const float4* __restrict__ tri, v3 o, v3 d, float tmin, Closest& best,
+                                           WideStack<GROUPS> stk) {
+    const RayC r = make_ray(o, d, tmin);
+    uint32_t level = 0, curr = 0;
+    for (;;) {
+        const float4 f0 = node[2 * (size_t)curr], f1 = node[2 * (size_t)curr + 1];
+        const uint32_t a = __float_as_uint(f0.w), cnt = __float_as_uint(f1.w);
+        if (slab(f0, f1, r, best.t)) {
+            if (cnt == 0u) {
+                const bool nl = dot(r.d, xyz(delta[curr])) > 0.f;
+                stk.put((int)(level & (STACK - 1)), nl ? a + 1u : a, 0.f);
+                ++level;
+                curr = nl ? a : a + 1u;
+                continue;
+            }
+#pragma unroll 1
+            for (uint32_t t = a; t < a + cnt; ++t) {
+                float tt, u, v;
+                if (!tri_hit_v(tri[3 * (size_t)t], tri[3 * (size_t)t + 1], tri[3 * (size_t)t + 2], r.o, r.d, &tt, &u, &v))
+                    continue;
+                if (ANY) {
+                    if (tt < best.t && tt > tmin) return true;
+                } else if (tt <= best.t && tt >= tmin) {
+                    best = Closest{tt, u, v, (int32_t)t};
+                }
+            }
+        }
+        if (level == 0 || level >= STACK) return false;
+        curr = stk.get((int)--level).x;
+    }
+}
+
 // Variant dispatch: 0 = single node, 1 = single node + early delta load,
 // 2 = sibling pairs.
 // Called by every lane of the wave; `start` says whether the lane has a ray.
@@ -789,6 +1132,79 @@ __global__ __launch_bounds__(TB) void k_trace(const float4* __restrict__ node, c
     }
 }
 
+// Where a closest-hit launch reads its rays and writes its records.
+struct TraceIo {
+    const float4* __restrict__ node;
+    const float4* __restrict__ delta;
+    const float4* __restrict__ wide;
+    const float4* __restrict__ tri;
+    const float4* __restrict__ nrm;
+    const float2* __restrict__ uvs;
+    const float4* __restrict__ ori4;
+    const float4* __restrict__ dir4;
+    uint32_t* __restrict__ flags;
+    float* __restrict__ t;
+    int32_t* __restrict__ id;
+    float2* __restrict__ bary;
+    float4* __restrict__ n4;
+    float4* __restrict__ p4;
+    float2* __restrict__ uv2;
+    uint32_t* __restrict__ list;
+    uint32_t* __restrict__ list_count;
+};
+
+// Closest hit and record of the group's ray rr, by the wide walk; called by
+// the whole wave.
+template <int GROUPS>
+__device__ __forceinline__ void wide_trace(const TraceIo& io, uint64_t rr, bool active, WideStack<GROUPS> stk,
+                                           uint32_t coop) {
+    Closest best{0.f, 0.f, 0.f, -1};
+    WideRay r{};
+    bool redo = false;
+    if (active) {
+        const float4 o = io.ori4[rr], dd = io.dir4[rr];
+        const RayC rc = make_ray(xyz(o), xyz(dd), o.w);
+        r = wide_ray(rc);
+        redo = wide_odd(rc);
+        best.t = dd.w;
+    }
+    if (wide_closest<GROUPS>(io.node, io.wide, io.tri, r, best, stk, coop, active && !redo)) redo = true;
+    if (redo) {
+        best = Closest{io.dir4[rr].w, 0.f, 0.f, -1};
+        exact_walk<false, GROUPS>(io.node, io.delta, io.tri, r.o, r.d, r.tmin, best, stk);
+    }
+    const bool mine = active && (lane_id() & 3u) == 0u, hit = mine && best.id >= 0;
+    const uint64_t hb = ballot(hit);
+    uint32_t wbase = 0;
+    if (hb) {
+        if (lane_id() == (uint32_t)__builtin_ctzll(hb))
+            wbase = atomicAdd(io.list_count, (uint32_t)__builtin_popcountll(hb));
+        wbase = __shfl(wbase, __builtin_ctzll(hb), RTX_WAVE);
+    }
+    if (!mine) return;
+    if (!hit) {
+        write_miss_record(rr, io.flags, io.t, io.id, io.bary, io.n4, io.p4, io.uv2);
+        return;
+    }
+    io.list[wbase + lanes_below(hb)] = (uint32_t)rr;
+    RayC rc;
+    rc.o = r.o;
+    rc.d = r.d;
+    write_hit_record(io.tri, io.nrm, io.uvs, rc, best, rr, io.flags, io.t, io.id, io.bary, io.n4, io.p4, io.uv2);
+}
+
+// The wide walk: a block of TB threads holds TB / 4 rays.
+template <int TB>
+__global__ __launch_bounds__(TB) void k_trace_w(TraceIo io, const uint32_t* __restrict__ dcount, uint64_t hcount,
+                                                uint32_t coop) {
+    constexpr int GROUPS = TB / 4;
+    __shared__ uint2 s_stk[WIDE_STACK * GROUPS];
+    const uint32_t group = threadIdx.x >> 2;
+    const uint64_t n = ray_count(dcount, hcount);
+    for (uint64_t base = (uint64_t)blockIdx.x * GROUPS; base < n; base += (uint64_t)gridDim.x * GROUPS)
+        wide_trace<GROUPS>(io, base + group, base + group < n, WideStack<GROUPS>{s_stk + group}, coop);
+}
+
 // Hit list from the flags (when hits were written from the host).
 __global__ __launch_bounds__(256) void k_hit_list(const uint32_t* __restrict__ flags, const uint32_t* dcount,
                                                   uint64_t hcount, uint32_t* __restrict__ hit_list,
@@ -917,6 +1333,102 @@ __global__ __launch_bounds__(TB) void k_shadow(const float4* __restrict__ node, 
         if (any_var<VAR>(node, delta, tri, rc, tmax, stk, coop, trace, parent, bound, ordered != 0))  // whole wave
             shadowed = true;
         if (valid) set_shadow_bit(&fl[rr], l, shadowed);
+    }
+    if (shadow_count) {
+        if (traced) atomicAdd(&s_cnt, traced);
+        __syncthreads();
+        if (threadIdx.x == 0 && s_cnt) atomicAdd(shadow_count, (unsigned long long)s_cnt);
+    }
+}
+
+// The shadow ray of point p toward light L (shadow_trace_single): false where
+// none is traced, with `shadowed` the result.
+__device__ __forceinline__ bool shadow_ray(const rtx_light& L, v3 p, v3& dir, float& tmax, bool& shadowed) {
+    tmax = 1e37f;
+    if (L.type == RTX_LIGHT_DIR) {
+        dir = -mk3(L.dir[0], L.dir[1], L.dir[2]);
+        return true;
+    }
+    if (L.type == RTX_LIGHT_SPOT) {
+        dir = normalize(mk3(L.pos[0], L.pos[1], L.pos[2]) - p);
+        if (!(dot(-dir, mk3(L.dir[0], L.dir[1], L.dir[2])) < L.angle)) return true;
+    } else if (L.type == RTX_LIGHT_POINT) {
+        const v3 toL = mk3(L.pos[0], L.pos[1], L.pos[2]) - p;
+        tmax = __builtin_sqrtf(dot(toL, toL));
+        dir = normalize(toL);
+        return true;
+    }
+    shadowed = true;
+    return false;
+}
+
+// Shadow bit of the group's (hit rr, light l) pair, by the wide walk; called
+// by the whole wave.  Returns whether a ray was traced.
+template <bool ORDERED, int GROUPS>
+__device__ __forceinline__ bool wide_shadow(const float4* __restrict__ node, const float4* __restrict__ delta,
+                                            const float4* __restrict__ wide, const float4* __restrict__ tri,
+                                            const rtx_lights* __restrict__ lights, const float4* __restrict__ p4,
+                                            uint32_t* __restrict__ flags, uint32_t rr, int l, bool valid,
+                                            WideStack<GROUPS> stk, uint32_t coop) {
+    WideRay r{};
+    float tmax = 1e37f;
+    bool shadowed = false, trace = false, redo = false;
+    if (valid) {
+        const v3 p = xyz(p4[rr]);
+        v3 dir = mk3(0.f, 0.f, 0.f);
+        trace = shadow_ray(lights->l[l], p, dir, tmax, shadowed);
+        if (trace) {
+            const RayC rc = make_ray(p, dir, 0.01f);
+            r = wide_ray(rc);
+            redo = wide_odd(rc);
+        }
+    }
+    if (wide_any<ORDERED, GROUPS>(node, wide, tri, r, tmax, stk, coop, trace && !redo, redo)) shadowed = true;
+    if (redo) {
+        Closest c{tmax, 0.f, 0.f, -1};
+        shadowed = exact_walk<true, GROUPS>(node, delta, tri, r.o, r.d, r.tmin, c, stk);
+    }
+    if (valid && (lane_id() & 3u) == 0u) set_shadow_bit(&flags[rr], l, shadowed);
+    return trace;
+}
+
+template <bool ORDERED, int TB>
+__global__ __launch_bounds__(TB) void k_shadow_w(const float4* __restrict__ node, const float4* __restrict__ delta,
+                                                 const float4* __restrict__ wide, const float4* __restrict__ tri,
+                                                 const rtx_lights* __restrict__ lights, ShadowSegs segs,
+                                                 unsigned long long* shadow_count, uint32_t coop) {
+    constexpr int GROUPS = TB / 4;
+    __shared__ uint2 s_stk[WIDE_STACK * GROUPS];
+    __shared__ uint32_t s_cnt;
+    __shared__ uint64_t s_end[RTX_SEG_MAX];
+    const uint32_t group = threadIdx.x >> 2;
+    const int nl = lights->count;
+    if (threadIdx.x == 0) {
+        s_cnt = 0;
+        uint64_t acc = 0;
+        for (int k = 0; k < segs.n; ++k) {
+            acc += (uint64_t)(*segs.s[k].count) * (uint64_t)nl;
+            s_end[k] = acc;
+        }
+    }
+    __syncthreads();
+    const uint64_t items = segs.n ? s_end[segs.n - 1] : 0;
+    uint32_t traced = 0;
+    for (uint64_t base = (uint64_t)blockIdx.x * GROUPS; base < items; base += (uint64_t)gridDim.x * GROUPS) {
+        const uint64_t it = base + group;
+        const bool valid = it < items;
+        uint32_t rr = 0;
+        int l = 0, sg = 0;
+        if (valid) {
+            while (it >= s_end[sg]) ++sg;
+            const uint64_t first = sg ? s_end[sg - 1] : 0, local = it - first, nh = (s_end[sg] - first) / (uint64_t)nl;
+            rr = segs.s[sg].list[local % nh];  // light-major, as k_shadow
+            l = (int)(local / nh);
+        }
+        if (wide_shadow<ORDERED, GROUPS>(node, delta, wide, tri, lights, segs.s[sg].p4, segs.s[sg].flags, rr, l, valid,
+                                         WideStack<GROUPS>{s_stk + group}, coop) &&
+            (threadIdx.x & 3u) == 0u)
+            ++traced;
     }
     if (shadow_count) {
         if (traced) atomicAdd(&s_cnt, traced);
@@ -2046,6 +2558,54 @@ __global__ __launch_bounds__(TB) void k_wf_trace_ord(const WfSeg* __restrict__ s
     wf_trace_chunk<VAR>(segs[sg], c - c0, stk, coop, threadIdx.x & (RTX_WAVE - 1));
 }
 
+// The same by the wide walk: the chunk's 64 rays as four rounds of 16.
+template <int GROUPS>
+__device__ __forceinline__ void wf_trace_chunk_w(const WfSeg& S, uint32_t cl, WideStack<GROUPS> stk, uint32_t coop,
+                                                 uint32_t lane) {
+    constexpr uint32_t PER_TILE = WF_GEN_TILE / RTX_WAVE;
+    if (S.gen && cl % PER_TILE == 0u && lane == 0) S.status[cl / PER_TILE] = 0u;
+    const uint32_t n = S.count[0];
+    const TraceIo io{gptr(S.node), gptr(S.delta), gptr(S.wide), gptr(S.tri), gptr(S.nrm), gptr(S.uv), gptr(S.ori4),
+                     gptr(S.dir4), gptr(S.flags), gptr(S.t), gptr(S.id), gptr(S.bary), gptr(S.n4), gptr(S.p4),
+                     gptr(S.uv2), gptr(S.list), S.list_count};
+#pragma unroll 1
+    for (uint32_t k = 0; k < 4u && cl * RTX_WAVE + 16u * k < n; ++k) {
+        const uint32_t rr = cl * RTX_WAVE + 16u * k + (lane >> 2);
+        wide_trace<GROUPS>(io, rr, rr < n, stk, coop);
+    }
+}
+
+template <int TB>
+__global__ __launch_bounds__(TB) void k_wf_trace_w(const WfSeg* __restrict__ segs, uint32_t nseg,
+                                                   uint32_t* __restrict__ queue, uint32_t coop, uint32_t grain) {
+    __shared__ uint2 s_stk[WIDE_STACK * (TB / 4)];
+    WaveChunks<WF_RAYS> wc;
+    wc.init(segs, nseg, RTX_WAVE);
+    ChunkSched sch;
+    sch.init(wc.total, queue, grain);
+    for (uint32_t c = 0; sch.next(c);) {
+        uint32_t c0 = 0;
+        const uint32_t sg = __builtin_amdgcn_readfirstlane(wc.find(c, c0));
+        wf_trace_chunk_w<TB / 4>(segs[sg], c - c0, WideStack<TB / 4>{s_stk + (threadIdx.x >> 2)}, coop,
+                                 threadIdx.x & (RTX_WAVE - 1));
+    }
+}
+
+template <int TB>
+__global__ __launch_bounds__(TB) void k_wf_trace_ord_w(const WfSeg* __restrict__ segs, uint32_t nseg,
+                                                       const uint32_t* __restrict__ ctr, uint32_t coop) {
+    __shared__ uint2 s_stk[WIDE_STACK * (TB / 4)];
+    const uint32_t total = ctr[WF_TOTAL];
+    const uint32_t c = blockIdx.x * (TB / RTX_WAVE) + threadIdx.x / RTX_WAVE;
+    if (c >= total) return;  // whole waves (no block barrier follows)
+    WaveChunks<WF_RAYS> wc;
+    wc.load(ctr + WF_TAB, nseg, total);
+    uint32_t c0 = 0;
+    const uint32_t sg = __builtin_amdgcn_readfirstlane(wc.find(c, c0));
+    wf_trace_chunk_w<TB / 4>(segs[sg], c - c0, WideStack<TB / 4>{s_stk + (threadIdx.x >> 2)}, coop,
+                             threadIdx.x & (RTX_WAVE - 1));
+}
+
 // One 64-pair chunk (chunk cl of segment S) of the shadow launch: the
 // (hit, light) pairs of k_shadow, light-major (a wave traces one light's
 // rays from neighbouring hits).  The whole wave calls it.
@@ -2112,6 +2672,60 @@ __global__ __launch_bounds__(TB) void k_wf_shadow(const WfSeg* __restrict__ segs
         const uint32_t sg = __builtin_amdgcn_readfirstlane(wc.find(c, c0));
         wf_shadow_chunk<VAR>(segs[sg], c - c0, stk, coop, lane, ordered != 0);
     }
+}
+
+// The same by the wide walk.
+template <bool ORDERED, int GROUPS>
+__device__ __forceinline__ void wf_shadow_chunk_w(const WfSeg& S, uint32_t cl, WideStack<GROUPS> stk, uint32_t coop,
+                                                  uint32_t lane) {
+    const uint64_t nh = S.list_count[0], items = nh * (uint64_t)S.lights->count;
+    uint32_t traced = 0;
+#pragma unroll 1
+    for (uint32_t k = 0; k < 4u && (uint64_t)cl * RTX_WAVE + 16u * k < items; ++k) {
+        const uint64_t it = (uint64_t)cl * RTX_WAVE + 16u * k + (lane >> 2);
+        const bool valid = it < items;
+        uint32_t rr = 0;
+        int l = 0;
+        if (valid) {
+            rr = gptr(S.list)[it % nh];
+            l = (int)(it / nh);
+        }
+        const bool t = wide_shadow<ORDERED, GROUPS>(gptr(S.node), gptr(S.delta), gptr(S.wide), gptr(S.tri),
+                                                    gptr(S.lights), gptr(S.p4), gptr(S.flags), rr, l, valid, stk, coop);
+        traced += (uint32_t)__builtin_popcountll(ballot(t && (lane & 3u) == 0u));
+    }
+    if (lane == 0 && traced) atomicAdd(&S.stats[1], (unsigned long long)traced);
+}
+
+template <bool ORDERED, int TB>
+__global__ __launch_bounds__(TB) void k_wf_shadow_w(const WfSeg* __restrict__ segs, uint32_t nseg,
+                                                    uint32_t* __restrict__ queue, uint32_t coop, uint32_t grain) {
+    __shared__ uint2 s_stk[WIDE_STACK * (TB / 4)];
+    WaveChunks<WF_PAIRS> wc;
+    wc.init(segs, nseg, RTX_WAVE);
+    ChunkSched sch;
+    sch.init(wc.total, queue, grain);
+    for (uint32_t c = 0; sch.next(c);) {
+        uint32_t c0 = 0;
+        const uint32_t sg = __builtin_amdgcn_readfirstlane(wc.find(c, c0));
+        wf_shadow_chunk_w<ORDERED, TB / 4>(segs[sg], c - c0, WideStack<TB / 4>{s_stk + (threadIdx.x >> 2)}, coop,
+                                           threadIdx.x & (RTX_WAVE - 1));
+    }
+}
+
+template <bool ORDERED, int TB>
+__global__ __launch_bounds__(TB) void k_wf_shadow_ord_w(const WfSeg* __restrict__ segs, uint32_t nseg,
+                                                        const uint32_t* __restrict__ ctr, uint32_t coop) {
+    __shared__ uint2 s_stk[WIDE_STACK * (TB / 4)];
+    const uint32_t total = ctr[WF_STOTAL];
+    const uint32_t c = blockIdx.x * (TB / RTX_WAVE) + threadIdx.x / RTX_WAVE;
+    if (c >= total) return;  // whole waves (no block barrier follows)
+    WaveChunks<WF_PAIRS> wc;
+    wc.load(ctr + WF_STAB, nseg, total);
+    uint32_t c0 = 0;
+    const uint32_t sg = __builtin_amdgcn_readfirstlane(wc.find(c, c0));
+    wf_shadow_chunk_w<ORDERED, TB / 4>(segs[sg], c - c0, WideStack<TB / 4>{s_stk + (threadIdx.x >> 2)}, coop,
+                                       threadIdx.x & (RTX_WAVE - 1));
 }
 
 // Between the trace and the in-order shadow launch: the shadow chunk table
@@ -2193,6 +2807,26 @@ static uint32_t resident_grid(int block, int cus, int share) {
 
 void rtx_wf_trace(const WfSeg* segs, uint32_t nseg, uint32_t* ctr, int var, int tb, int sr, uint32_t coop,
                   uint32_t grain, int sched, uint64_t max_chunks, int cus, int share, hipStream_t st) {
+    if (var == WF_WIDE) {
+        const uint64_t g = (max_chunks + tb / RTX_WAVE - 1) / (tb / RTX_WAVE);
+#define RTX_WF_TRACE_W(B)                                                                                           \
+    do {                                                                                                            \
+        if (sched == 0)                                                                                             \
+            hipLaunchKernelGGL((k_wf_trace_ord_w<B>), dim3((uint32_t)(g ? g : 1)), dim3(B), 0, st, segs, nseg, ctr, \
+                               coop);                                                                               \
+        else                                                                                                        \
+            hipLaunchKernelGGL((k_wf_trace_w<B>), dim3(resident_grid<k_wf_trace_w<B>>(B, cus, share)), dim3(B), 0, \
+                               st, segs, nseg, ctr + WF_Q_TRACE, coop, grain);                                      \
+    } while (0)
+        if (tb == 64)
+            RTX_WF_TRACE_W(64);
+        else if (tb == 256)
+            RTX_WF_TRACE_W(256);
+        else
+            RTX_WF_TRACE_W(128);
+#undef RTX_WF_TRACE_W
+        return;
+    }
     if (sched == 0) {
         const uint64_t g = (max_chunks + tb / RTX_WAVE - 1) / (tb / RTX_WAVE);
 #define RTX_WF_TRACE_ORD(V, B, S)                                                                                \
@@ -2212,8 +2846,34 @@ void rtx_wf_trace(const WfSeg* segs, uint32_t nseg, uint32_t* ctr, int var, int 
 void rtx_wf_shadow(const WfSeg* segs, uint32_t nseg, uint32_t* ctr, int var, int tb, int sr, uint32_t coop,
                    uint32_t grain, int sched, uint64_t max_chunks, int cus, int share, bool ordered,
                    hipStream_t st) {
+    if (sched == 0) hipLaunchKernelGGL(k_wf_plan_shadow, dim3(1), dim3(RTX_WF_MAX_SEGS), 0, st, segs, nseg, ctr);
+    if (var == WF_WIDE) {
+        const uint64_t g = (max_chunks + tb / RTX_WAVE - 1) / (tb / RTX_WAVE);
+#define RTX_WF_SHADOW_W(O, B)                                                                                       \
+    do {                                                                                                            \
+        if (sched == 0)                                                                                             \
+            hipLaunchKernelGGL((k_wf_shadow_ord_w<O, B>), dim3((uint32_t)(g ? g : 1)), dim3(B), 0, st, segs, nseg,  \
+                               ctr, coop);                                                                          \
+        else                                                                                                        \
+            hipLaunchKernelGGL((k_wf_shadow_w<O, B>), dim3(resident_grid<k_wf_shadow_w<O, B>>(B, cus, share)),     \
+                               dim3(B), 0, st, segs, nseg, ctr + WF_Q_SHADOW, coop, grain);                         \
+    } while (0)
+#define RTX_WF_SHADOW_WB(B)                                       \
+    do {                                                          \
+        if (ordered) RTX_WF_SHADOW_W(true, B);                    \
+        else RTX_WF_SHADOW_W(false, B);                           \
+    } while (0)
+        if (tb == 64)
+            RTX_WF_SHADOW_WB(64);
+        else if (tb == 256)
+            RTX_WF_SHADOW_WB(256);
+        else
+            RTX_WF_SHADOW_WB(128);
+#undef RTX_WF_SHADOW_WB
+#undef RTX_WF_SHADOW_W
+        return;
+    }
     if (sched == 0) {
-        hipLaunchKernelGGL(k_wf_plan_shadow, dim3(1), dim3(RTX_WF_MAX_SEGS), 0, st, segs, nseg, ctr);
         const uint64_t g = (max_chunks + tb / RTX_WAVE - 1) / (tb / RTX_WAVE);
 #define RTX_WF_SHADOW_ORD(V, B, S)                                                                                \
     hipLaunchKernelGGL((k_wf_shadow_ord<V, B, S>), dim3((uint32_t)(g ? g : 1)), dim3(B), 0, st, segs, nseg, ctr, \
@@ -2406,6 +3066,16 @@ static int traversal_variant(const rtx_scene* s, const SceneView& sv) {
     return (var == 2 && depth >= STACK) ? 1 : var;
 }
 
+// Whether the tree has wide records.
+static bool wide_walk(const rtx_scene* s, const SceneView& sv) { return sv.wide && s->T <= WIDE_MAX_TRIS; }
+
+// Four lanes per item, up to 64 groups per CU (then grid-stride).
+static uint32_t wide_grid(rtx_ctx* c, uint64_t count, uint64_t cap, int TB) {
+    const uint64_t n = count == RTX_DEVICE_COUNT ? cap : count;
+    const uint64_t g = (4 * n + TB - 1) / TB, gmax = (uint64_t)c->cus * 64;
+    return (uint32_t)(g > gmax ? gmax : (g ? g : 1));
+}
+
 // Iteration bound of the stackless walk: a tree of N <= 2T - 1 nodes allows
 // at most 3 visits per node.
 static uint32_t stackless_bound(const rtx_scene* s) { return 6u * s->T + 8u; }
@@ -2423,6 +3093,27 @@ int32_t rtx_trace(rtx_scene* s, rtx_rays* rays, rtx_hits* hits, uint64_t count, 
     ProfScope ps(s->ctx, st, "trace");
     const SceneView sv = scene_view(s);
     const int var = traversal_variant(s, sv), tb = (int)s->ctx->tune.trace_block;
+    if (var == 1 && wide_walk(s, sv)) {
+        const TraceIo io{sv.node, sv.delta, sv.wide, sv.tri, sv.nrm, s->uv.as<float2>(), rays->ori4.as<float4>(),
+                         rays->dir4.as<float4>(), hits->flags.as<uint32_t>(), hits->t.as<float>(),
+                         hits->id.as<int32_t>(), hits->bary.as<float2>(), hits->n4.as<float4>(),
+                         hits->p4.as<float4>(), hits->uv2.as<float2>(), hits->list.as<uint32_t>(),
+                         hits->list_count.as<uint32_t>()};
+#define RTX_TRACE_W(B)                                                                                          \
+    hipLaunchKernelGGL((k_trace_w<B>), dim3(wide_grid(s->ctx, count, rays->cap, B)), dim3(B), 0, st, io,       \
+                       rays->count.as<uint32_t>(), count, rtx_wide_coop(s->ctx))
+        if (tb == 64)
+            RTX_TRACE_W(64);
+        else if (tb == 256)
+            RTX_TRACE_W(256);
+        else
+            RTX_TRACE_W(128);
+#undef RTX_TRACE_W
+        RTX_CHECK_HIP(hipGetLastError());
+        hits->list_valid = true;
+        hits->list_for = count;
+        return RTX_OK;
+    }
     if (var == 3) {
 #define RTX_TRACE_P(B)                                                                                              \
     hipLaunchKernelGGL((k_trace_p<B>), dim3(persist_grid(s->ctx, count, rays->cap, B)), dim3(B), 0, st,            \
@@ -2497,6 +3188,25 @@ int32_t rtx_trace_shadow_multi(rtx_scene* s, rtx_rays* const* rays, rtx_hits* co
     const SceneView sv = scene_view(s);
     uint64_t n = max_items * (uint64_t)nl;
     const int var = traversal_variant(s, sv), tb = (int)s->ctx->tune.trace_block;
+    // the reference's child order only where a ray's stack can reach MAX_LEVELS
+    // (the stackless walk has none)
+    const int depth = s->ext ? s->ext->depth : s->depth;
+    const uint32_t ordered = (s->ctx->tune.shadow_order != 0 || (depth >= STACK && var != 4)) ? 1u : 0u;
+    if (var == 1 && wide_walk(s, sv)) {
+#define RTX_SHADOW_W(B)                                                                                        \
+    hipLaunchKernelGGL((ordered ? k_shadow_w<true, B> : k_shadow_w<false, B>), dim3(wide_grid(s->ctx, n, n, B)), \
+                       dim3(B), 0, st, sv.node, sv.delta, sv.wide, sv.tri, s->lights.as<rtx_lights>(), segs, (unsigned long long*)dev_shadow_count,      \
+                       rtx_wide_coop(s->ctx))
+        if (tb == 64)
+            RTX_SHADOW_W(64);
+        else if (tb == 256)
+            RTX_SHADOW_W(256);
+        else
+            RTX_SHADOW_W(128);
+#undef RTX_SHADOW_W
+        RTX_CHECK_HIP(hipGetLastError());
+        return RTX_OK;
+    }
     if (var == 3) {
         // queue counter: word 2 of the first segment's hit-list counters
         uint32_t* queue = hits[0]->list_count.as<uint32_t>() + 2;
@@ -2521,10 +3231,6 @@ int32_t rtx_trace_shadow_multi(rtx_scene* s, rtx_rays* const* rays, rtx_hits* co
                        sv.delta, sv.tri, s->lights.as<rtx_lights>(), segs,                                     \
                        (unsigned long long*)dev_shadow_count, (uint32_t)s->ctx->tune.xcds, \
                        coop_threshold(s->ctx), sv.parent, stackless_bound(s), ordered)
-    // the reference's child order only where a ray's stack can reach MAX_LEVELS
-    // (the stackless walk has none)
-    const int depth = s->ext ? s->ext->depth : s->depth;
-    const uint32_t ordered = (s->ctx->tune.shadow_order != 0 || (depth >= STACK && var != 4)) ? 1u : 0u;
     RTX_DISPATCH_STACK_NS(RTX_SHADOW_LAUNCH, var, tb, (int)s->ctx->tune.stack_lds);
 #undef RTX_SHADOW_LAUNCH
     RTX_CHECK_HIP(hipGetLastError());
@@ -2555,7 +3261,7 @@ int32_t rtx_bvh_create(rtx_ctx* ctx, rtx_bvh** out) {
 int32_t rtx_bvh_destroy(rtx_bvh* b) {
     if (!b) return RTX_OK;
     rtx_scene::RenderCopy& c = b->copy;
-    for (DevBuf* d : {&c.node, &c.delta, &c.tri, &c.nrm, &c.matmap}) d->release();
+    for (DevBuf* d : {&c.node, &c.delta, &c.tri, &c.nrm, &c.matmap, &c.wide}) d->release();
     delete b;
     return RTX_OK;
 }

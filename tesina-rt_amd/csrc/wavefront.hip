@@ -31,6 +31,7 @@
 
 #include "arena.hpp"
 #include "rtx_impl.hpp"
+#include "wide.hpp"
 
 namespace {
 
@@ -215,6 +216,7 @@ static WfSeg make_seg(rtx_wavefront* wf, const WfFrame& fr, uint32_t fin) {
     WfSeg g{};
     g.node = sv.node;
     g.delta = sv.delta;
+    g.wide = s->T <= WIDE_MAX_TRIS ? sv.wide : nullptr;
     g.tri = sv.tri;
     g.nrm = sv.nrm;
     g.uv = s->uv.as<float2>();
@@ -282,7 +284,7 @@ int32_t rtx_wavefront_step_impl(rtx_wavefront* wf, hipStream_t st, int32_t* pend
     }
     WfSeg* T = wf->htab + (size_t)k * RTX_WF_MAX_SEGS;
     uint64_t px_new = 0, px_done = 0, max_chunks = 0, max_pair_chunks = 0;
-    bool gen = false, deep = false;
+    bool gen = false, deep = false, wide = true;
     std::vector<int> fin;
     const uint32_t n = (uint32_t)act.size();
     for (uint32_t i = 0; i < n; ++i) {
@@ -300,6 +302,7 @@ int32_t rtx_wavefront_step_impl(rtx_wavefront* wf, hipStream_t st, int32_t* pend
             gen = true;
         }
         if (fr.scene->depth >= 32) deep = true;
+        if (!T[i].wide) wide = false;
     }
     rtx_ctx* c = wf->ctx;
     WfSeg* D = wf->dtab.as<WfSeg>() + (size_t)k * RTX_WF_MAX_SEGS;
@@ -310,8 +313,10 @@ int32_t rtx_wavefront_step_impl(rtx_wavefront* wf, hipStream_t st, int32_t* pend
     // persistent and stackless forms have no segmented kernels
     int var = (int)c->tune.trace_variant;
     if (var > 2 || (var == 2 && deep)) var = 1;
+    if (var == 1 && wide) var = WF_WIDE;
     const int tb = (int)c->tune.trace_block;
-    const uint32_t coop = c->tune.coop_leaf > 0 ? (uint32_t)c->tune.coop_leaf : 0xffffffffu;
+    uint32_t coop = c->tune.coop_leaf > 0 ? (uint32_t)c->tune.coop_leaf : 0xffffffffu;
+    if (var == WF_WIDE) coop = rtx_wide_coop(c);
     const int share = c->tune.wf_share > 0 ? (int)c->tune.wf_share : wf->auto_share;
     RTX_CHECK_HIP(hipMemcpyAsync(D, T, sizeof(WfSeg) * n, hipMemcpyHostToDevice, st));
     {
