@@ -1,0 +1,129 @@
+"""The tile edges of the tree phase and the edges of the wide walk's encodings,
+against the oracle bit for bit.
+
+Tree phase: tiles of 1024 sorted positions; nodes and runs of equal codes that
+cross tile edges, whole trees of one leaf over several tiles, and the triangle
+count from which the ranks take wider tiles.
+
+Wide walk: rays with zero and huge direction components whose origins lie on
+box planes (an infinite reciprocal is walked node by node, a skipped axis is a
+NaN), infinite and tiny tMax, leaves around 15 triangles (the counts a stack
+entry holds) and around 32 (from which the whole wave tests a leaf)."""
+import numpy as np
+import pytest
+
+import oracle as O
+from test_gpu_parity import check_build, load_scene, random_scene
+
+pytestmark = pytest.mark.gpu
+
+
+def _scene(kind, T, seed):
+    pos, idx, nrm, uv, mm = random_scene(seed, T)
+    if kind == "runs":  # a few triangles, each in a run of up to a thousand equal codes
+        rng = np.random.default_rng(seed)
+        idx = idx[np.sort(rng.integers(0, max(1, T // 500), T))]
+    elif kind == "same":  # one code: a single leaf
+        idx = np.repeat(idx[:1], T, axis=0)
+    elif kind == "cluster":  # most triangles in one corner: deep and shallow subtrees side by side
+        pos[: len(pos) * 3 // 4] *= np.float32(0.001)
+    return pos, idx, nrm, uv, mm
+
+
+@pytest.mark.parametrize("kind,T,depth,min_leaf", [
+    ("random", 1023, 30, 1), ("random", 1024, 30, 1), ("random", 1025, 30, 1), ("random", 2049, 32, 3),
+    ("random", 5000, 7, 1), ("random", 5000, 1, 1), ("random", 6000, 30, 256), ("runs", 4096, 30, 1),
+    ("runs", 5001, 32, 2), ("same", 1024, 30, 1), ("same", 1025, 30, 1), ("same", 3500, 30, 1),
+    ("cluster", 9000, 30, 1), ("random", (1 << 19) - 1, 30, 1), ("random", (1 << 19) + 5, 30, 1)])
+def test_tree_tiles(ctx, kind, T, depth, min_leaf):
+    pos, idx, nrm, uv, mm = _scene(kind, T, 7 + T)
+    s = load_scene(ctx, pos, idx, nrm, uv, mm)
+    s.build(depth, min_leaf)
+    b = O.Build(pos, idx, mm, depth, min_leaf)
+    check_build(s, b, T)
+    if T < 10000:
+        pos2 = (pos * np.float32(0.75) + np.float32(0.5)).astype(np.float32)
+        s.update_positions(pos2)
+        s.refit()
+        b.refit(pos2)
+        g = s.nodes()
+        assert np.array_equal(g["lo"][:, :3], b.nodes["lo"][:, :3])
+        assert np.array_equal(g["hi"][:, :3], b.nodes["hi"][:, :3])
+        s.build(depth, min_leaf)  # from the permuted buffers
+        b2 = O.Build(pos2, b.idx.reshape(-1, 3), b.matmap, depth, min_leaf)
+        g = s.nodes()
+        assert np.array_equal(g["a"], b2.nodes["a"]) and np.array_equal(g["lo"][:, :3], b2.nodes["lo"][:, :3])
+    s.destroy()
+
+
+def _odd_rays(rng, pos, n):
+    """Axis-parallel and huge directions from vertex coordinates, with all kinds of tMin and tMax."""
+    o = pos[rng.integers(0, len(pos), n)].astype(np.float32)
+    o += (rng.integers(-1, 2, (n, 3)) * rng.integers(0, 30, (n, 1))).astype(np.float32)
+    d = rng.normal(size=(n, 3)).astype(np.float32)
+    d[rng.random((n, 3)) < 0.4] = 0.0
+    d[rng.random((n, 3)) < 0.05] = -0.0
+    d[(d == 0).all(1)] = (0, 0, 1)
+    d *= rng.choice(np.array([1.0, 3e6, 1e-5], np.float32), (n, 1), p=[0.8, 0.1, 0.1])
+    d[rng.random((n, 3)) < 0.02] = 1e-41  # 1/d overflows
+    ori4, dir4 = np.zeros((n, 4), np.float32), np.zeros((n, 4), np.float32)
+    ori4[:, :3], dir4[:, :3] = o, d
+    ori4[:, 3] = rng.choice(np.array([0.0, 1e-4, 1.0], np.float32), n)
+    dir4[:, 3] = rng.choice(np.array([1e36, np.inf, 25.0, 1e-3], np.float32), n)
+    return ori4, dir4
+
+
+def _compare(ctx, s, b, nrm, uv, ori4, dir4, lights):
+    import rtx
+    n = len(ori4)
+    r, h = rtx.Rays(ctx, n), rtx.Hits(ctx, n)
+    r.write(ori4, dir4)
+    rtx.trace(s, r, h, n)
+    rtx.trace_shadow(s, r, h, n)
+    g = h.read(n)
+    o = O.trace(b, nrm, uv, ori4, dir4)
+    o["flags"] = O.trace_shadow(b, O.lights_from(lights), o["flags"], o["p4"])
+    for k in ("id", "t", "bary", "flags", "n4", "p4"):
+        assert np.array_equal(g[k], o[k], equal_nan=g[k].dtype.kind == "f"), k
+    r.destroy()
+    h.destroy()
+    return o
+
+
+def _lights():
+    import rtx
+    return rtx.make_lights((0.1, 0.1, 0.1), [dict(type=rtx.LIGHT_POINT, pos=(2.0, 24.0, -4.0)),
+                                             dict(type=rtx.LIGHT_DIR, dir=(0.0, -1.0, 0.0))])
+
+
+@pytest.mark.parametrize("T,depth,flat,n", [(3000, 30, None, 4097), (3000, 30, 1, 4096), (3000, 32, 0, 1023),
+                                            (40000, 30, None, 4096), (2, 30, None, 65)])
+def test_wide_walk_odd_rays(ctx, T, depth, flat, n):
+    pos, idx, nrm, uv, mm = random_scene(31 + T, T, flat_axis=flat)
+    pos = np.round(pos).astype(np.float32) + np.float32(0.0)  # box planes that rays start on
+    lights = _lights()
+    s = load_scene(ctx, pos, idx, nrm, uv, mm, lights=lights)
+    s.build(depth, 1)
+    b = O.Build(pos, idx, mm, depth, 1)
+    ori4, dir4 = _odd_rays(np.random.default_rng(T + n), pos, n)
+    _compare(ctx, s, b, nrm, uv, ori4, dir4, lights)
+    s.destroy()
+
+
+@pytest.mark.parametrize("copies", [3, 4, 5, 14, 15, 16, 17, 31, 32, 33, 70])
+def test_wide_walk_leaf_sizes(ctx, copies):
+    rng = np.random.default_rng(copies)
+    pos, idx, nrm, uv, mm = random_scene(copies, 400)
+    idx = np.repeat(idx, copies, axis=0)[rng.permutation(400 * copies)]
+    mm = rng.integers(0, 3, len(idx)).astype(np.int32)
+    lights = _lights()
+    s = load_scene(ctx, pos, idx, nrm, uv, mm, lights=lights)
+    s.build()
+    b = O.Build(pos, idx, mm, 30, 1)
+    o = rng.uniform(-12, 12, (2048, 3))
+    d = rng.normal(size=(2048, 3))
+    ori4, dir4 = np.zeros((2048, 4), np.float32), np.full((2048, 4), 1e36, np.float32)
+    ori4[:, :3], dir4[:, :3] = o, d / np.linalg.norm(d, axis=1, keepdims=True)
+    res = _compare(ctx, s, b, nrm, uv, ori4, dir4, lights)
+    assert (res["id"] >= 0).sum() > 500
+    s.destroy()
