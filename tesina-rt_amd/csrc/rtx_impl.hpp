@@ -473,7 +473,7 @@ enum {
 void rtx_wf_init(const WfSeg* segs, uint32_t nseg, uint32_t* ctr, hipStream_t st);
 void rtx_wf_raygen(const WfSeg* segs, uint32_t nseg, uint64_t pixels, int cus, hipStream_t st);
 // var: a traversal form (trace_variant 0 to 2), or WF_WIDE: the wide walk.
-constexpr int WF_WIDE = -1;
+constexpr int WF_WIDE = 5;
 // sched 1: persistent waves over per-XCD queues; 0: one chunk per wave in
 // launch order over a grid of `max_chunks` (an upper bound of the chunks).
 void rtx_wf_trace(const WfSeg* segs, uint32_t nseg, uint32_t* ctr, int var, int tb, int sr, uint32_t coop,

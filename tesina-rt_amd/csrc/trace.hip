@@ -663,8 +663,15 @@ __device__ bool traverse_any_ns(const float4* __restrict__ node, const float4* _
 // ------------------------------------------------------- wide walk -------
 // Four lanes per ray over the wide records (wide.hpp): each lane tests one
 // slot, so a step costs one 128-byte line and one box test of latency for two
-// levels of the tree, and a wave holds 16 rays instead of waiting for the
-// slowest of 64.
+// levels of the tree.  Two ways to hand rays to the wave's 16 groups:
+//   WIDE_GROUP: 16 rays per wave, every lane of a group holding the group's
+//     ray (scene launches: short walks of neighbouring rays stay in step);
+//   WIDE: a ray per lane.  The rays that meet the root's box wait in LDS, and a
+//     group whose ray ends goes on with the next one (wavefront launches, whose
+//     chunks are 64 rays).
+// Measured, WIDE_GROUP against WIDE: 720p frame over a 200k SAH tree 463
+// against 549 us, 131k scattered rays 196 against 214; batch of 12 frames 8.1
+// against 6.5 ms.
 //
 // Equality with the node-by-node walk.  The reference visits leaves in a
 // fixed depth-first order of the ray (near child first by
@@ -678,10 +685,14 @@ __device__ bool traverse_any_ns(const float4* __restrict__ node, const float4* _
 // the odd levels in between are not tested: float subtraction, multiplication,
 // min and max are monotone, so a box inside another has the later entry and
 // the earlier exit and passes only where the outer box passes.
-// Two kinds of rays are walked node by node instead (exact_*): those with an
-// axis whose 1/dir is infinite (0 * inf is NaN, which min and max drop, and
-// the argument fails), and those that pass a WIDE_DEEP node, below which the
-// reference's stack count can reach MAX_LEVELS.
+// That argument fails on an axis whose 1/dir is infinite (0 * inf is NaN,
+// which min and max drop): for such rays the boxes of the odd levels, the
+// unions of two slots, are tested too.  They then pass at the push, and an
+// entry distance below infinity comes from the other axes alone, where the
+// inner box's is the later one; with an infinite tMax it can be infinite, and
+// those rays are walked node by node (exact_walk), as are rays that pass a
+// WIDE_DEEP node, below which the reference's stack count can reach
+// MAX_LEVELS, and rays that would overflow the group's stack.
 
 // Value of lane (lane ^ 1), (lane ^ 2) of the group of four, or of its lane 0.
 constexpr int QX1 = 0xB1, QX2 = 0x4E, QFIRST = 0x00;
@@ -698,40 +709,51 @@ __device__ __forceinline__ v3 quad_v(v3 a) {
     return mk3(quad_f<CTRL>(a.x), quad_f<CTRL>(a.y), quad_f<CTRL>(a.z));
 }
 
-// Ray constants of the wide walk: a skipped axis (RayC::ax etc. false) has a
-// NaN reciprocal, which min and max drop like the skip.  The origin,
-// direction and tMin are those of the ray.
+// A ray of the wide walk: a skipped axis (RayC::ax etc. false) has a NaN
+// reciprocal, which min and max drop like the skip.
 struct WideRay {
     v3 o, d, inv;
     float tmin;
 };
-__device__ __forceinline__ WideRay wide_ray(const RayC& r) {
+__device__ __forceinline__ v3 wide_inv(const RayC& r) {
     const float skip = __builtin_nanf("");
-    return WideRay{r.o, r.d, mk3(r.ax ? r.inv.x : skip, r.ay ? r.inv.y : skip, r.az ? r.inv.z : skip), r.tmin};
+    return mk3(r.ax ? r.inv.x : skip, r.ay ? r.inv.y : skip, r.az ? r.inv.z : skip);
 }
-__device__ __forceinline__ bool wide_odd(const RayC& r) { return isinf(r.inv.x) || isinf(r.inv.y) || isinf(r.inv.z); }
+__device__ __forceinline__ bool wide_odd(v3 inv) { return isinf(inv.x) || isinf(inv.y) || isinf(inv.z); }
 
 // slab() with the entry distance.
-__device__ __forceinline__ bool wide_slab(float4 lo4, float4 hi4, const WideRay& r, float tmax, float& t0) {
-    const v3 tl = (xyz(lo4) - r.o) * r.inv, th = (xyz(hi4) - r.o) * r.inv;
+__device__ __forceinline__ bool wide_slab(v3 lo, v3 hi, const WideRay& r, float tmax, float& t0) {
+    const v3 tl = (lo - r.o) * r.inv, th = (hi - r.o) * r.inv;
     const v3 tM = vmax(tl, th), tm = vmin(tl, th);
     t0 = fmaxf(fmaxf(fmaxf(r.tmin, tm.x), tm.y), tm.z);
     const float t1 = fminf(fminf(fminf(tmax, tM.x), tM.y), tM.z);
     return t0 <= t1;
 }
 
-// Stack of a group in LDS: entry lv of the block's groups side by side.
-template <int GROUPS>
-struct WideStack {
-    uint2* e;
-    __device__ __forceinline__ void put(int lv, uint32_t ref, float t0) {
-        e[lv * GROUPS] = make_uint2(ref, __float_as_uint(t0));
+// LDS of a wave: the rays {o, tMin}{d, tMax}{1/d, t0 of the root} (not for
+// WIDE_GROUP), their results, and the groups' stacks ([entry][group], an entry
+// is a reference and, for closest hits, its t0).
+constexpr int WIDE_GROUPS = RTX_WAVE / 4;
+template <bool ANY, bool GROUP>
+struct WideLds {
+    static constexpr int N = GROUP ? WIDE_GROUPS : RTX_WAVE;
+    static constexpr int RAY = GROUP ? 0 : 3 * 4 * N, RES = ANY ? N : 4 * N;
+    static constexpr int WORDS = RAY + RES + WIDE_STACK * WIDE_GROUPS * (ANY ? 1 : 2);
+    uint32_t* m;
+    __device__ __forceinline__ WideLds(uint32_t* lds, uint32_t tid, uint32_t*) : m(lds + (tid / RTX_WAVE) * WORDS) {}
+    __device__ __forceinline__ float4* ray(int part) const { return reinterpret_cast<float4*>(m) + part * N; }
+    __device__ __forceinline__ float4* res() const { return reinterpret_cast<float4*>(m + RAY); }
+    __device__ __forceinline__ uint32_t* hit() const { return m + RAY; }
+    __device__ __forceinline__ uint2* stack2() const {
+        return reinterpret_cast<uint2*>(m + RAY + RES) + ((threadIdx.x & (RTX_WAVE - 1)) >> 2);
     }
-    __device__ __forceinline__ uint2 get(int lv) const { return e[lv * GROUPS]; }
+    __device__ __forceinline__ uint32_t* stack1() const {
+        return m + RAY + RES + ((threadIdx.x & (RTX_WAVE - 1)) >> 2);
+    }
 };
 
-// Orders the pushes of a group's lanes before the pops of its other lanes (one
-// wave: no instruction, only the compiler is held).
+// Orders LDS accesses of different lanes (one wave: no instruction, only the
+// compiler is held).
 __device__ __forceinline__ void wide_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -746,18 +768,28 @@ struct WideStep {
     int after, total;
 };
 template <bool ORDERED>
-__device__ __forceinline__ WideStep wide_step(float4 f0, float4 f1, const WideRay& r, float tmax, uint32_t q) {
+__device__ __forceinline__ WideStep wide_step(float4 f0, float4 f1, const WideRay& r, bool any_odd, bool odd,
+                                              float tmax, uint32_t q) {
     WideStep s;
-    s.pass = wide_slab(f0, f1, r, tmax, s.t0) && __float_as_uint(f0.w) != WIDE_EMPTY;
+    const v3 lo = xyz(f0), hi = xyz(f1);
+    s.pass = wide_slab(lo, hi, r, tmax, s.t0) && __float_as_uint(f0.w) != WIDE_EMPTY;
     bool first = (q & 1u) == 0u, first_pair = (q & 2u) == 0u;
     if (ORDERED) {
         // dot(d, right.lo - left.lo) on the right lane, its exact negation on the left
-        const v3 lo = xyz(f0), sib = quad_v<QX1>(lo);
+        const v3 sib = quad_v<QX1>(lo);
         const float din = dot(r.d, lo - sib);
         first = first ? din < 0.f : !(din > 0.f);
         const v3 plo = vmin(lo, sib);
         const float dout = dot(r.d, plo - quad_v<QX2>(plo));
         first_pair = first_pair ? dout < 0.f : !(dout > 0.f);
+    }
+    if (any_odd) {  // the box of the level between
+        // an empty slot lends its sibling's box: +inf in lo is dropped by the min
+        const v3 sib = quad_v<QX1>(hi);
+        const bool empty = __float_as_uint(f0.w) == WIDE_EMPTY, sib_empty = quad_i<QX1>(empty ? 1 : 0) != 0;
+        const v3 phi = empty ? sib : (sib_empty ? hi : vmax(hi, sib));
+        float t;
+        if (!wide_slab(vmin(lo, quad_v<QX1>(lo)), phi, r, tmax, t) && odd) s.pass = false;
     }
     const int me = s.pass ? 1 : 0;
     const int sib = quad_i<QX1>(me), pair = me + sib, other = quad_i<QX2>(pair);
@@ -778,200 +810,14 @@ __device__ __forceinline__ void wide_leaf(const float4* __restrict__ node, uint3
     }
 }
 
-// The root's entry, when its box passes.
-__device__ __forceinline__ bool wide_root(const float4* __restrict__ node, const WideRay& r, float tmax, uint32_t& ref,
-                                          float& t0) {
-    const float4 f0 = node[0], f1 = node[1];
-    ref = wide_ref(0u, __float_as_uint(f0.w), __float_as_uint(f1.w));
-    return wide_slab(f0, f1, r, tmax, t0);
-}
-
-// Closest hit of the group's ray; called by the whole wave, `start` the same
-// on the four lanes.  best is kept equal on them.  Leaves are tested four
-// triangles at a time, one per lane, leaves of at least `coop` triangles by
-// the whole wave.  True: the ray has to be walked by exact_closest instead.
-template <int GROUPS>
-__device__ __forceinline__ bool wide_closest(const float4* __restrict__ node, const float4* __restrict__ wide,
-                                             const float4* __restrict__ tri, const WideRay& r, Closest& best,
-                                             WideStack<GROUPS> stk, uint32_t coop, bool start) {
-    const uint32_t q = lane_id() & 3u;
-    int level = 0;
-    bool redo = false;
-    if (start) {
-        uint32_t ref;
-        float t0;
-        if (wide_root(node, r, best.t, ref, t0)) {
-            stk.put(0, ref, t0);
-            level = 1;
-        }
-    }
-    while (ballot(level > 0)) {
-        wide_sync();
-        uint32_t la = 0, lcnt = 0;
-        if (level > 0) {
-            const uint2 e = stk.get(--level);
-            if (__uint_as_float(e.y) <= best.t) {
-                // the slot or the group's first four triangles: one round trip
-                // whichever a group needs
-                const bool leaf = (e.x & WIDE_LEAF) != 0u;
-                uint32_t first = 0, cnt = 0;
-                const char* p = reinterpret_cast<const char*>(wide) + ((e.x << 7) | (q << 5));
-                if (leaf) {
-                    wide_leaf(node, e.x, first, cnt);
-                    p = reinterpret_cast<const char*>(tri) + 48 * (size_t)(first + (q < cnt ? q : 0u));
-                }
-                const float4* p4 = reinterpret_cast<const float4*>(p);
-                float4 f0 = p4[0], f1 = p4[1], f2 = make_float4(0.f, 0.f, 0.f, 0.f);
-                if (leaf) f2 = p4[2];
-                if (!leaf) {
-                    if (e.x & WIDE_DEEP) {
-                        redo = true;
-                        level = 0;
-                    } else {
-                        const WideStep s = wide_step<true>(f0, f1, r, best.t, q);
-                        if (s.pass) stk.put(level + s.after, __float_as_uint(f0.w), s.t0);
-                        level += s.total;
-                    }
-                } else if (cnt >= coop) {
-                    la = first;
-                    lcnt = cnt;
-                } else {
-                    for (uint32_t b = 0;;) {
-                        const uint32_t i = b + q;
-                        float tt, u, v;
-                        const bool h =
-                            tri_hit_v(f0, f1, f2, r.o, r.d, &tt, &u, &v) && i < cnt && tt <= best.t && tt >= r.tmin;
-                        if (ballot(h)) {
-                            // the smallest t and, among equal ones, the latest triangle: what the
-                            // in-order loop with its `t <= best` update keeps
-                            int id = h ? (int)(first + i) : -1;
-                            tt = h ? tt : INFINITY;
-#pragma unroll
-                            for (int x = 0; x < 2; ++x) {
-                                const float ot = x ? quad_f<QX2>(tt) : quad_f<QX1>(tt);
-                                const float ou = x ? quad_f<QX2>(u) : quad_f<QX1>(u);
-                                const float ov = x ? quad_f<QX2>(v) : quad_f<QX1>(v);
-                                const int oi = x ? quad_i<QX2>(id) : quad_i<QX1>(id);
-                                const bool take = ot < tt || (ot == tt && oi > id);
-                                tt = take ? ot : tt;
-                                u = take ? ou : u;
-                                v = take ? ov : v;
-                                id = take ? oi : id;
-                            }
-                            if (id >= 0) best = Closest{tt, u, v, id};
-                        }
-                        b += 4;
-                        if (b >= cnt) break;
-                        const float4* t4 = tri + 3 * (size_t)(first + (b + q < cnt ? b + q : 0u));
-                        f0 = t4[0];
-                        f1 = t4[1];
-                        f2 = t4[2];
-                    }
-                }
-            }
-        }
-        if (ballot(lcnt != 0u)) {
-            RayC rc;
-            rc.o = r.o;
-            rc.d = r.d;
-            rc.tmin = r.tmin;
-            coop_closest(tri, la, q == 0u ? lcnt : 0u, rc, best, ~0ull);
-            best.t = quad_f<QFIRST>(best.t);
-            best.u = quad_f<QFIRST>(best.u);
-            best.v = quad_f<QFIRST>(best.v);
-            best.id = quad_i<QFIRST>(best.id);
-        }
-    }
-    return redo;
-}
-
-// Any hit with tMin < t < tMax.  ORDERED where the order can matter (trees of
-// 32 levels); `redo` as above.
-template <bool ORDERED, int GROUPS>
-__device__ __forceinline__ bool wide_any(const float4* __restrict__ node, const float4* __restrict__ wide,
-                                         const float4* __restrict__ tri, const WideRay& r, float tmax,
-                                         WideStack<GROUPS> stk, uint32_t coop, bool start, bool& redo) {
-    const uint32_t q = lane_id() & 3u;
-    int level = 0;
-    bool found = false;
-    if (start) {
-        uint32_t ref;
-        float t0;
-        if (wide_root(node, r, tmax, ref, t0)) {
-            stk.put(0, ref, t0);
-            level = 1;
-        }
-    }
-    while (ballot(level > 0)) {
-        wide_sync();
-        uint32_t la = 0, lcnt = 0;
-        if (level > 0) {
-            const uint32_t e = stk.get(--level).x;
-            const bool leaf = (e & WIDE_LEAF) != 0u;
-            uint32_t first = 0, cnt = 0;
-            const char* p = reinterpret_cast<const char*>(wide) + ((e << 7) | (q << 5));
-            if (leaf) {
-                wide_leaf(node, e, first, cnt);
-                p = reinterpret_cast<const char*>(tri) + 48 * (size_t)(first + (q < cnt ? q : 0u));
-            }
-            const float4* p4 = reinterpret_cast<const float4*>(p);
-            float4 f0 = p4[0], f1 = p4[1], f2 = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (leaf) f2 = p4[2];
-            if (!leaf) {
-                if (ORDERED && (e & WIDE_DEEP)) {
-                    redo = true;
-                    level = 0;
-                } else {
-                    const WideStep s = wide_step<ORDERED>(f0, f1, r, tmax, q);
-                    if (s.pass) stk.put(level + s.after, __float_as_uint(f0.w), s.t0);
-                    level += s.total;
-                }
-            } else if (cnt >= coop) {
-                la = first;
-                lcnt = cnt;
-            } else {
-                int h = 0;
-                for (uint32_t b = 0;;) {
-                    float tt, u, v;
-                    if (tri_hit_v(f0, f1, f2, r.o, r.d, &tt, &u, &v) && b + q < cnt && tt < tmax && tt > r.tmin) h = 1;
-                    b += 4;
-                    if (b >= cnt) break;
-                    const float4* t4 = tri + 3 * (size_t)(first + (b + q < cnt ? b + q : 0u));
-                    f0 = t4[0];
-                    f1 = t4[1];
-                    f2 = t4[2];
-                }
-                h |= quad_i<QX1>(h);
-                h |= quad_i<QX2>(h);
-                if (h) {
-                    found = true;
-                    level = 0;
-                }
-            }
-        }
-        if (ballot(lcnt != 0u)) {
-            RayC rc;
-            rc.o = r.o;
-            rc.d = r.d;
-            rc.tmin = r.tmin;
-            const int h = coop_any(tri, la, q == 0u ? lcnt : 0u, rc, tmax, ~0ull) ? 1 : 0;
-            if (quad_i<QFIRST>(h)) {
-                found = true;
-                level = 0;
-            }
-        }
-    }
-    return found;
-}
-
 // The reference's walk, node by node, for the rays the wide walk leaves: the
 // steps of traverse_closest_node / traverse_any_node (near child first, pops
 // only below MAX_LEVELS) with the leaf loop a triangle at a time, the same on
 // the four lanes of a group.  Few rays come here, so it is kept small.
-template <bool ANY, int GROUPS>
+template <bool ANY>
 __device__ __forceinline__ bool exact_walk(const float4* __restrict__ node, const float4* __restrict__ delta,
                                            const float4* __restrict__ tri, v3 o, v3 d, float tmin, Closest& best,
-                                           WideStack<GROUPS> stk) {
+                                           uint32_t* stk) {
     const RayC r = make_ray(o, d, tmin);
     uint32_t level = 0, curr = 0;
     for (;;) {
@@ -980,7 +826,7 @@ __device__ __forceinline__ bool exact_walk(const float4* __restrict__ node, cons
         if (slab(f0, f1, r, best.t)) {
             if (cnt == 0u) {
                 const bool nl = dot(r.d, xyz(delta[curr])) > 0.f;
-                stk.put((int)(level & (STACK - 1)), nl ? a + 1u : a, 0.f);
+                stk[(level & (STACK - 1)) * WIDE_GROUPS] = nl ? a + 1u : a;
                 ++level;
                 curr = nl ? a : a + 1u;
                 continue;
@@ -998,19 +844,305 @@ __device__ __forceinline__ bool exact_walk(const float4* __restrict__ node, cons
             }
         }
         if (level == 0 || level >= STACK) return false;
-        curr = stk.get((int)--level).x;
+        curr = stk[--level * WIDE_GROUPS];
     }
 }
 
+// Results in LDS: closest {t, u, v, id} with id -1 for no hit; any hit 0 or 1;
+// REDO: the ray is left to exact_walk.
+constexpr int32_t REDO = -2;
+// Groups that have to be idle before rays are handed out (a hand-out runs for
+// the idle groups alone): 1, 3 and 16 gave 7.03, 7.51 and 8.46 ms on the batch.
+constexpr uint32_t WIDE_REFILL = 1;
+
+// Walks the groups' rays, then rays [0, n) of the wave's LDS, all of which meet
+// the root's box; the results are left in LDS.  r, level, bt, mine: the
+// group's ray, 1 where it has one (with the root on its stack), its best
+// distance (ANY: its tMax), and its place among the results.  Leaves are
+// tested four triangles at a time, one per lane, leaves of at least `coop`
+// triangles by the whole wave.  ANY: stops a ray at its first hit with
+// tMin < t < tMax.
+template <bool ANY, bool ORDERED, bool GROUP>
+__device__ __forceinline__ void wide_walk(const float4* __restrict__ node, const float4* __restrict__ wide,
+                                          const float4* __restrict__ tri, WideLds<ANY, GROUP> lds, uint32_t root,
+                                          uint32_t n, uint32_t coop, WideRay r, int level, float bt, uint32_t mine) {
+    const uint32_t q = lane_id() & 3u;
+    uint2* const stk2 = lds.stack2();
+    uint32_t* const stk1 = lds.stack1();
+    float4* const res = lds.res();
+    uint32_t* const hit = lds.hit();
+    uint32_t next = 0;  // next ray to hand out (wave-uniform)
+    bool odd = wide_odd(r.inv);
+    bool any_odd = ballot(odd && level > 0) != 0ull;  // on any ray of the wave
+    for (;;) {
+        const uint64_t idle = ballot(level == 0);
+        if (!GROUP && next < n && (uint32_t)__builtin_popcountll(idle) >= 4u * WIDE_REFILL) {
+            const uint32_t i = next + (lanes_below(idle) >> 2);
+            if (level == 0 && i < n) {
+                const float4 a = lds.ray(0)[i], b = lds.ray(1)[i], c = lds.ray(2)[i];
+                r = WideRay{xyz(a), xyz(b), xyz(c), a.w};
+                bt = b.w;
+                odd = wide_odd(r.inv);
+                mine = i;
+                if (ANY)
+                    stk1[0] = root;
+                else
+                    stk2[0] = make_uint2(root, __float_as_uint(c.w));
+                level = 1;
+            }
+            any_odd = ballot(odd && level > 0) != 0ull;
+            next += (uint32_t)__builtin_popcountll(idle) >> 2;
+        } else if (idle == ~0ull) {
+            break;
+        }
+        wide_sync();
+        uint32_t la = 0, lcnt = 0;
+        if (level > 0) {
+            --level;
+            const uint2 e = ANY ? make_uint2(stk1[level * WIDE_GROUPS], 0u) : stk2[level * WIDE_GROUPS];
+            if (ANY || __uint_as_float(e.y) <= bt) {
+                // the slot or the group's first four triangles: one round trip
+                // whichever a group needs
+                const bool leaf = (e.x & WIDE_LEAF) != 0u;
+                uint32_t first = 0, cnt = 0;
+                const char* p = reinterpret_cast<const char*>(wide) + ((e.x << 7) | (q << 5));
+                if (leaf) {
+                    wide_leaf(node, e.x, first, cnt);
+                    p = reinterpret_cast<const char*>(tri) + 48 * (size_t)(first + (q < cnt ? q : 0u));
+                }
+                const float4* p4 = reinterpret_cast<const float4*>(p);
+                float4 f0 = p4[0], f1 = p4[1], f2 = make_float4(0.f, 0.f, 0.f, 0.f);
+                if (leaf) f2 = p4[2];
+                // keeps the loads here: the compiler would sink a copy of them into each
+                // branch, and a wave with both kinds would wait twice
+                __asm__ volatile("" : "+v"(f0.x), "+v"(f0.y), "+v"(f0.z), "+v"(f0.w), "+v"(f1.x), "+v"(f1.y), "+v"(f1.z));
+                if (!leaf) {
+                    const WideStep s = wide_step<ORDERED>(f0, f1, r, any_odd, odd, bt, q);
+                    if ((ORDERED && (e.x & WIDE_DEEP)) || level + s.total > WIDE_STACK) {
+                        if (q == 0u) {
+                            if (ANY)
+                                hit[mine] = (uint32_t)REDO;
+                            else
+                                res[mine].w = __int_as_float(REDO);
+                        }
+                        level = 0;
+                    } else {
+                        if (s.pass) {
+                            const int at = (level + s.after) * WIDE_GROUPS;
+                            if (ANY)
+                                stk1[at] = __float_as_uint(f0.w);
+                            else
+                                stk2[at] = make_uint2(__float_as_uint(f0.w), __float_as_uint(s.t0));
+                        }
+                        level += s.total;
+                    }
+                } else if (cnt >= coop) {
+                    la = first;
+                    lcnt = cnt;
+                } else {
+                    int any = 0;
+                    for (uint32_t b = 0;;) {
+                        const uint32_t i = b + q;
+                        float tt, u, v;
+                        const bool in = tri_hit_v(f0, f1, f2, r.o, r.d, &tt, &u, &v) && i < cnt;
+                        if (ANY) {
+                            if (in && tt < bt && tt > r.tmin) any = 1;
+                        } else if (ballot(in && tt <= bt && tt >= r.tmin)) {
+                            // the smallest t and, among equal ones, the latest triangle: what the
+                            // in-order loop with its `t <= best` update keeps
+                            const bool h = in && tt <= bt && tt >= r.tmin;
+                            const int id = h ? (int)(first + i) : -1;
+                            const float t = h ? tt : INFINITY;
+                            float m = fminf(t, quad_f<QX1>(t));
+                            m = fminf(m, quad_f<QX2>(m));
+                            const int w = h && t == m ? id : -1;
+                            int last = max(w, quad_i<QX1>(w));
+                            last = max(last, quad_i<QX2>(last));
+                            if (last >= 0) bt = m;
+                            if (last >= 0 && w == last) res[mine] = make_float4(tt, u, v, __int_as_float(id));
+                        }
+                        b += 4;
+                        if (b >= cnt) break;
+                        const float4* t4 = tri + 3 * (size_t)(first + (b + q < cnt ? b + q : 0u));
+                        f0 = t4[0];
+                        f1 = t4[1];
+                        f2 = t4[2];
+                    }
+                    if (ANY) {
+                        any |= quad_i<QX1>(any);
+                        any |= quad_i<QX2>(any);
+                        if (any) {
+                            if (q == 0u) hit[mine] = 1u;
+                            level = 0;
+                        }
+                    }
+                }
+            }
+        }
+        if (ballot(lcnt != 0u)) {
+            RayC rc;
+            rc.o = r.o;
+            rc.d = r.d;
+            rc.tmin = r.tmin;
+            if (ANY) {
+                const int h = coop_any(tri, la, q == 0u ? lcnt : 0u, rc, bt, ~0ull) ? 1 : 0;
+                if (quad_i<QFIRST>(h)) {
+                    if (q == 0u) hit[mine] = 1u;
+                    level = 0;
+                }
+            } else {
+                Closest c{bt, 0.f, 0.f, -1};
+                coop_closest(tri, la, q == 0u ? lcnt : 0u, rc, c, ~0ull);
+                if (q == 0u && c.id >= 0) res[mine] = make_float4(c.t, c.u, c.v, __int_as_float(c.id));
+                bt = quad_f<QFIRST>(c.t);
+            }
+        }
+    }
+    wide_sync();
+}
+
+// Closest hit (ANY: any hit, best.id 0 where there is one) of every lane's
+// ray; called by the whole wave, lanes without a ray pass start = false.  The rays wait in LDS, so that the walk has the
+// registers: rc's origin and direction and best are read back from there, and
+// hold nothing on lanes without a hit but best.id = -1.
+template <bool ANY, bool ORDERED>
+__device__ __forceinline__ void wide_rays(const float4* __restrict__ node, const float4* __restrict__ delta,
+                                          const float4* __restrict__ wide, const float4* __restrict__ tri, RayC& rc,
+                                          Closest& best, WideLds<ANY, false> lds, uint32_t coop, bool start) {
+    const float4 n0 = node[0], n1 = node[1];
+    const uint32_t root = wide_ref(0u, __float_as_uint(n0.w), __float_as_uint(n1.w));
+    uint64_t wm, rm;  // lanes whose ray is walked, and walked node by node
+    {
+        const WideRay r{rc.o, rc.d, wide_inv(rc), rc.tmin};
+        float t0;
+        // an infinite reciprocal with an infinite (or NaN) tMax: see above
+        const bool redo = start && wide_odd(r.inv) && !(best.t < INFINITY);
+        const bool walk = start && !redo && wide_slab(xyz(n0), xyz(n1), r, best.t, t0);
+        wm = ballot(walk);
+        rm = ballot(redo);
+        if (walk || redo) {
+            const uint32_t slot = walk ? lanes_below(wm) : (uint32_t)__builtin_popcountll(wm) + lanes_below(rm);
+            lds.ray(0)[slot] = make_float4(r.o.x, r.o.y, r.o.z, r.tmin);
+            lds.ray(1)[slot] = make_float4(r.d.x, r.d.y, r.d.z, best.t);
+            lds.ray(2)[slot] = make_float4(r.inv.x, r.inv.y, r.inv.z, t0);
+            if (ANY)
+                lds.hit()[slot] = walk ? 0u : (uint32_t)REDO;
+            else
+                lds.res()[slot] = make_float4(0.f, 0.f, 0.f, __int_as_float(walk ? -1 : REDO));
+        }
+    }
+    const uint32_t nw = (uint32_t)__builtin_popcountll(wm), n = nw + (uint32_t)__builtin_popcountll(rm);
+    wide_sync();
+    if (wm) wide_walk<ANY, ORDERED>(node, wide, tri, lds, root, nw, coop, WideRay{}, 0, 0.f, 0u);
+    // the rays left to the exact walk, by groups
+    const uint32_t lane = lane_id();
+    const bool left = lane < n && (ANY ? lds.hit()[lane] == (uint32_t)REDO : __float_as_int(lds.res()[lane].w) == REDO);
+    if (ballot(left)) {
+        for (uint32_t i = lane >> 2; i < n; i += WIDE_GROUPS) {
+            if (ANY ? lds.hit()[i] != (uint32_t)REDO : __float_as_int(lds.res()[i].w) != REDO) continue;
+            const float4 a = lds.ray(0)[i], b = lds.ray(1)[i];
+            Closest c{b.w, 0.f, 0.f, -1};
+            const bool h = exact_walk<ANY>(node, delta, tri, xyz(a), xyz(b), a.w, c, lds.stack1());
+            if (ANY)
+                lds.hit()[i] = h ? 1u : 0u;
+            else
+                lds.res()[i] = make_float4(c.t, c.u, c.v, __int_as_float(c.id));
+        }
+        wide_sync();
+    }
+    const bool walked = (wm >> lane) & 1ull, mine = walked || ((rm >> lane) & 1ull);
+    const uint32_t slot = mine ? (walked ? lanes_below(wm) : nw + lanes_below(rm)) : 0u;
+    if (ANY) {
+        best.id = mine && lds.hit()[slot] == 1u ? 0 : -1;
+    } else {
+        const float4 a = lds.ray(0)[slot], b = lds.ray(1)[slot], c = lds.res()[slot];
+        rc.o = xyz(a);
+        rc.d = xyz(b);
+        best = Closest{c.x, c.y, c.z, mine ? __float_as_int(c.w) : -1};
+    }
+    wide_sync();  // the wave's next rays reuse the LDS
+}
+
+// The same for WIDE_GROUP: the four lanes of a group hold the group's ray, and
+// best is the same on them.
+template <bool ANY, bool ORDERED>
+__device__ __forceinline__ void wide_group(const float4* __restrict__ node, const float4* __restrict__ delta,
+                                           const float4* __restrict__ wide, const float4* __restrict__ tri,
+                                           const RayC& rc, Closest& best, WideLds<ANY, true> lds, uint32_t coop,
+                                           bool start) {
+    const float4 n0 = node[0], n1 = node[1];
+    const uint32_t root = wide_ref(0u, __float_as_uint(n0.w), __float_as_uint(n1.w));
+    const uint32_t group = lane_id() >> 2;
+    const WideRay r{rc.o, rc.d, wide_inv(rc), rc.tmin};
+    float t0;
+    // an infinite reciprocal with an infinite (or NaN) tMax: see above
+    const bool redo = start && wide_odd(r.inv) && !(best.t < INFINITY);
+    const bool walk = start && !redo && wide_slab(xyz(n0), xyz(n1), r, best.t, t0);
+    if (ANY)
+        lds.hit()[group] = redo ? (uint32_t)REDO : 0u;
+    else
+        lds.res()[group] = make_float4(0.f, 0.f, 0.f, __int_as_float(redo ? REDO : -1));
+    if (walk) {
+        if (ANY)
+            lds.stack1()[0] = root;
+        else
+            lds.stack2()[0] = make_uint2(root, __float_as_uint(t0));
+    }
+    const float tmax = best.t;
+    wide_walk<ANY, ORDERED>(node, wide, tri, lds, root, 0u, coop, r, walk ? 1 : 0, tmax, group);
+    if (ANY) {
+        best.id = lds.hit()[group] == 1u ? 0 : -1;
+        if (lds.hit()[group] == (uint32_t)REDO) {
+            Closest c{tmax, 0.f, 0.f, -1};
+            if (exact_walk<true>(node, delta, tri, r.o, r.d, r.tmin, c, lds.stack1())) best.id = 0;
+        }
+    } else {
+        const float4 c = lds.res()[group];
+        best = Closest{c.x, c.y, c.z, __float_as_int(c.w)};
+        if (best.id == REDO) {
+            best = Closest{tmax, 0.f, 0.f, -1};
+            exact_walk<false>(node, delta, tri, r.o, r.d, r.tmin, best, lds.stack1());
+        }
+    }
+    wide_sync();  // the wave's next rays reuse the LDS
+}
+
+// The forms of this walk in the kernels' VAR parameter (trace_variant 1 where
+// the tree has wide records).
+constexpr int WIDE = WF_WIDE, WIDE_GROUP = WF_WIDE + 1;
+template <int VAR>
+constexpr bool is_wide() {
+    return VAR == WIDE || VAR == WIDE_GROUP;
+}
+// LDS of a block's walks, the type that hands it to them, and the waves per
+// SIMD that the kernel's registers have to allow (the wide walk is bound by
+// VALU issue and fetch latency: 5 and 7 waves gave 5681 and 5013 us on water).
+template <int VAR, int TB, int SR, bool ANY>
+constexpr int walk_words() {
+    return is_wide<VAR>() ? TB / RTX_WAVE * WideLds<ANY, VAR == WIDE_GROUP>::WORDS : (VAR == 4 ? 1 : SR * TB);
+}
+template <int VAR, int TB, int SR, bool ANY>
+using WalkStack =
+    typename std::conditional<is_wide<VAR>(), WideLds<ANY, VAR == WIDE_GROUP>, TraversalStack<TB, SR>>::type;
+template <int VAR>
+constexpr int walk_waves() {
+    return is_wide<VAR>() ? 7 : 1;
+}
+
 // Variant dispatch: 0 = single node, 1 = single node + early delta load,
-// 2 = sibling pairs.
+// 2 = sibling pairs, WIDE = the wide walk.
 // Called by every lane of the wave; `start` says whether the lane has a ray.
 template <int VAR, class Stack>
 __device__ __forceinline__ void closest_var(const float4* __restrict__ node, const float4* __restrict__ delta,
-                                            const float4* __restrict__ tri, const RayC& r, Closest& best,
-                                            Stack& stk, uint32_t coop, bool start,
-                                            const uint32_t* __restrict__ parent = nullptr, uint32_t bound = 0) {
-    if (VAR == 4) {
+                                            const float4* __restrict__ tri, RayC& r, Closest& best, Stack& stk,
+                                            uint32_t coop, bool start,
+                                            const uint32_t* __restrict__ parent = nullptr, uint32_t bound = 0,
+                                            const float4* __restrict__ wide = nullptr) {
+    if constexpr (VAR == WIDE) {
+        wide_rays<false, true>(node, delta, wide, tri, r, best, stk, coop, start);
+    } else if constexpr (VAR == WIDE_GROUP) {
+        wide_group<false, true>(node, delta, wide, tri, r, best, stk, coop, start);
+    } else if (VAR == 4) {
         if (start) traverse_closest_ns(node, delta, parent, tri, r, best, bound);
     } else if (VAR == 2) {
         if (start) traverse_closest(node, tri, r, best, stk);
@@ -1023,21 +1155,36 @@ __device__ __forceinline__ void closest_var(const float4* __restrict__ node, con
 // see traverse_any_node; wave-uniform).
 template <int VAR, class Stack>
 __device__ __forceinline__ bool any_var(const float4* __restrict__ node, const float4* __restrict__ delta,
-                                        const float4* __restrict__ tri, const RayC& r, float tmax, Stack& stk,
+                                        const float4* __restrict__ tri, RayC& r, float tmax, Stack& stk,
                                         uint32_t coop, bool start, const uint32_t* __restrict__ parent = nullptr,
-                                        uint32_t bound = 0, bool ordered = true) {
-    if (VAR == 4) {
+                                        uint32_t bound = 0, bool ordered = true,
+                                        const float4* __restrict__ wide = nullptr) {
+    if constexpr (is_wide<VAR>()) {
+        Closest c{tmax, 0.f, 0.f, -1};
+        if constexpr (VAR == WIDE) {
+            if (ordered)
+                wide_rays<true, true>(node, delta, wide, tri, r, c, stk, coop, start);
+            else
+                wide_rays<true, false>(node, delta, wide, tri, r, c, stk, coop, start);
+        } else {
+            if (ordered)
+                wide_group<true, true>(node, delta, wide, tri, r, c, stk, coop, start);
+            else
+                wide_group<true, false>(node, delta, wide, tri, r, c, stk, coop, start);
+        }
+        return c.id >= 0;
+    } else if constexpr (VAR == 4) {
         bool h = false;
         if (start) h = traverse_any_ns(node, delta, parent, tri, r, tmax, bound, ordered);
         return h;
-    }
-    if (VAR == 2) {
+    } else if constexpr (VAR == 2) {
         bool h = false;
         if (start) h = traverse_any(node, tri, r, tmax, stk);
         return h;
+    } else {
+        if (!ordered) return traverse_any_node<false, false>(node, delta, tri, r, tmax, stk, coop, start);
+        return traverse_any_node<VAR == 1, true>(node, delta, tri, r, tmax, stk, coop, start);
     }
-    if (!ordered) return traverse_any_node<false, false>(node, delta, tri, r, tmax, stk, coop, start);
-    return traverse_any_node<VAR == 1, true>(node, delta, tri, r, tmax, stk, coop, start);
 }
 
 // -------------------------------------------------------------- trace ----
@@ -1087,7 +1234,7 @@ __device__ __forceinline__ void write_hit_record(const float4* __restrict__ tri,
 // also appended (wave-aggregated) to the bundle's hit list, which the shadow
 // stage walks densely.
 template <int VAR, int TB, int SR>
-__global__ __launch_bounds__(TB) void k_trace(const float4* __restrict__ node, const float4* __restrict__ delta,
+__global__ __launch_bounds__(TB, walk_waves<VAR>()) void k_trace(const float4* __restrict__ node, const float4* __restrict__ delta,
                                               const float4* __restrict__ tri,
                                               const float4* __restrict__ nrm, const float2* __restrict__ uvs,
                                               const float4* __restrict__ ori4, const float4* __restrict__ dir4,
@@ -1097,16 +1244,18 @@ __global__ __launch_bounds__(TB) void k_trace(const float4* __restrict__ node, c
                                               float4* __restrict__ n4, float4* __restrict__ p4,
                                               float2* __restrict__ uv2, uint32_t* __restrict__ hit_list,
                                               uint32_t* __restrict__ hit_count, uint32_t xcds, uint32_t coop,
-                                              const uint32_t* __restrict__ parent, uint32_t bound) {
-    __shared__ uint32_t s_id[VAR == 4 ? 1 : SR * TB];
+                                              const uint32_t* __restrict__ parent, uint32_t bound,
+                                              const float4* __restrict__ wide) {
+    __shared__ __align__(16) uint32_t s_id[walk_words<VAR, TB, SR, false>()];
     uint32_t s_low[stack_private_words<SR>()];
-    TraversalStack<TB, SR> stk{s_id, threadIdx.x, s_low};
+    WalkStack<VAR, TB, SR, false> stk{s_id, threadIdx.x, s_low};
     const uint64_t n = ray_count(dcount, hcount);
     const uint32_t lane = threadIdx.x & 63;
-    const XcdSpan sp = xcd_span(n, xcds, TB);
+    constexpr uint32_t LANES = VAR == WIDE_GROUP ? 4u : 1u;  // lanes per ray
+    const XcdSpan sp = xcd_span(n, xcds, TB / LANES);
     for (uint64_t base = sp.begin; base < sp.end; base += sp.stride) {
-        const uint64_t rr = base + threadIdx.x;
-        const bool active = rr < sp.end;
+        const uint64_t rr = base + threadIdx.x / LANES;
+        bool active = rr < sp.end;
         Closest best{0.f, 0.f, 0.f, -1};
         RayC rc{};
         if (active) {
@@ -1114,7 +1263,8 @@ __global__ __launch_bounds__(TB) void k_trace(const float4* __restrict__ node, c
             rc = make_ray(xyz(o), xyz(dd), o.w);
             best.t = dd.w;
         }
-        closest_var<VAR>(node, delta, tri, rc, best, stk, coop, active, parent, bound);  // whole wave
+        closest_var<VAR>(node, delta, tri, rc, best, stk, coop, active, parent, bound, wide);  // whole wave
+        active = active && threadIdx.x % LANES == 0u;
         const bool hit = active && best.id >= 0;
         const uint64_t hb = ballot(hit);
         uint32_t wbase = 0;
@@ -1130,79 +1280,6 @@ __global__ __launch_bounds__(TB) void k_trace(const float4* __restrict__ node, c
         hit_list[wbase + lanes_below(hb)] = (uint32_t)rr;
         write_hit_record(tri, nrm, uvs, rc, best, rr, flags, tout, idout, bary, n4, p4, uv2);
     }
-}
-
-// Where a closest-hit launch reads its rays and writes its records.
-struct TraceIo {
-    const float4* __restrict__ node;
-    const float4* __restrict__ delta;
-    const float4* __restrict__ wide;
-    const float4* __restrict__ tri;
-    const float4* __restrict__ nrm;
-    const float2* __restrict__ uvs;
-    const float4* __restrict__ ori4;
-    const float4* __restrict__ dir4;
-    uint32_t* __restrict__ flags;
-    float* __restrict__ t;
-    int32_t* __restrict__ id;
-    float2* __restrict__ bary;
-    float4* __restrict__ n4;
-    float4* __restrict__ p4;
-    float2* __restrict__ uv2;
-    uint32_t* __restrict__ list;
-    uint32_t* __restrict__ list_count;
-};
-
-// Closest hit and record of the group's ray rr, by the wide walk; called by
-// the whole wave.
-template <int GROUPS>
-__device__ __forceinline__ void wide_trace(const TraceIo& io, uint64_t rr, bool active, WideStack<GROUPS> stk,
-                                           uint32_t coop) {
-    Closest best{0.f, 0.f, 0.f, -1};
-    WideRay r{};
-    bool redo = false;
-    if (active) {
-        const float4 o = io.ori4[rr], dd = io.dir4[rr];
-        const RayC rc = make_ray(xyz(o), xyz(dd), o.w);
-        r = wide_ray(rc);
-        redo = wide_odd(rc);
-        best.t = dd.w;
-    }
-    if (wide_closest<GROUPS>(io.node, io.wide, io.tri, r, best, stk, coop, active && !redo)) redo = true;
-    if (redo) {
-        best = Closest{io.dir4[rr].w, 0.f, 0.f, -1};
-        exact_walk<false, GROUPS>(io.node, io.delta, io.tri, r.o, r.d, r.tmin, best, stk);
-    }
-    const bool mine = active && (lane_id() & 3u) == 0u, hit = mine && best.id >= 0;
-    const uint64_t hb = ballot(hit);
-    uint32_t wbase = 0;
-    if (hb) {
-        if (lane_id() == (uint32_t)__builtin_ctzll(hb))
-            wbase = atomicAdd(io.list_count, (uint32_t)__builtin_popcountll(hb));
-        wbase = __shfl(wbase, __builtin_ctzll(hb), RTX_WAVE);
-    }
-    if (!mine) return;
-    if (!hit) {
-        write_miss_record(rr, io.flags, io.t, io.id, io.bary, io.n4, io.p4, io.uv2);
-        return;
-    }
-    io.list[wbase + lanes_below(hb)] = (uint32_t)rr;
-    RayC rc;
-    rc.o = r.o;
-    rc.d = r.d;
-    write_hit_record(io.tri, io.nrm, io.uvs, rc, best, rr, io.flags, io.t, io.id, io.bary, io.n4, io.p4, io.uv2);
-}
-
-// The wide walk: a block of TB threads holds TB / 4 rays.
-template <int TB>
-__global__ __launch_bounds__(TB) void k_trace_w(TraceIo io, const uint32_t* __restrict__ dcount, uint64_t hcount,
-                                                uint32_t coop) {
-    constexpr int GROUPS = TB / 4;
-    __shared__ uint2 s_stk[WIDE_STACK * GROUPS];
-    const uint32_t group = threadIdx.x >> 2;
-    const uint64_t n = ray_count(dcount, hcount);
-    for (uint64_t base = (uint64_t)blockIdx.x * GROUPS; base < n; base += (uint64_t)gridDim.x * GROUPS)
-        wide_trace<GROUPS>(io, base + group, base + group < n, WideStack<GROUPS>{s_stk + group}, coop);
 }
 
 // Hit list from the flags (when hits were written from the host).
@@ -1262,16 +1339,16 @@ __device__ __forceinline__ void set_shadow_bit(uint32_t* f, int l, bool shadowed
 // (outside the cone = shadowed), POINT toward pos with tMax = distance; any
 // hit with tMin 0.01 < t < tMax sets bit 8+l of the ray's flags.
 template <int VAR, int TB, int SR>
-__global__ __launch_bounds__(TB) void k_shadow(const float4* __restrict__ node, const float4* __restrict__ delta,
+__global__ __launch_bounds__(TB, walk_waves<VAR>()) void k_shadow(const float4* __restrict__ node, const float4* __restrict__ delta,
                                                const float4* __restrict__ tri, const rtx_lights* __restrict__ lights,
                                                ShadowSegs segs, unsigned long long* shadow_count, uint32_t xcds,
                                                uint32_t coop, const uint32_t* __restrict__ parent, uint32_t bound,
-                                               uint32_t ordered) {
-    __shared__ uint32_t s_id[VAR == 4 ? 1 : SR * TB];
+                                               uint32_t ordered, const float4* __restrict__ wide) {
+    __shared__ __align__(16) uint32_t s_id[walk_words<VAR, TB, SR, true>()];
     __shared__ uint32_t s_cnt;
     __shared__ uint64_t s_end[RTX_SEG_MAX];
     uint32_t s_low[stack_private_words<SR>()];
-    TraversalStack<TB, SR> stk{s_id, threadIdx.x, s_low};
+    WalkStack<VAR, TB, SR, true> stk{s_id, threadIdx.x, s_low};
     const int nl = lights->count;
     if (threadIdx.x == 0) {
         s_cnt = 0;
@@ -1284,11 +1361,12 @@ __global__ __launch_bounds__(TB) void k_shadow(const float4* __restrict__ node, 
     __syncthreads();
     const uint64_t items = segs.n ? s_end[segs.n - 1] : 0;
     uint32_t traced = 0;
-    const XcdSpan sp = xcd_span(items, xcds, TB);
+    constexpr uint32_t LANES = VAR == WIDE_GROUP ? 4u : 1u;  // lanes per item
+    const XcdSpan sp = xcd_span(items, xcds, TB / LANES);
     // wave-uniform loop: every lane reaches the traversal call (lanes past the
     // end or with nothing to trace pass start = false)
     for (uint64_t base = sp.begin; base < sp.end; base += sp.stride) {
-        const uint64_t it = base + threadIdx.x;
+        const uint64_t it = base + threadIdx.x / LANES;
         const bool valid = it < sp.end;
         uint32_t rr = 0;
         int l = 0;
@@ -1326,109 +1404,13 @@ __global__ __launch_bounds__(TB) void k_shadow(const float4* __restrict__ node, 
                 trace = false;
             }
             if (trace) {
-                ++traced;
+                if (threadIdx.x % LANES == 0u) ++traced;
                 rc = make_ray(p, dir, 0.01f);
             }
         }
-        if (any_var<VAR>(node, delta, tri, rc, tmax, stk, coop, trace, parent, bound, ordered != 0))  // whole wave
+        if (any_var<VAR>(node, delta, tri, rc, tmax, stk, coop, trace, parent, bound, ordered != 0, wide))  // whole wave
             shadowed = true;
-        if (valid) set_shadow_bit(&fl[rr], l, shadowed);
-    }
-    if (shadow_count) {
-        if (traced) atomicAdd(&s_cnt, traced);
-        __syncthreads();
-        if (threadIdx.x == 0 && s_cnt) atomicAdd(shadow_count, (unsigned long long)s_cnt);
-    }
-}
-
-// The shadow ray of point p toward light L (shadow_trace_single): false where
-// none is traced, with `shadowed` the result.
-__device__ __forceinline__ bool shadow_ray(const rtx_light& L, v3 p, v3& dir, float& tmax, bool& shadowed) {
-    tmax = 1e37f;
-    if (L.type == RTX_LIGHT_DIR) {
-        dir = -mk3(L.dir[0], L.dir[1], L.dir[2]);
-        return true;
-    }
-    if (L.type == RTX_LIGHT_SPOT) {
-        dir = normalize(mk3(L.pos[0], L.pos[1], L.pos[2]) - p);
-        if (!(dot(-dir, mk3(L.dir[0], L.dir[1], L.dir[2])) < L.angle)) return true;
-    } else if (L.type == RTX_LIGHT_POINT) {
-        const v3 toL = mk3(L.pos[0], L.pos[1], L.pos[2]) - p;
-        tmax = __builtin_sqrtf(dot(toL, toL));
-        dir = normalize(toL);
-        return true;
-    }
-    shadowed = true;
-    return false;
-}
-
-// Shadow bit of the group's (hit rr, light l) pair, by the wide walk; called
-// by the whole wave.  Returns whether a ray was traced.
-template <bool ORDERED, int GROUPS>
-__device__ __forceinline__ bool wide_shadow(const float4* __restrict__ node, const float4* __restrict__ delta,
-                                            const float4* __restrict__ wide, const float4* __restrict__ tri,
-                                            const rtx_lights* __restrict__ lights, const float4* __restrict__ p4,
-                                            uint32_t* __restrict__ flags, uint32_t rr, int l, bool valid,
-                                            WideStack<GROUPS> stk, uint32_t coop) {
-    WideRay r{};
-    float tmax = 1e37f;
-    bool shadowed = false, trace = false, redo = false;
-    if (valid) {
-        const v3 p = xyz(p4[rr]);
-        v3 dir = mk3(0.f, 0.f, 0.f);
-        trace = shadow_ray(lights->l[l], p, dir, tmax, shadowed);
-        if (trace) {
-            const RayC rc = make_ray(p, dir, 0.01f);
-            r = wide_ray(rc);
-            redo = wide_odd(rc);
-        }
-    }
-    if (wide_any<ORDERED, GROUPS>(node, wide, tri, r, tmax, stk, coop, trace && !redo, redo)) shadowed = true;
-    if (redo) {
-        Closest c{tmax, 0.f, 0.f, -1};
-        shadowed = exact_walk<true, GROUPS>(node, delta, tri, r.o, r.d, r.tmin, c, stk);
-    }
-    if (valid && (lane_id() & 3u) == 0u) set_shadow_bit(&flags[rr], l, shadowed);
-    return trace;
-}
-
-template <bool ORDERED, int TB>
-__global__ __launch_bounds__(TB) void k_shadow_w(const float4* __restrict__ node, const float4* __restrict__ delta,
-                                                 const float4* __restrict__ wide, const float4* __restrict__ tri,
-                                                 const rtx_lights* __restrict__ lights, ShadowSegs segs,
-                                                 unsigned long long* shadow_count, uint32_t coop) {
-    constexpr int GROUPS = TB / 4;
-    __shared__ uint2 s_stk[WIDE_STACK * GROUPS];
-    __shared__ uint32_t s_cnt;
-    __shared__ uint64_t s_end[RTX_SEG_MAX];
-    const uint32_t group = threadIdx.x >> 2;
-    const int nl = lights->count;
-    if (threadIdx.x == 0) {
-        s_cnt = 0;
-        uint64_t acc = 0;
-        for (int k = 0; k < segs.n; ++k) {
-            acc += (uint64_t)(*segs.s[k].count) * (uint64_t)nl;
-            s_end[k] = acc;
-        }
-    }
-    __syncthreads();
-    const uint64_t items = segs.n ? s_end[segs.n - 1] : 0;
-    uint32_t traced = 0;
-    for (uint64_t base = (uint64_t)blockIdx.x * GROUPS; base < items; base += (uint64_t)gridDim.x * GROUPS) {
-        const uint64_t it = base + group;
-        const bool valid = it < items;
-        uint32_t rr = 0;
-        int l = 0, sg = 0;
-        if (valid) {
-            while (it >= s_end[sg]) ++sg;
-            const uint64_t first = sg ? s_end[sg - 1] : 0, local = it - first, nh = (s_end[sg] - first) / (uint64_t)nl;
-            rr = segs.s[sg].list[local % nh];  // light-major, as k_shadow
-            l = (int)(local / nh);
-        }
-        if (wide_shadow<ORDERED, GROUPS>(node, delta, wide, tri, lights, segs.s[sg].p4, segs.s[sg].flags, rr, l, valid,
-                                         WideStack<GROUPS>{s_stk + group}, coop) &&
-            (threadIdx.x & 3u) == 0u)
-            ++traced;
+        if (valid && threadIdx.x % LANES == 0u) set_shadow_bit(&fl[rr], l, shadowed);
     }
     if (shadow_count) {
         if (traced) atomicAdd(&s_cnt, traced);
@@ -1750,20 +1732,33 @@ __global__ __launch_bounds__(TB) void k_shadow_p(const float4* __restrict__ node
     } while (0)
 #define RTX_DISPATCH_STACK(M, var, tb, sr)                  \
     do {                                                    \
-        if (sr == 8) RTX_DISPATCH_VB(M, var, tb, 8);        \
+        if (var == WIDE) {                                  \
+            if (tb == 64) M(WIDE, 64, 32);                  \
+            else if (tb == 256) M(WIDE, 256, 32);           \
+            else M(WIDE, 128, 32);                          \
+        } else if (sr == 8) RTX_DISPATCH_VB(M, var, tb, 8); \
         else if (sr == 16) RTX_DISPATCH_VB(M, var, tb, 16); \
         else RTX_DISPATCH_VB(M, var, tb, 32);               \
     } while (0)
-// Scene kernels: also the stackless form (4), which has no stack.
-#define RTX_DISPATCH_STACK_NS(M, var, tb, sr)   \
-    do {                                        \
-        if (var == 4) {                         \
-            if (tb == 64) M(4, 64, 32);         \
-            else if (tb == 256) M(4, 256, 32);  \
-            else M(4, 128, 32);                 \
-        } else {                                \
-            RTX_DISPATCH_STACK(M, var, tb, sr); \
-        }                                       \
+// Scene kernels: also the stackless form (4), which has no stack, and the wide
+// walk with a ray per group.
+#define RTX_DISPATCH_STACK_NS(M, var, tb, sr)           \
+    do {                                                \
+        if (var == 4) {                                 \
+            if (tb == 64) M(4, 64, 32);                 \
+            else if (tb == 256) M(4, 256, 32);          \
+            else M(4, 128, 32);                         \
+        } else if (var == WIDE_GROUP) {                 \
+            if (tb == 64) M(WIDE_GROUP, 64, 32);        \
+            else if (tb == 256) M(WIDE_GROUP, 256, 32); \
+            else M(WIDE_GROUP, 128, 32);                \
+        } else if (sr == 8) {                           \
+            RTX_DISPATCH_VB(M, var, tb, 8);             \
+        } else if (sr == 16) {                          \
+            RTX_DISPATCH_VB(M, var, tb, 16);            \
+        } else {                                        \
+            RTX_DISPATCH_VB(M, var, tb, 32);            \
+        }                                               \
     } while (0)
 
 // Persistent traversal grid: enough groups to fill every CU at 20 waves
@@ -1887,7 +1882,7 @@ __global__ __launch_bounds__(TB) void k_trace_inst(const InstRoot* __restrict__ 
         for (int i = 0; i < nroots; ++i) {  // wave-uniform
             const InstRoot& R = roots[i];
             const v3 to = mul_h(R.tr_inv, o, 1.f, 1e-26f), td = mul_h(R.tr_inv, d, 0.f, 1e-26f);
-            const RayC rc = make_ray(to, td, tmin);
+            RayC rc = make_ray(to, td, tmin);
             Closest c{tmax, 0.f, 0.f, -1};
             closest_var<VAR>(R.node, R.delta, R.tri, rc, c, stk, coop, active);  // whole wave
             if (active && c.id >= 0) {
@@ -2478,9 +2473,6 @@ __global__ __launch_bounds__(256) void k_wf_raygen(const WfSeg* __restrict__ seg
     }
 }
 
-// Closest hit over every frame's rays: persistent waves take 64-ray chunks
-// (ChunkSched).  A chunk that starts a secondary-generation tile also clears
-// that tile's look-back word for this step's generation.
 // One 64-ray chunk (chunk cl of segment S) of the closest-hit launch; the
 // whole wave calls it.  A chunk that starts a secondary-generation tile also
 // clears that tile's look-back word for this step's generation.
@@ -2498,7 +2490,8 @@ __device__ __forceinline__ void wf_trace_chunk(const WfSeg& S, uint32_t cl, Stac
         rc = make_ray(xyz(o), xyz(dd), o.w);
         best.t = dd.w;
     }
-    closest_var<VAR>(gptr(S.node), gptr(S.delta), gptr(S.tri), rc, best, stk, coop, active);  // whole wave
+    closest_var<VAR>(gptr(S.node), gptr(S.delta), gptr(S.tri), rc, best, stk, coop, active, nullptr, 0,
+                     gptr(S.wide));  // whole wave
     const bool hit = active && best.id >= 0;
     const uint64_t hb = ballot(hit);
     uint32_t wbase = 0;
@@ -2521,11 +2514,11 @@ __device__ __forceinline__ void wf_trace_chunk(const WfSeg& S, uint32_t cl, Stac
 // Closest hit over every frame's rays, persistent form: waves take 64-ray
 // chunks (ChunkSched).
 template <int VAR, int TB, int SR>
-__global__ __launch_bounds__(TB) void k_wf_trace(const WfSeg* __restrict__ segs, uint32_t nseg,
+__global__ __launch_bounds__(TB, walk_waves<VAR>()) void k_wf_trace(const WfSeg* __restrict__ segs, uint32_t nseg,
                                                  uint32_t* __restrict__ queue, uint32_t coop, uint32_t grain) {
-    __shared__ uint32_t s_id[SR * TB];
+    __shared__ __align__(16) uint32_t s_id[walk_words<VAR, TB, SR, false>()];
     uint32_t s_low[stack_private_words<SR>()];
-    TraversalStack<TB, SR> stk{s_id, threadIdx.x, s_low};
+    WalkStack<VAR, TB, SR, false> stk{s_id, threadIdx.x, s_low};
     WaveChunks<WF_RAYS> wc;
     wc.init(segs, nseg, RTX_WAVE);
     ChunkSched sch;
@@ -2543,67 +2536,19 @@ __global__ __launch_bounds__(TB) void k_wf_trace(const WfSeg* __restrict__ segs,
 // chunks in order, so the waves in flight always cover neighbouring rays,
 // with no queue atomics; waves past the step's chunk total leave at once.
 template <int VAR, int TB, int SR>
-__global__ __launch_bounds__(TB) void k_wf_trace_ord(const WfSeg* __restrict__ segs, uint32_t nseg,
+__global__ __launch_bounds__(TB, walk_waves<VAR>()) void k_wf_trace_ord(const WfSeg* __restrict__ segs, uint32_t nseg,
                                                      const uint32_t* __restrict__ ctr, uint32_t coop) {
-    __shared__ uint32_t s_id[SR * TB];
+    __shared__ __align__(16) uint32_t s_id[walk_words<VAR, TB, SR, false>()];
     const uint32_t total = ctr[WF_TOTAL];
     const uint32_t c = blockIdx.x * (TB / RTX_WAVE) + threadIdx.x / RTX_WAVE;
     if (c >= total) return;  // whole waves (no block barrier follows)
     uint32_t s_low[stack_private_words<SR>()];
-    TraversalStack<TB, SR> stk{s_id, threadIdx.x, s_low};
+    WalkStack<VAR, TB, SR, false> stk{s_id, threadIdx.x, s_low};
     WaveChunks<WF_RAYS> wc;
     wc.load(ctr + WF_TAB, nseg, total);
     uint32_t c0 = 0;
     const uint32_t sg = __builtin_amdgcn_readfirstlane(wc.find(c, c0));
     wf_trace_chunk<VAR>(segs[sg], c - c0, stk, coop, threadIdx.x & (RTX_WAVE - 1));
-}
-
-// The same by the wide walk: the chunk's 64 rays as four rounds of 16.
-template <int GROUPS>
-__device__ __forceinline__ void wf_trace_chunk_w(const WfSeg& S, uint32_t cl, WideStack<GROUPS> stk, uint32_t coop,
-                                                 uint32_t lane) {
-    constexpr uint32_t PER_TILE = WF_GEN_TILE / RTX_WAVE;
-    if (S.gen && cl % PER_TILE == 0u && lane == 0) S.status[cl / PER_TILE] = 0u;
-    const uint32_t n = S.count[0];
-    const TraceIo io{gptr(S.node), gptr(S.delta), gptr(S.wide), gptr(S.tri), gptr(S.nrm), gptr(S.uv), gptr(S.ori4),
-                     gptr(S.dir4), gptr(S.flags), gptr(S.t), gptr(S.id), gptr(S.bary), gptr(S.n4), gptr(S.p4),
-                     gptr(S.uv2), gptr(S.list), S.list_count};
-#pragma unroll 1
-    for (uint32_t k = 0; k < 4u && cl * RTX_WAVE + 16u * k < n; ++k) {
-        const uint32_t rr = cl * RTX_WAVE + 16u * k + (lane >> 2);
-        wide_trace<GROUPS>(io, rr, rr < n, stk, coop);
-    }
-}
-
-template <int TB>
-__global__ __launch_bounds__(TB) void k_wf_trace_w(const WfSeg* __restrict__ segs, uint32_t nseg,
-                                                   uint32_t* __restrict__ queue, uint32_t coop, uint32_t grain) {
-    __shared__ uint2 s_stk[WIDE_STACK * (TB / 4)];
-    WaveChunks<WF_RAYS> wc;
-    wc.init(segs, nseg, RTX_WAVE);
-    ChunkSched sch;
-    sch.init(wc.total, queue, grain);
-    for (uint32_t c = 0; sch.next(c);) {
-        uint32_t c0 = 0;
-        const uint32_t sg = __builtin_amdgcn_readfirstlane(wc.find(c, c0));
-        wf_trace_chunk_w<TB / 4>(segs[sg], c - c0, WideStack<TB / 4>{s_stk + (threadIdx.x >> 2)}, coop,
-                                 threadIdx.x & (RTX_WAVE - 1));
-    }
-}
-
-template <int TB>
-__global__ __launch_bounds__(TB) void k_wf_trace_ord_w(const WfSeg* __restrict__ segs, uint32_t nseg,
-                                                       const uint32_t* __restrict__ ctr, uint32_t coop) {
-    __shared__ uint2 s_stk[WIDE_STACK * (TB / 4)];
-    const uint32_t total = ctr[WF_TOTAL];
-    const uint32_t c = blockIdx.x * (TB / RTX_WAVE) + threadIdx.x / RTX_WAVE;
-    if (c >= total) return;  // whole waves (no block barrier follows)
-    WaveChunks<WF_RAYS> wc;
-    wc.load(ctr + WF_TAB, nseg, total);
-    uint32_t c0 = 0;
-    const uint32_t sg = __builtin_amdgcn_readfirstlane(wc.find(c, c0));
-    wf_trace_chunk_w<TB / 4>(segs[sg], c - c0, WideStack<TB / 4>{s_stk + (threadIdx.x >> 2)}, coop,
-                             threadIdx.x & (RTX_WAVE - 1));
 }
 
 // One 64-pair chunk (chunk cl of segment S) of the shadow launch: the
@@ -2646,8 +2591,8 @@ __device__ __forceinline__ void wf_shadow_chunk(const WfSeg& S, uint32_t cl, Sta
         }
         if (trace) rc = make_ray(p, dir, 0.01f);
     }
-    if (any_var<VAR>(gptr(S.node), gptr(S.delta), gptr(S.tri), rc, tmax, stk, coop, trace, nullptr, 0,
-                     ordered))  // whole wave
+    if (any_var<VAR>(gptr(S.node), gptr(S.delta), gptr(S.tri), rc, tmax, stk, coop, trace, nullptr, 0, ordered,
+                     gptr(S.wide)))  // whole wave
         shadowed = true;
     if (valid) set_shadow_bit(gptr(S.flags) + rr, l, shadowed);
     const uint64_t tb = ballot(trace);
@@ -2656,12 +2601,12 @@ __device__ __forceinline__ void wf_shadow_chunk(const WfSeg& S, uint32_t cl, Sta
 
 // Shadow rays of every frame's pairs, persistent form (ChunkSched).
 template <int VAR, int TB, int SR>
-__global__ __launch_bounds__(TB) void k_wf_shadow(const WfSeg* __restrict__ segs, uint32_t nseg,
+__global__ __launch_bounds__(TB, walk_waves<VAR>()) void k_wf_shadow(const WfSeg* __restrict__ segs, uint32_t nseg,
                                                   uint32_t* __restrict__ queue, uint32_t coop, uint32_t grain,
                                                   uint32_t ordered) {
-    __shared__ uint32_t s_id[SR * TB];
+    __shared__ __align__(16) uint32_t s_id[walk_words<VAR, TB, SR, true>()];
     uint32_t s_low[stack_private_words<SR>()];
-    TraversalStack<TB, SR> stk{s_id, threadIdx.x, s_low};
+    WalkStack<VAR, TB, SR, true> stk{s_id, threadIdx.x, s_low};
     WaveChunks<WF_PAIRS> wc;
     wc.init(segs, nseg, RTX_WAVE);
     ChunkSched sch;
@@ -2672,60 +2617,6 @@ __global__ __launch_bounds__(TB) void k_wf_shadow(const WfSeg* __restrict__ segs
         const uint32_t sg = __builtin_amdgcn_readfirstlane(wc.find(c, c0));
         wf_shadow_chunk<VAR>(segs[sg], c - c0, stk, coop, lane, ordered != 0);
     }
-}
-
-// The same by the wide walk.
-template <bool ORDERED, int GROUPS>
-__device__ __forceinline__ void wf_shadow_chunk_w(const WfSeg& S, uint32_t cl, WideStack<GROUPS> stk, uint32_t coop,
-                                                  uint32_t lane) {
-    const uint64_t nh = S.list_count[0], items = nh * (uint64_t)S.lights->count;
-    uint32_t traced = 0;
-#pragma unroll 1
-    for (uint32_t k = 0; k < 4u && (uint64_t)cl * RTX_WAVE + 16u * k < items; ++k) {
-        const uint64_t it = (uint64_t)cl * RTX_WAVE + 16u * k + (lane >> 2);
-        const bool valid = it < items;
-        uint32_t rr = 0;
-        int l = 0;
-        if (valid) {
-            rr = gptr(S.list)[it % nh];
-            l = (int)(it / nh);
-        }
-        const bool t = wide_shadow<ORDERED, GROUPS>(gptr(S.node), gptr(S.delta), gptr(S.wide), gptr(S.tri),
-                                                    gptr(S.lights), gptr(S.p4), gptr(S.flags), rr, l, valid, stk, coop);
-        traced += (uint32_t)__builtin_popcountll(ballot(t && (lane & 3u) == 0u));
-    }
-    if (lane == 0 && traced) atomicAdd(&S.stats[1], (unsigned long long)traced);
-}
-
-template <bool ORDERED, int TB>
-__global__ __launch_bounds__(TB) void k_wf_shadow_w(const WfSeg* __restrict__ segs, uint32_t nseg,
-                                                    uint32_t* __restrict__ queue, uint32_t coop, uint32_t grain) {
-    __shared__ uint2 s_stk[WIDE_STACK * (TB / 4)];
-    WaveChunks<WF_PAIRS> wc;
-    wc.init(segs, nseg, RTX_WAVE);
-    ChunkSched sch;
-    sch.init(wc.total, queue, grain);
-    for (uint32_t c = 0; sch.next(c);) {
-        uint32_t c0 = 0;
-        const uint32_t sg = __builtin_amdgcn_readfirstlane(wc.find(c, c0));
-        wf_shadow_chunk_w<ORDERED, TB / 4>(segs[sg], c - c0, WideStack<TB / 4>{s_stk + (threadIdx.x >> 2)}, coop,
-                                           threadIdx.x & (RTX_WAVE - 1));
-    }
-}
-
-template <bool ORDERED, int TB>
-__global__ __launch_bounds__(TB) void k_wf_shadow_ord_w(const WfSeg* __restrict__ segs, uint32_t nseg,
-                                                        const uint32_t* __restrict__ ctr, uint32_t coop) {
-    __shared__ uint2 s_stk[WIDE_STACK * (TB / 4)];
-    const uint32_t total = ctr[WF_STOTAL];
-    const uint32_t c = blockIdx.x * (TB / RTX_WAVE) + threadIdx.x / RTX_WAVE;
-    if (c >= total) return;  // whole waves (no block barrier follows)
-    WaveChunks<WF_PAIRS> wc;
-    wc.load(ctr + WF_STAB, nseg, total);
-    uint32_t c0 = 0;
-    const uint32_t sg = __builtin_amdgcn_readfirstlane(wc.find(c, c0));
-    wf_shadow_chunk_w<ORDERED, TB / 4>(segs[sg], c - c0, WideStack<TB / 4>{s_stk + (threadIdx.x >> 2)}, coop,
-                                       threadIdx.x & (RTX_WAVE - 1));
 }
 
 // Between the trace and the in-order shadow launch: the shadow chunk table
@@ -2758,15 +2649,15 @@ __global__ __launch_bounds__(RTX_WF_MAX_SEGS) void k_wf_plan_shadow(const WfSeg*
 
 // Shadow rays, one chunk per wave in launch order (see k_wf_trace_ord).
 template <int VAR, int TB, int SR>
-__global__ __launch_bounds__(TB) void k_wf_shadow_ord(const WfSeg* __restrict__ segs, uint32_t nseg,
+__global__ __launch_bounds__(TB, walk_waves<VAR>()) void k_wf_shadow_ord(const WfSeg* __restrict__ segs, uint32_t nseg,
                                                       const uint32_t* __restrict__ ctr, uint32_t coop,
                                                       uint32_t ordered) {
-    __shared__ uint32_t s_id[SR * TB];
+    __shared__ __align__(16) uint32_t s_id[walk_words<VAR, TB, SR, true>()];
     const uint32_t total = ctr[WF_STOTAL];
     const uint32_t c = blockIdx.x * (TB / RTX_WAVE) + threadIdx.x / RTX_WAVE;
     if (c >= total) return;  // whole waves (no block barrier follows)
     uint32_t s_low[stack_private_words<SR>()];
-    TraversalStack<TB, SR> stk{s_id, threadIdx.x, s_low};
+    WalkStack<VAR, TB, SR, true> stk{s_id, threadIdx.x, s_low};
     WaveChunks<WF_PAIRS> wc;
     wc.load(ctr + WF_STAB, nseg, total);
     uint32_t c0 = 0;
@@ -2807,26 +2698,6 @@ static uint32_t resident_grid(int block, int cus, int share) {
 
 void rtx_wf_trace(const WfSeg* segs, uint32_t nseg, uint32_t* ctr, int var, int tb, int sr, uint32_t coop,
                   uint32_t grain, int sched, uint64_t max_chunks, int cus, int share, hipStream_t st) {
-    if (var == WF_WIDE) {
-        const uint64_t g = (max_chunks + tb / RTX_WAVE - 1) / (tb / RTX_WAVE);
-#define RTX_WF_TRACE_W(B)                                                                                           \
-    do {                                                                                                            \
-        if (sched == 0)                                                                                             \
-            hipLaunchKernelGGL((k_wf_trace_ord_w<B>), dim3((uint32_t)(g ? g : 1)), dim3(B), 0, st, segs, nseg, ctr, \
-                               coop);                                                                               \
-        else                                                                                                        \
-            hipLaunchKernelGGL((k_wf_trace_w<B>), dim3(resident_grid<k_wf_trace_w<B>>(B, cus, share)), dim3(B), 0, \
-                               st, segs, nseg, ctr + WF_Q_TRACE, coop, grain);                                      \
-    } while (0)
-        if (tb == 64)
-            RTX_WF_TRACE_W(64);
-        else if (tb == 256)
-            RTX_WF_TRACE_W(256);
-        else
-            RTX_WF_TRACE_W(128);
-#undef RTX_WF_TRACE_W
-        return;
-    }
     if (sched == 0) {
         const uint64_t g = (max_chunks + tb / RTX_WAVE - 1) / (tb / RTX_WAVE);
 #define RTX_WF_TRACE_ORD(V, B, S)                                                                                \
@@ -2846,34 +2717,8 @@ void rtx_wf_trace(const WfSeg* segs, uint32_t nseg, uint32_t* ctr, int var, int 
 void rtx_wf_shadow(const WfSeg* segs, uint32_t nseg, uint32_t* ctr, int var, int tb, int sr, uint32_t coop,
                    uint32_t grain, int sched, uint64_t max_chunks, int cus, int share, bool ordered,
                    hipStream_t st) {
-    if (sched == 0) hipLaunchKernelGGL(k_wf_plan_shadow, dim3(1), dim3(RTX_WF_MAX_SEGS), 0, st, segs, nseg, ctr);
-    if (var == WF_WIDE) {
-        const uint64_t g = (max_chunks + tb / RTX_WAVE - 1) / (tb / RTX_WAVE);
-#define RTX_WF_SHADOW_W(O, B)                                                                                       \
-    do {                                                                                                            \
-        if (sched == 0)                                                                                             \
-            hipLaunchKernelGGL((k_wf_shadow_ord_w<O, B>), dim3((uint32_t)(g ? g : 1)), dim3(B), 0, st, segs, nseg,  \
-                               ctr, coop);                                                                          \
-        else                                                                                                        \
-            hipLaunchKernelGGL((k_wf_shadow_w<O, B>), dim3(resident_grid<k_wf_shadow_w<O, B>>(B, cus, share)),     \
-                               dim3(B), 0, st, segs, nseg, ctr + WF_Q_SHADOW, coop, grain);                         \
-    } while (0)
-#define RTX_WF_SHADOW_WB(B)                                       \
-    do {                                                          \
-        if (ordered) RTX_WF_SHADOW_W(true, B);                    \
-        else RTX_WF_SHADOW_W(false, B);                           \
-    } while (0)
-        if (tb == 64)
-            RTX_WF_SHADOW_WB(64);
-        else if (tb == 256)
-            RTX_WF_SHADOW_WB(256);
-        else
-            RTX_WF_SHADOW_WB(128);
-#undef RTX_WF_SHADOW_WB
-#undef RTX_WF_SHADOW_W
-        return;
-    }
     if (sched == 0) {
+        hipLaunchKernelGGL(k_wf_plan_shadow, dim3(1), dim3(RTX_WF_MAX_SEGS), 0, st, segs, nseg, ctr);
         const uint64_t g = (max_chunks + tb / RTX_WAVE - 1) / (tb / RTX_WAVE);
 #define RTX_WF_SHADOW_ORD(V, B, S)                                                                                \
     hipLaunchKernelGGL((k_wf_shadow_ord<V, B, S>), dim3((uint32_t)(g ? g : 1)), dim3(B), 0, st, segs, nseg, ctr, \
@@ -3058,22 +2903,19 @@ int32_t rtx_raygen_primary(rtx_rays* rays, const rtx_camera* cam, int32_t width,
 // ends a ray at a pop with MAX_LEVELS entries; that count can only reach
 // MAX_LEVELS in trees of 32 levels, which therefore use the single-node form.
 static int traversal_variant(const rtx_scene* s, const SceneView& sv) {
-    const int var = (int)s->ctx->tune.trace_variant;
+    int var = (int)s->ctx->tune.trace_variant;
     // the stackless form needs the parents of the nodes it reads (a render
     // copy of the pipelined frame holds none): the single-node form instead
-    if (var == 4 && !sv.parent) return 1;
+    if (var == 4 && !sv.parent) var = 1;
     const int depth = s->ext ? s->ext->depth : s->depth;
-    return (var == 2 && depth >= STACK) ? 1 : var;
+    if (var == 2 && depth >= STACK) return 1;
+    return var == 1 && sv.wide && s->T <= WIDE_MAX_TRIS ? WIDE_GROUP : var;
 }
 
-// Whether the tree has wide records.
-static bool wide_walk(const rtx_scene* s, const SceneView& sv) { return sv.wide && s->T <= WIDE_MAX_TRIS; }
-
-// Four lanes per item, up to 64 groups per CU (then grid-stride).
-static uint32_t wide_grid(rtx_ctx* c, uint64_t count, uint64_t cap, int TB) {
+// Grid of a scene walk: four lanes per item for WIDE_GROUP.
+static uint32_t walk_grid(rtx_ctx* c, int var, uint64_t count, uint64_t cap, int TB) {
     const uint64_t n = count == RTX_DEVICE_COUNT ? cap : count;
-    const uint64_t g = (4 * n + TB - 1) / TB, gmax = (uint64_t)c->cus * 64;
-    return (uint32_t)(g > gmax ? gmax : (g ? g : 1));
+    return trace_grid(c, var == WIDE_GROUP ? 4 * n : n, 0, TB);
 }
 
 // Iteration bound of the stackless walk: a tree of N <= 2T - 1 nodes allows
@@ -3093,27 +2935,6 @@ int32_t rtx_trace(rtx_scene* s, rtx_rays* rays, rtx_hits* hits, uint64_t count, 
     ProfScope ps(s->ctx, st, "trace");
     const SceneView sv = scene_view(s);
     const int var = traversal_variant(s, sv), tb = (int)s->ctx->tune.trace_block;
-    if (var == 1 && wide_walk(s, sv)) {
-        const TraceIo io{sv.node, sv.delta, sv.wide, sv.tri, sv.nrm, s->uv.as<float2>(), rays->ori4.as<float4>(),
-                         rays->dir4.as<float4>(), hits->flags.as<uint32_t>(), hits->t.as<float>(),
-                         hits->id.as<int32_t>(), hits->bary.as<float2>(), hits->n4.as<float4>(),
-                         hits->p4.as<float4>(), hits->uv2.as<float2>(), hits->list.as<uint32_t>(),
-                         hits->list_count.as<uint32_t>()};
-#define RTX_TRACE_W(B)                                                                                          \
-    hipLaunchKernelGGL((k_trace_w<B>), dim3(wide_grid(s->ctx, count, rays->cap, B)), dim3(B), 0, st, io,       \
-                       rays->count.as<uint32_t>(), count, rtx_wide_coop(s->ctx))
-        if (tb == 64)
-            RTX_TRACE_W(64);
-        else if (tb == 256)
-            RTX_TRACE_W(256);
-        else
-            RTX_TRACE_W(128);
-#undef RTX_TRACE_W
-        RTX_CHECK_HIP(hipGetLastError());
-        hits->list_valid = true;
-        hits->list_for = count;
-        return RTX_OK;
-    }
     if (var == 3) {
 #define RTX_TRACE_P(B)                                                                                              \
     hipLaunchKernelGGL((k_trace_p<B>), dim3(persist_grid(s->ctx, count, rays->cap, B)), dim3(B), 0, st,            \
@@ -3136,13 +2957,14 @@ int32_t rtx_trace(rtx_scene* s, rtx_rays* rays, rtx_hits* hits, uint64_t count, 
         return RTX_OK;
     }
 #define RTX_TRACE_LAUNCH(V, B, S)                                                                                    \
-    hipLaunchKernelGGL((k_trace<V, B, S>), dim3(trace_grid(s->ctx, count, rays->cap, B)), dim3(B), 0, st,              \
+    hipLaunchKernelGGL((k_trace<V, B, S>), dim3(walk_grid(s->ctx, V, count, rays->cap, B)), dim3(B), 0, st,            \
                        sv.node, sv.delta, sv.tri, sv.nrm,                                                 \
                        s->uv.as<float2>(), rays->ori4.as<float4>(), rays->dir4.as<float4>(),                        \
                        rays->count.as<uint32_t>(), count, hits->flags.as<uint32_t>(), hits->t.as<float>(),          \
                        hits->id.as<int32_t>(), hits->bary.as<float2>(), hits->n4.as<float4>(), hits->p4.as<float4>(), \
                        hits->uv2.as<float2>(), hits->list.as<uint32_t>(), hits->list_count.as<uint32_t>(),           \
-                       (uint32_t)s->ctx->tune.xcds, coop_threshold(s->ctx), sv.parent, stackless_bound(s))
+                       (uint32_t)s->ctx->tune.xcds, var == WIDE_GROUP ? rtx_wide_coop(s->ctx) : coop_threshold(s->ctx), sv.parent,     \
+                       stackless_bound(s), sv.wide)
     RTX_DISPATCH_STACK_NS(RTX_TRACE_LAUNCH, var, tb, (int)s->ctx->tune.stack_lds);
 #undef RTX_TRACE_LAUNCH
     RTX_CHECK_HIP(hipGetLastError());
@@ -3192,21 +3014,6 @@ int32_t rtx_trace_shadow_multi(rtx_scene* s, rtx_rays* const* rays, rtx_hits* co
     // (the stackless walk has none)
     const int depth = s->ext ? s->ext->depth : s->depth;
     const uint32_t ordered = (s->ctx->tune.shadow_order != 0 || (depth >= STACK && var != 4)) ? 1u : 0u;
-    if (var == 1 && wide_walk(s, sv)) {
-#define RTX_SHADOW_W(B)                                                                                        \
-    hipLaunchKernelGGL((ordered ? k_shadow_w<true, B> : k_shadow_w<false, B>), dim3(wide_grid(s->ctx, n, n, B)), \
-                       dim3(B), 0, st, sv.node, sv.delta, sv.wide, sv.tri, s->lights.as<rtx_lights>(), segs, (unsigned long long*)dev_shadow_count,      \
-                       rtx_wide_coop(s->ctx))
-        if (tb == 64)
-            RTX_SHADOW_W(64);
-        else if (tb == 256)
-            RTX_SHADOW_W(256);
-        else
-            RTX_SHADOW_W(128);
-#undef RTX_SHADOW_W
-        RTX_CHECK_HIP(hipGetLastError());
-        return RTX_OK;
-    }
     if (var == 3) {
         // queue counter: word 2 of the first segment's hit-list counters
         uint32_t* queue = hits[0]->list_count.as<uint32_t>() + 2;
@@ -3227,10 +3034,11 @@ int32_t rtx_trace_shadow_multi(rtx_scene* s, rtx_rays* const* rays, rtx_hits* co
         return RTX_OK;
     }
 #define RTX_SHADOW_LAUNCH(V, B, S)                                                                              \
-    hipLaunchKernelGGL((k_shadow<V, B, S>), dim3(trace_grid(s->ctx, n, n, B)), dim3(B), 0, st, sv.node,    \
+    hipLaunchKernelGGL((k_shadow<V, B, S>), dim3(walk_grid(s->ctx, V, n, n, B)), dim3(B), 0, st, sv.node,  \
                        sv.delta, sv.tri, s->lights.as<rtx_lights>(), segs,                                     \
                        (unsigned long long*)dev_shadow_count, (uint32_t)s->ctx->tune.xcds, \
-                       coop_threshold(s->ctx), sv.parent, stackless_bound(s), ordered)
+                       var == WIDE_GROUP ? rtx_wide_coop(s->ctx) : coop_threshold(s->ctx), sv.parent,                   \
+                       stackless_bound(s), ordered, sv.wide)
     RTX_DISPATCH_STACK_NS(RTX_SHADOW_LAUNCH, var, tb, (int)s->ctx->tune.stack_lds);
 #undef RTX_SHADOW_LAUNCH
     RTX_CHECK_HIP(hipGetLastError());

@@ -24,10 +24,10 @@ constexpr uint32_t WIDE_LEAF = 0x80000000u, WIDE_DEEP = 0x10000000u, WIDE_LOW = 
 // Most triangles of a tree with wide records (27-bit references; record
 // offsets in 32 bits).
 constexpr uint32_t WIDE_MAX_TRIS = 1u << 25;
-// Stack entries per ray: a step replaces one entry by at most four, and a
-// walk leaves the wide form below level 30 (WIDE_DEEP), so a ray's path has
-// at most 16 wide levels: 1 + 3 * 16.
-constexpr int WIDE_STACK = 49;
+// Stack entries per ray.  A step replaces one entry by at most four, so 49
+// would hold any walk above level 30; rays that need more than these are
+// walked node by node.  32 leave the LDS of the chip to 7 waves per SIMD.
+constexpr int WIDE_STACK = 32;
 
 __device__ __forceinline__ uint32_t wide_ref(uint32_t n, uint32_t a, uint32_t cnt) {
     if (cnt == 0u) return (a - 1u) >> 1;

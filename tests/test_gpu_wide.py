@@ -127,3 +127,67 @@ def test_wide_walk_leaf_sizes(ctx, copies):
     res = _compare(ctx, s, b, nrm, uv, ori4, dir4, lights)
     assert (res["id"] >= 0).sum() > 500
     s.destroy()
+
+
+def _nested_scene(n=20000, size=0.12):
+    """Triangles of one size around centroids that crowd towards a point: a ray through it
+    passes most boxes of every level."""
+    rng = np.random.default_rng(1)
+    c = 0.5 + 0.5 * rng.random((n, 3)) * 2.0 ** -rng.integers(0, 10, (n, 1))
+    e = rng.normal(size=(n, 3, 3))
+    e = (e - e.mean(1, keepdims=True)) * size
+    pos = (c[:, None] + e).reshape(-1, 3).astype(np.float32)
+    return pos, np.arange(3 * n, dtype=np.uint32).reshape(-1, 3)
+
+
+def _wide_entries(b, o, d):
+    """Most stack entries that the ray's wide walk holds before its first leaf (float64 slabs)."""
+    lo, hi, leaf = b.nodes["lo"][:, :3].astype(np.float64), b.nodes["hi"][:, :3].astype(np.float64), b.nodes["leaf"]
+
+    def near_first(n):
+        a = int(b.nodes["a"][n])
+        return (a, a + 1) if np.dot(d, lo[a + 1] - lo[a]) > 0 else (a + 1, a)
+
+    def passes(n):
+        t = np.array([(lo[n] - o) / d, (hi[n] - o) / d])
+        return max(0.0, t.min(0).max()) <= t.max(0).min()
+
+    stack, most = [0], 1
+    while not leaf[stack[-1]]:
+        slots = [g for k in near_first(stack.pop()) for g in ((k,) if leaf[k] else near_first(k))]
+        stack += [g for g in slots[::-1] if passes(g)]
+        most = max(most, len(stack))
+    return most
+
+
+def test_wide_walk_full_stack(ctx):
+    """Rays that need more entries than a group's stack holds (32) go on node by node: in the
+    scene launches, and in the wavefront frame of the same rays."""
+    import rtx
+    pos, idx = _nested_scene()
+    T = len(idx)
+    nrm = np.tile(np.array([[0, 0, -1]], np.float32), (len(pos), 1))
+    mm = np.zeros(T, np.int32)
+    lights = rtx.make_lights((0.1, 0.1, 0.1), [dict(type=rtx.LIGHT_POINT, pos=(1.5, 1.6, 1.7))])
+    s = load_scene(ctx, pos, idx, nrm, None, mm, mats=rtx.make_materials([(0.8, 0.3, 0.2, 0.5, 0.5, 0.0)]),
+                   lights=lights)
+    s.build(30, 1)
+    b = O.Build(pos, idx, mm, 30, 1)
+    rng = np.random.default_rng(3)
+    d = rng.uniform(0.5, 1.0, (512, 3)).astype(np.float32)
+    at = (0.5 + rng.uniform(-0.01, 0.01, (512, 3))).astype(np.float32)
+    ori4, dir4 = np.zeros((512, 4), np.float32), np.full((512, 4), 1e36, np.float32)
+    ori4[:, :3], dir4[:, :3] = at - d, d
+    need = [_wide_entries(b, ori4[i, :3].astype(float), d[i].astype(float)) for i in range(0, 512, 32)]
+    assert max(need) > 32, need
+    _compare(ctx, s, b, nrm, np.zeros((len(pos), 2), np.float32), ori4, dir4, lights)
+    cam = rtx.camera_set((-0.3, -0.35, -0.4), (0.5, 0.5, 0.5), (0, 1, 0), 0.2, 1.0)
+    R = rtx.Renderer(ctx, 64, 64, 1)
+    st = R.frame(s, cam, rebuild=False)
+    wf = rtx.Wavefront(ctx, arena_bytes=1 << 28, max_frames=1)
+    fid = wf.add(s, cam, 64, 64, 1)
+    wf.run()
+    assert np.array_equal(wf.accum(fid), R.fb.accum()) and wf.stats(fid).shadow_rays == st.shadow_rays
+    wf.destroy()
+    R.destroy()
+    s.destroy()
