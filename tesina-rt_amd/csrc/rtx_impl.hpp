@@ -277,9 +277,12 @@ struct InstRoot {
     const float2* uv;
     uint32_t base;
     uint32_t ntri;
+    const float4* wide;  // wide records; null where the tree has none
+    uint64_t pad;        // the rows of the matrices are read as float4
     float tr[16];
     float tr_inv[16];
 };
+static_assert(sizeof(InstRoot) == 192, "InstRoot rows must be 16-byte aligned");
 
 // World-space box of a root for the lane-roots kernels' culling: the root
 // node's box under tr, inflated at use by k * (2 |o| + s) (k < 0: never

@@ -694,8 +694,9 @@ __device__ bool traverse_any_ns(const float4* __restrict__ node, const float4* _
 // WIDE_DEEP node, below which the reference's stack count can reach
 // MAX_LEVELS, and rays that would overflow the group's stack.
 
-// Value of lane (lane ^ 1), (lane ^ 2) of the group of four, or of its lane 0.
-constexpr int QX1 = 0xB1, QX2 = 0x4E, QFIRST = 0x00;
+// Value of lane (lane ^ 1), (lane ^ 2) of the group of four, or of its lane 0,
+// 1, 2 or 3.
+constexpr int QX1 = 0xB1, QX2 = 0x4E, QFIRST = 0x00, Q1 = 0x55, Q2 = 0xAA, Q3 = 0xFF;
 template <int CTRL>
 __device__ __forceinline__ int quad_i(int x) {
     return __builtin_amdgcn_mov_dpp(x, CTRL, 0xf, 0xf, true);
@@ -730,25 +731,33 @@ __device__ __forceinline__ bool wide_slab(v3 lo, v3 hi, const WideRay& r, float 
     return t0 <= t1;
 }
 
-// LDS of a wave: the rays {o, tMin}{d, tMax}{1/d, t0 of the root} (not for
-// WIDE_GROUP), their results, and the groups' stacks ([entry][group], an entry
-// is a reference and, for closest hits, its t0).
+// How the groups get their walks: RAY_FEED a wave's 64 rays, GROUP_FEED one
+// ray each, ROOT_FEED one ray each through the trees of an instance set.
+enum WideFeed { RAY_FEED, GROUP_FEED, ROOT_FEED };
+
+// LDS of a wave: the rays ({o, tMin}{d, tMax}, RAY_FEED also {1/d, t0 of the
+// root}; GROUP_FEED keeps them in registers), the walks' results, ROOT_FEED's
+// best hit over the roots {t, u, v, id} and its root, and the groups' stacks
+// ([entry][group], an entry is a reference and, for closest hits, its t0).
 constexpr int WIDE_GROUPS = RTX_WAVE / 4;
-template <bool ANY, bool GROUP>
+template <bool ANY, WideFeed FEED>
 struct WideLds {
-    static constexpr int N = GROUP ? WIDE_GROUPS : RTX_WAVE;
-    static constexpr int RAY = GROUP ? 0 : 3 * 4 * N, RES = ANY ? N : 4 * N;
-    static constexpr int WORDS = RAY + RES + WIDE_STACK * WIDE_GROUPS * (ANY ? 1 : 2);
+    static constexpr int N = FEED == RAY_FEED ? RTX_WAVE : WIDE_GROUPS;
+    static constexpr int RAY = (FEED == RAY_FEED ? 3 : FEED == ROOT_FEED ? 2 : 0) * 4 * N, RES = ANY ? N : 4 * N;
+    static constexpr int BEST = FEED == ROOT_FEED && !ANY ? 5 * N : 0;
+    static constexpr int WORDS = RAY + RES + BEST + WIDE_STACK * WIDE_GROUPS * (ANY ? 1 : 2);
     uint32_t* m;
     __device__ __forceinline__ WideLds(uint32_t* lds, uint32_t tid, uint32_t*) : m(lds + (tid / RTX_WAVE) * WORDS) {}
     __device__ __forceinline__ float4* ray(int part) const { return reinterpret_cast<float4*>(m) + part * N; }
     __device__ __forceinline__ float4* res() const { return reinterpret_cast<float4*>(m + RAY); }
     __device__ __forceinline__ uint32_t* hit() const { return m + RAY; }
+    __device__ __forceinline__ float4* best() const { return reinterpret_cast<float4*>(m + RAY + RES); }
+    __device__ __forceinline__ int32_t* best_root() const { return reinterpret_cast<int32_t*>(m + RAY + RES + 4 * N); }
     __device__ __forceinline__ uint2* stack2() const {
-        return reinterpret_cast<uint2*>(m + RAY + RES) + ((threadIdx.x & (RTX_WAVE - 1)) >> 2);
+        return reinterpret_cast<uint2*>(m + RAY + RES + BEST) + ((threadIdx.x & (RTX_WAVE - 1)) >> 2);
     }
     __device__ __forceinline__ uint32_t* stack1() const {
-        return m + RAY + RES + ((threadIdx.x & (RTX_WAVE - 1)) >> 2);
+        return m + RAY + RES + BEST + ((threadIdx.x & (RTX_WAVE - 1)) >> 2);
     }
 };
 
@@ -851,50 +860,87 @@ __device__ __forceinline__ bool exact_walk(const float4* __restrict__ node, cons
 // Results in LDS: closest {t, u, v, id} with id -1 for no hit; any hit 0 or 1;
 // REDO: the ray is left to exact_walk.
 constexpr int32_t REDO = -2;
-// Groups that have to be idle before rays are handed out (a hand-out runs for
-// the idle groups alone): 1, 3 and 16 gave 7.03, 7.51 and 8.46 ms on the batch.
-constexpr uint32_t WIDE_REFILL = 1;
+// One walk of a group: its ray, `level` > 0 while it is under way (the entries
+// on the group's stack), its best distance (ANY: its tMax) and its place among
+// the results.
+struct WideWalk {
+    WideRay r;
+    int level;
+    float bt;
+    uint32_t mine;
+    bool odd;
+};
 
-// Walks the groups' rays, then rays [0, n) of the wave's LDS, all of which meet
-// the root's box; the results are left in LDS.  r, level, bt, mine: the
-// group's ray, 1 where it has one (with the root on its stack), its best
-// distance (ANY: its tMax), and its place among the results.  Leaves are
+// Starts a group's walk at its tree's root.
+template <bool ANY, class Lds>
+__device__ __forceinline__ void wide_start(const Lds& lds, uint32_t root, float t0, WideWalk& w) {
+    if (ANY)
+        lds.stack1()[0] = root;
+    else
+        lds.stack2()[0] = make_uint2(root, __float_as_uint(t0));
+    w.level = 1;
+}
+
+// The feeds: next() gives idle groups their next walk and says whether any
+// group has one; `fresh` is set where walks were started.
+struct GroupFeed {
+    static constexpr bool ROOTS = false;
+    const float4 *node_, *wide_, *tri_;
+    __device__ __forceinline__ const float4* node() const { return node_; }
+    __device__ __forceinline__ const float4* wide() const { return wide_; }
+    __device__ __forceinline__ const float4* tri() const { return tri_; }
+    __device__ __forceinline__ bool next(WideWalk& w, bool&) { return ballot(w.level == 0) != ~0ull; }
+};
+
+// Rays [0, n) of the wave's LDS, all of which meet the root's box.  Handed out
+// as soon as one group is idle: 1, 3 and 16 groups gave 7.03, 7.51 and 8.46 ms
+// on the batch of 12 frames.
+template <bool ANY>
+struct RayFeed {
+    static constexpr bool ROOTS = false;
+    const float4 *node_, *wide_, *tri_;
+    WideLds<ANY, RAY_FEED> lds;
+    uint32_t root, n, at;  // at: the next ray (wave-uniform)
+    __device__ __forceinline__ const float4* node() const { return node_; }
+    __device__ __forceinline__ const float4* wide() const { return wide_; }
+    __device__ __forceinline__ const float4* tri() const { return tri_; }
+    __device__ __forceinline__ bool next(WideWalk& w, bool& fresh) {
+        const uint64_t idle = ballot(w.level == 0);
+        if (at >= n || !idle) return idle != ~0ull;
+        const uint32_t i = at + (lanes_below(idle) >> 2);
+        if (w.level == 0 && i < n) {
+            const float4 a = lds.ray(0)[i], b = lds.ray(1)[i], c = lds.ray(2)[i];
+            w.r = WideRay{xyz(a), xyz(b), xyz(c), a.w};
+            w.bt = b.w;
+            w.odd = wide_odd(w.r.inv);
+            w.mine = i;
+            wide_start<ANY>(lds, root, c.w, w);
+        }
+        at += (uint32_t)__builtin_popcountll(idle) >> 2;
+        fresh = true;
+        return true;
+    }
+};
+
+// Walks what the feed hands out; the results are left in LDS.  Leaves are
 // tested four triangles at a time, one per lane, leaves of at least `coop`
 // triangles by the whole wave.  ANY: stops a ray at its first hit with
 // tMin < t < tMax.
-template <bool ANY, bool ORDERED, bool GROUP>
-__device__ __forceinline__ void wide_walk(const float4* __restrict__ node, const float4* __restrict__ wide,
-                                          const float4* __restrict__ tri, WideLds<ANY, GROUP> lds, uint32_t root,
-                                          uint32_t n, uint32_t coop, WideRay r, int level, float bt, uint32_t mine) {
+template <bool ANY, bool ORDERED, class Feed, class Lds>
+__device__ __forceinline__ void wide_walk(Feed& feed, Lds lds, uint32_t coop, WideWalk w) {
     const uint32_t q = lane_id() & 3u;
     uint2* const stk2 = lds.stack2();
     uint32_t* const stk1 = lds.stack1();
     float4* const res = lds.res();
     uint32_t* const hit = lds.hit();
-    uint32_t next = 0;  // next ray to hand out (wave-uniform)
-    bool odd = wide_odd(r.inv);
-    bool any_odd = ballot(odd && level > 0) != 0ull;  // on any ray of the wave
+    WideRay& r = w.r;
+    int& level = w.level;
+    float& bt = w.bt;
+    bool any_odd = ballot(w.odd && level > 0) != 0ull;  // on any ray of the wave
     for (;;) {
-        const uint64_t idle = ballot(level == 0);
-        if (!GROUP && next < n && (uint32_t)__builtin_popcountll(idle) >= 4u * WIDE_REFILL) {
-            const uint32_t i = next + (lanes_below(idle) >> 2);
-            if (level == 0 && i < n) {
-                const float4 a = lds.ray(0)[i], b = lds.ray(1)[i], c = lds.ray(2)[i];
-                r = WideRay{xyz(a), xyz(b), xyz(c), a.w};
-                bt = b.w;
-                odd = wide_odd(r.inv);
-                mine = i;
-                if (ANY)
-                    stk1[0] = root;
-                else
-                    stk2[0] = make_uint2(root, __float_as_uint(c.w));
-                level = 1;
-            }
-            any_odd = ballot(odd && level > 0) != 0ull;
-            next += (uint32_t)__builtin_popcountll(idle) >> 2;
-        } else if (idle == ~0ull) {
-            break;
-        }
+        bool fresh = false;
+        if (!feed.next(w, fresh)) break;
+        if (fresh) any_odd = ballot(w.odd && level > 0) != 0ull;
         wide_sync();
         uint32_t la = 0, lcnt = 0;
         if (level > 0) {
@@ -905,10 +951,10 @@ __device__ __forceinline__ void wide_walk(const float4* __restrict__ node, const
                 // whichever a group needs
                 const bool leaf = (e.x & WIDE_LEAF) != 0u;
                 uint32_t first = 0, cnt = 0;
-                const char* p = reinterpret_cast<const char*>(wide) + ((e.x << 7) | (q << 5));
+                const char* p = reinterpret_cast<const char*>(feed.wide()) + ((e.x << 7) | (q << 5));
                 if (leaf) {
-                    wide_leaf(node, e.x, first, cnt);
-                    p = reinterpret_cast<const char*>(tri) + 48 * (size_t)(first + (q < cnt ? q : 0u));
+                    wide_leaf(feed.node(), e.x, first, cnt);
+                    p = reinterpret_cast<const char*>(feed.tri()) + 48 * (size_t)(first + (q < cnt ? q : 0u));
                 }
                 const float4* p4 = reinterpret_cast<const float4*>(p);
                 float4 f0 = p4[0], f1 = p4[1], f2 = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -917,13 +963,13 @@ __device__ __forceinline__ void wide_walk(const float4* __restrict__ node, const
                 // branch, and a wave with both kinds would wait twice
                 __asm__ volatile("" : "+v"(f0.x), "+v"(f0.y), "+v"(f0.z), "+v"(f0.w), "+v"(f1.x), "+v"(f1.y), "+v"(f1.z));
                 if (!leaf) {
-                    const WideStep s = wide_step<ORDERED>(f0, f1, r, any_odd, odd, bt, q);
+                    const WideStep s = wide_step<ORDERED>(f0, f1, r, any_odd, w.odd, bt, q);
                     if ((ORDERED && (e.x & WIDE_DEEP)) || level + s.total > WIDE_STACK) {
                         if (q == 0u) {
                             if (ANY)
-                                hit[mine] = (uint32_t)REDO;
+                                hit[w.mine] = (uint32_t)REDO;
                             else
-                                res[mine].w = __int_as_float(REDO);
+                                res[w.mine].w = __int_as_float(REDO);
                         }
                         level = 0;
                     } else {
@@ -955,15 +1001,15 @@ __device__ __forceinline__ void wide_walk(const float4* __restrict__ node, const
                             const float t = h ? tt : INFINITY;
                             float m = fminf(t, quad_f<QX1>(t));
                             m = fminf(m, quad_f<QX2>(m));
-                            const int w = h && t == m ? id : -1;
-                            int last = max(w, quad_i<QX1>(w));
+                            const int win = h && t == m ? id : -1;
+                            int last = max(win, quad_i<QX1>(win));
                             last = max(last, quad_i<QX2>(last));
                             if (last >= 0) bt = m;
-                            if (last >= 0 && w == last) res[mine] = make_float4(tt, u, v, __int_as_float(id));
+                            if (last >= 0 && win == last) res[w.mine] = make_float4(tt, u, v, __int_as_float(id));
                         }
                         b += 4;
                         if (b >= cnt) break;
-                        const float4* t4 = tri + 3 * (size_t)(first + (b + q < cnt ? b + q : 0u));
+                        const float4* t4 = feed.tri() + 3 * (size_t)(first + (b + q < cnt ? b + q : 0u));
                         f0 = t4[0];
                         f1 = t4[1];
                         f2 = t4[2];
@@ -972,7 +1018,7 @@ __device__ __forceinline__ void wide_walk(const float4* __restrict__ node, const
                         any |= quad_i<QX1>(any);
                         any |= quad_i<QX2>(any);
                         if (any) {
-                            if (q == 0u) hit[mine] = 1u;
+                            if (q == 0u) hit[w.mine] = 1u;
                             level = 0;
                         }
                     }
@@ -985,15 +1031,15 @@ __device__ __forceinline__ void wide_walk(const float4* __restrict__ node, const
             rc.d = r.d;
             rc.tmin = r.tmin;
             if (ANY) {
-                const int h = coop_any(tri, la, q == 0u ? lcnt : 0u, rc, bt, ~0ull) ? 1 : 0;
+                const int h = coop_any<Feed::ROOTS>(feed.tri(), la, q == 0u ? lcnt : 0u, rc, bt, ~0ull) ? 1 : 0;
                 if (quad_i<QFIRST>(h)) {
-                    if (q == 0u) hit[mine] = 1u;
+                    if (q == 0u) hit[w.mine] = 1u;
                     level = 0;
                 }
             } else {
                 Closest c{bt, 0.f, 0.f, -1};
-                coop_closest(tri, la, q == 0u ? lcnt : 0u, rc, c, ~0ull);
-                if (q == 0u && c.id >= 0) res[mine] = make_float4(c.t, c.u, c.v, __int_as_float(c.id));
+                coop_closest<Feed::ROOTS>(feed.tri(), la, q == 0u ? lcnt : 0u, rc, c, ~0ull);
+                if (q == 0u && c.id >= 0) res[w.mine] = make_float4(c.t, c.u, c.v, __int_as_float(c.id));
                 bt = quad_f<QFIRST>(c.t);
             }
         }
@@ -1008,7 +1054,7 @@ __device__ __forceinline__ void wide_walk(const float4* __restrict__ node, const
 template <bool ANY, bool ORDERED>
 __device__ __forceinline__ void wide_rays(const float4* __restrict__ node, const float4* __restrict__ delta,
                                           const float4* __restrict__ wide, const float4* __restrict__ tri, RayC& rc,
-                                          Closest& best, WideLds<ANY, false> lds, uint32_t coop, bool start) {
+                                          Closest& best, WideLds<ANY, RAY_FEED> lds, uint32_t coop, bool start) {
     const float4 n0 = node[0], n1 = node[1];
     const uint32_t root = wide_ref(0u, __float_as_uint(n0.w), __float_as_uint(n1.w));
     uint64_t wm, rm;  // lanes whose ray is walked, and walked node by node
@@ -1033,7 +1079,10 @@ __device__ __forceinline__ void wide_rays(const float4* __restrict__ node, const
     }
     const uint32_t nw = (uint32_t)__builtin_popcountll(wm), n = nw + (uint32_t)__builtin_popcountll(rm);
     wide_sync();
-    if (wm) wide_walk<ANY, ORDERED>(node, wide, tri, lds, root, nw, coop, WideRay{}, 0, 0.f, 0u);
+    if (wm) {
+        RayFeed<ANY> feed{node, wide, tri, lds, root, nw, 0u};
+        wide_walk<ANY, ORDERED>(feed, lds, coop, WideWalk{});
+    }
     // the rays left to the exact walk, by groups
     const uint32_t lane = lane_id();
     const bool left = lane < n && (ANY ? lds.hit()[lane] == (uint32_t)REDO : __float_as_int(lds.res()[lane].w) == REDO);
@@ -1068,7 +1117,7 @@ __device__ __forceinline__ void wide_rays(const float4* __restrict__ node, const
 template <bool ANY, bool ORDERED>
 __device__ __forceinline__ void wide_group(const float4* __restrict__ node, const float4* __restrict__ delta,
                                            const float4* __restrict__ wide, const float4* __restrict__ tri,
-                                           const RayC& rc, Closest& best, WideLds<ANY, true> lds, uint32_t coop,
+                                           const RayC& rc, Closest& best, WideLds<ANY, GROUP_FEED> lds, uint32_t coop,
                                            bool start) {
     const float4 n0 = node[0], n1 = node[1];
     const uint32_t root = wide_ref(0u, __float_as_uint(n0.w), __float_as_uint(n1.w));
@@ -1077,19 +1126,15 @@ __device__ __forceinline__ void wide_group(const float4* __restrict__ node, cons
     float t0;
     // an infinite reciprocal with an infinite (or NaN) tMax: see above
     const bool redo = start && wide_odd(r.inv) && !(best.t < INFINITY);
-    const bool walk = start && !redo && wide_slab(xyz(n0), xyz(n1), r, best.t, t0);
+    const float tmax = best.t;
+    WideWalk w{r, 0, tmax, group, wide_odd(r.inv)};
     if (ANY)
         lds.hit()[group] = redo ? (uint32_t)REDO : 0u;
     else
         lds.res()[group] = make_float4(0.f, 0.f, 0.f, __int_as_float(redo ? REDO : -1));
-    if (walk) {
-        if (ANY)
-            lds.stack1()[0] = root;
-        else
-            lds.stack2()[0] = make_uint2(root, __float_as_uint(t0));
-    }
-    const float tmax = best.t;
-    wide_walk<ANY, ORDERED>(node, wide, tri, lds, root, 0u, coop, r, walk ? 1 : 0, tmax, group);
+    if (start && !redo && wide_slab(xyz(n0), xyz(n1), r, tmax, t0)) wide_start<ANY>(lds, root, t0, w);
+    GroupFeed feed{node, wide, tri};
+    wide_walk<ANY, ORDERED>(feed, lds, coop, w);
     if (ANY) {
         best.id = lds.hit()[group] == 1u ? 0 : -1;
         if (lds.hit()[group] == (uint32_t)REDO) {
@@ -1119,11 +1164,11 @@ constexpr bool is_wide() {
 // VALU issue and fetch latency: 5 and 7 waves gave 5681 and 5013 us on water).
 template <int VAR, int TB, int SR, bool ANY>
 constexpr int walk_words() {
-    return is_wide<VAR>() ? TB / RTX_WAVE * WideLds<ANY, VAR == WIDE_GROUP>::WORDS : (VAR == 4 ? 1 : SR * TB);
+    return is_wide<VAR>() ? TB / RTX_WAVE * WideLds<ANY, VAR == WIDE_GROUP ? GROUP_FEED : RAY_FEED>::WORDS : (VAR == 4 ? 1 : SR * TB);
 }
 template <int VAR, int TB, int SR, bool ANY>
 using WalkStack =
-    typename std::conditional<is_wide<VAR>(), WideLds<ANY, VAR == WIDE_GROUP>, TraversalStack<TB, SR>>::type;
+    typename std::conditional<is_wide<VAR>(), WideLds<ANY, VAR == WIDE_GROUP ? GROUP_FEED : RAY_FEED>, TraversalStack<TB, SR>>::type;
 template <int VAR>
 constexpr int walk_waves() {
     return is_wide<VAR>() ? 7 : 1;
@@ -2025,16 +2070,18 @@ __global__ void k_root_boxes(const InstRoot* __restrict__ roots, int n, RootBox*
 }
 
 // Bit k set: the segment [tmin, tmax] of the ray (o, d) meets root k's
-// widened world box, or the root is never culled.  n <= 64.  The loop is
-// wave-uniform (the boxes are read as scalars).
-__device__ __forceinline__ uint64_t root_candidates(const RootBox* __restrict__ wb, int n, v3 o, v3 d, float tmin,
-                                                    float tmax) {
+// widened world box, or the root is never culled; k = first, first + STEP,
+// ... < n <= 64.  With first = 0 and STEP = 1 the loop is wave-uniform (the
+// boxes are read as scalars).
+template <int STEP = 1>
+__device__ __forceinline__ uint64_t root_candidates(const RootBox* __restrict__ wb, int first, int n, v3 o, v3 d,
+                                                    float tmin, float tmax) {
     const float io[3] = {o.x, o.y, o.z}, id[3] = {d.x, d.y, d.z};
     float inv[3];
     for (int a = 0; a < 3; ++a) inv[a] = id[a] != 0.f ? 1.f / id[a] : 0.f;
     const float mo = fmaxf(fabsf(o.x), fmaxf(fabsf(o.y), fabsf(o.z)));
     uint64_t m = 0;
-    for (int k = 0; k < n; ++k) {
+    for (int k = first; k < n; k += STEP) {
         const RootBox b = wb[k];
         bool meet = true;
         if (b.k >= 0.f) {
@@ -2122,7 +2169,7 @@ __global__ __launch_bounds__(TB) void k_trace_inst_lr(const InstRoot* __restrict
         };
         const uint64_t live = ballot(true);
         auto walk = [&](int c0, int cn) {
-            uint64_t cand = cull ? root_candidates(wbox + c0, cn, o, d, tmin, tmax) : 0;
+            uint64_t cand = cull ? root_candidates(wbox + c0, 0, cn, o, d, tmin, tmax) : 0;
             i = c0 - 1;
             auto next = [&]() -> bool {
                 if (cull) {
@@ -2268,7 +2315,7 @@ __global__ __launch_bounds__(TB) void k_shadow_inst_lr(const InstRoot* __restric
         bool shadowed = false;
         const uint64_t live = ballot(true);
         auto walk = [&](int c0, int cn) {
-            uint64_t cand = cull ? root_candidates(wbox + c0, cn, p, dir, 0.01f, tmax) : 0;
+            uint64_t cand = cull ? root_candidates(wbox + c0, 0, cn, p, dir, 0.01f, tmax) : 0;
             int k = 0;
             auto next = [&]() -> bool {
                 if (cull) {
@@ -2353,6 +2400,259 @@ __global__ __launch_bounds__(TB) void k_shadow_inst_lr(const InstRoot* __restric
             walk(0, nroots);
         }
         if (valid) set_shadow_bit(&flags[rr], l, shadowed);
+    }
+    if (shadow_count) {
+        if (traced) atomicAdd(&s_cnt, traced);
+        __syncthreads();
+        if (threadIdx.x == 0 && s_cnt) atomicAdd(shadow_count, (unsigned long long)s_cnt);
+    }
+}
+
+// ---- wide walk over the roots: four lanes per ray, as k_trace / k_shadow's
+// WIDE_GROUP.  A group whose walk of a root ends merges it and enters its next
+// candidate root in the same pass as the other groups' steps, so the roots of
+// a wave's 16 rays overlap.  Each root is walked from the ray's own tMax and
+// merged in ascending order with the loops' test, so the records are theirs.
+// Bound by VALU issue and fetch latency like the scene walk; 5 waves per SIMD
+// hold it without scratch (6 spill 15 registers: 1108 against 1091 us).  A
+// 720p frame over 12 objects, two bounces: closest hits 1430 to 537 us, shadow
+// rays 892 to 258 us against one lane per ray (k_trace_inst_lr).  Walks cut
+// at the best hit so far took another 1.5% with a bound that rests on the
+// rounding margin, so they are not.
+
+// Row q of M per lane: (M (v, vw)) on the four lanes of a group, as mul_h.
+__device__ __forceinline__ v3 quad_mul(const float* __restrict__ M, v3 v, float vw, float wmin) {
+    const float4 m = reinterpret_cast<const float4*>(gptr(M))[lane_id() & 3u];
+    float r = ((m.x * v.x + m.y * v.y) + m.z * v.z) + m.w * vw;
+    const float w = quad_f<Q3>(r);
+    if (fabsf(w) > wmin && w != 1.f) r = r / w;
+    return mk3(quad_f<QFIRST>(r), quad_f<Q1>(r), quad_f<Q2>(r));
+}
+
+// root_candidates with the boxes shared out over the group's lanes.
+__device__ __forceinline__ uint64_t quad_candidates(const RootBox* __restrict__ wb, int n, v3 o, v3 d, float tmin,
+                                                    float tmax) {
+    const uint64_t m = root_candidates<4>(wb, (int)(lane_id() & 3u), n, o, d, tmin, tmax);
+    int lo = (int)(uint32_t)m, hi = (int)(uint32_t)(m >> 32);
+    lo |= quad_i<QX1>(lo);
+    lo |= quad_i<QX2>(lo);
+    hi |= quad_i<QX1>(hi);
+    hi |= quad_i<QX2>(hi);
+    return ((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo;
+}
+
+template <bool ANY>
+struct RootFeed {
+    static constexpr bool ROOTS = true;
+    static constexpr float WMIN = ANY ? 0.00001f : 1e-26f;
+    const InstRoot* roots;
+    WideLds<ANY, ROOT_FEED> lds;
+    const float4 *wide_, *tri_;
+    uint64_t cand;  // candidate roots of [c0, c0 + 64) still to walk
+    int c0, i;      // i: the group's current root, -1: none
+    int own;        // ANY: the root to begin with where it is a candidate
+    __device__ __forceinline__ const float4* node() const { return gptr(roots[i].node); }
+    __device__ __forceinline__ const float4* wide() const { return gptr(wide_); }
+    __device__ __forceinline__ const float4* tri() const { return gptr(tri_); }
+    __device__ __forceinline__ bool next(WideWalk& w, bool& fresh) {
+        const bool go = w.level == 0 && (i >= 0 || cand);
+        if (!ballot(go)) return ballot(w.level == 0) != ~0ull;
+        wide_sync();  // results of the groups' lanes
+        if (go) {
+            const uint32_t g = w.mine;
+            const float4 wo = lds.ray(0)[g];
+            if (ANY) {
+                if (lds.hit()[g] != 0u) cand = 0;  // blocked, or left to the exact walk
+            } else if (i >= 0) {
+                const float4 c = lds.res()[g];
+                const int32_t id = __float_as_int(c.w);
+                if (id == REDO) {
+                    lds.best()[g].w = c.w;
+                    cand = 0;
+                } else if (id >= 0) {
+                    const v3 hw = quad_mul(roots[i].tr, w.r.o + w.r.d * c.x, 1.f, WMIN);
+                    const v3 dv = hw - xyz(wo);
+                    const float tw = __builtin_sqrtf(dot(dv, dv));
+                    const float4 b = lds.best()[g];
+                    if (__float_as_int(b.w) < 0 || tw < b.x) {
+                        lds.best()[g] = make_float4(tw, c.y, c.z, c.w);
+                        lds.best_root()[g] = i;
+                    }
+                }
+            }
+            i = -1;
+            if (cand) {
+                const int k = ANY && own >= 0 && ((cand >> own) & 1ull) ? own : __builtin_ctzll(cand);
+                cand &= ~(1ull << k);
+                i = c0 + k;
+                const InstRoot& R = roots[i];
+                const float4* n = gptr(R.node);
+                wide_ = R.wide;
+                tri_ = R.tri;
+                const float4 wd = lds.ray(1)[g], n0 = n[0], n1 = n[1];
+                const v3 o = quad_mul(R.tr_inv, xyz(wo), 1.f, WMIN), d = quad_mul(R.tr_inv, xyz(wd), 0.f, WMIN);
+                const RayC rc = make_ray(o, d, wo.w);
+                w.r = WideRay{o, d, wide_inv(rc), wo.w};
+                w.odd = wide_odd(w.r.inv);
+                w.bt = wd.w;
+                float t0;
+                const bool redo = w.odd && !(w.bt < INFINITY);  // as wide_rays
+                if (!ANY) lds.res()[g] = make_float4(0.f, 0.f, 0.f, __int_as_float(redo ? REDO : -1));
+                if (ANY && redo) lds.hit()[g] = (uint32_t)REDO;
+                if (!redo && wide_slab(xyz(n0), xyz(n1), w.r, w.bt, t0))
+                    wide_start<ANY>(lds, wide_ref(0u, __float_as_uint(n0.w), __float_as_uint(n1.w)), t0, w);
+            }
+        }
+        fresh = true;
+        return true;
+    }
+};
+
+// The group's ray over every root, node by node (rays the wide walk leaves).
+template <bool ANY>
+__device__ __forceinline__ void exact_roots(const InstRoot* __restrict__ roots, int nroots, const RootBox* __restrict__ wbox,
+                                         WideLds<ANY, ROOT_FEED> lds, uint32_t g) {
+    const float4 wo = lds.ray(0)[g], wd = lds.ray(1)[g];
+    float4 best = make_float4(0.f, 0.f, 0.f, __int_as_float(-1));
+    int broot = 0;
+    bool found = false;
+    for (int i = 0; i < nroots && !found; ++i) {
+        if (!root_candidates<1>(wbox + i, 0, 1, xyz(wo), xyz(wd), wo.w, wd.w)) continue;
+        const InstRoot& R = roots[i];
+        const v3 o = quad_mul(R.tr_inv, xyz(wo), 1.f, RootFeed<ANY>::WMIN);
+        const v3 d = quad_mul(R.tr_inv, xyz(wd), 0.f, RootFeed<ANY>::WMIN);
+        Closest c{wd.w, 0.f, 0.f, -1};
+        const bool h = exact_walk<ANY>(gptr(R.node), gptr(R.delta), gptr(R.tri), o, d, wo.w, c, lds.stack1());
+        if (ANY) {
+            found = h;
+        } else if (c.id >= 0) {
+            const v3 dv = quad_mul(R.tr, o + d * c.t, 1.f, RootFeed<ANY>::WMIN) - xyz(wo);
+            const float tw = __builtin_sqrtf(dot(dv, dv));
+            if (__float_as_int(best.w) < 0 || tw < best.x) {
+                best = make_float4(tw, c.u, c.v, __int_as_float(c.id));
+                broot = i;
+            }
+        }
+    }
+    if (ANY) {
+        lds.hit()[g] = found ? 1u : 0u;
+    } else {
+        lds.best()[g] = best;
+        lds.best_root()[g] = broot;
+    }
+}
+
+// The wave's 16 rays (in LDS) over the roots; the groups' results in LDS
+// (best(), best_root(); ANY: hit()).
+template <bool ANY, bool ORDERED>
+__device__ __forceinline__ void wide_roots(const InstRoot* __restrict__ roots, int nroots,
+                                           const RootBox* __restrict__ wbox, WideLds<ANY, ROOT_FEED> lds,
+                                           uint32_t coop, bool start, v3 o, v3 d, float tmin, float tmax, int own) {
+    const uint32_t g = lane_id() >> 2;
+    lds.ray(0)[g] = make_float4(o.x, o.y, o.z, tmin);
+    lds.ray(1)[g] = make_float4(d.x, d.y, d.z, tmax);
+    if (ANY) {
+        lds.hit()[g] = 0u;
+    } else {
+        lds.best()[g] = make_float4(0.f, 0.f, 0.f, __int_as_float(-1));
+        lds.best_root()[g] = 0;
+    }
+    for (int c0 = 0; c0 < nroots; c0 += 64) {  // wave-uniform
+        const int cn = nroots - c0 < 64 ? nroots - c0 : 64;
+        RootFeed<ANY> feed{roots, lds, nullptr, nullptr, 0ull, c0, -1, -1};
+        wide_sync();
+        const bool on = start && (ANY ? lds.hit()[g] == 0u : __float_as_int(lds.best()[g].w) != REDO);
+        if (on) {
+            const float4 wo = lds.ray(0)[g], wd = lds.ray(1)[g];
+            feed.cand = quad_candidates(wbox + c0, cn, xyz(wo), xyz(wd), wo.w, wd.w);
+            feed.own = own >= c0 && own < c0 + cn ? own - c0 : -1;
+        }
+        wide_walk<ANY, ORDERED>(feed, lds, coop, WideWalk{WideRay{}, 0, 0.f, g, false});
+    }
+    wide_sync();
+    if (start && (ANY ? lds.hit()[g] == (uint32_t)REDO : __float_as_int(lds.best()[g].w) == REDO))
+        exact_roots<ANY>(roots, nroots, wbox, lds, g);
+    wide_sync();
+}
+
+template <int TB>
+__global__ __launch_bounds__(TB, 5) void k_trace_inst_w(
+    const InstRoot* __restrict__ roots, int nroots, const float4* __restrict__ ori4, const float4* __restrict__ dir4,
+    const uint32_t* __restrict__ dcount, uint64_t hcount, uint32_t* __restrict__ flags, float* __restrict__ tout,
+    int32_t* __restrict__ idout, float2* __restrict__ bary, float4* __restrict__ n4, float4* __restrict__ p4,
+    float2* __restrict__ uv2, uint32_t* __restrict__ hit_list, uint32_t* __restrict__ hit_count,
+    uint32_t* __restrict__ hit_root, uint32_t coop, const RootBox* __restrict__ wbox, uint32_t xcds) {
+    __shared__ __align__(16) uint32_t s_w[TB / RTX_WAVE * WideLds<false, ROOT_FEED>::WORDS];
+    const WideLds<false, ROOT_FEED> lds{s_w, threadIdx.x, nullptr};
+    const XcdSpan sp = xcd_span(ray_count(dcount, hcount), xcds, TB / 4);
+    for (uint64_t base = sp.begin; base < sp.end; base += sp.stride) {
+        const uint64_t rr = base + threadIdx.x / 4;
+        const bool active = rr < sp.end;
+        v3 o = mk3(0.f, 0.f, 0.f), d = o;
+        float tmin = 0.f, tmax = 0.f;
+        if (active) {
+            const float4 o4 = ori4[rr], d4 = dir4[rr];
+            o = xyz(o4);
+            d = xyz(d4);
+            tmin = o4.w;
+            tmax = d4.w;
+        }
+        wide_roots<false, true>(roots, nroots, wbox, lds, coop, active, o, d, tmin, tmax, -1);
+        const uint32_t g = lane_id() >> 2;
+        const float4 wo = lds.ray(0)[g], wd = lds.ray(1)[g], b = lds.best()[g];
+        inst_record(roots, rr, active && threadIdx.x % 4 == 0, xyz(wo), xyz(wd), b.x, b.y, b.z, __float_as_int(b.w),
+                    lds.best_root()[g], flags, tout, idout, bary, n4, p4, uv2, hit_list, hit_count, hit_root);
+        wide_sync();
+    }
+}
+
+template <bool ORDERED, int TB>
+__global__ __launch_bounds__(TB, 5) void k_shadow_inst_w(
+    const InstRoot* __restrict__ roots, int nroots, const rtx_lights lights, const uint32_t* __restrict__ list,
+    const uint32_t* __restrict__ list_count, uint32_t* __restrict__ flags, const float4* __restrict__ p4,
+    const uint32_t* __restrict__ hit_root, unsigned long long* shadow_count, uint32_t coop,
+    const RootBox* __restrict__ wbox, uint32_t xcds) {
+    __shared__ __align__(16) uint32_t s_w[TB / RTX_WAVE * WideLds<true, ROOT_FEED>::WORDS];
+    __shared__ uint32_t s_cnt;
+    const WideLds<true, ROOT_FEED> lds{s_w, threadIdx.x, nullptr};
+    if (threadIdx.x == 0) s_cnt = 0;
+    __syncthreads();
+    const int nl = lights.count;
+    const uint64_t nh = *list_count;
+    uint32_t traced = 0;
+    const XcdSpan sp = xcd_span(nh * (uint64_t)nl, xcds, TB / 4);
+    for (uint64_t base = sp.begin; base < sp.end; base += sp.stride) {
+        const uint64_t it = base + threadIdx.x / 4;
+        const bool valid = it < sp.end;
+        uint32_t rr = 0;
+        int l = 0, own = -1;
+        v3 p = mk3(0.f, 0.f, 0.f), dir = p;
+        float tmax = 1e37f;
+        bool trace = false;
+        if (valid) {
+            rr = list[it % nh];  // light-major: neighbouring items are one light's rays
+            l = (int)(it / nh);
+            const rtx_light& L = lights.l[l];
+            p = xyz(p4[rr]);
+            trace = true;
+            if (L.type == RTX_LIGHT_DIR) {
+                dir = -mk3(L.dir[0], L.dir[1], L.dir[2]);
+            } else if (L.type == RTX_LIGHT_SPOT) {
+                dir = normalize(mk3(L.pos[0], L.pos[1], L.pos[2]) - p);
+                if (dot(dir, mk3(L.dir[0], L.dir[1], L.dir[2])) < L.angle) trace = false;
+            } else if (L.type == RTX_LIGHT_POINT) {
+                const v3 toL = mk3(L.pos[0], L.pos[1], L.pos[2]) - p;
+                tmax = __builtin_sqrtf(dot(toL, toL));
+                dir = normalize(toL);
+            } else {
+                trace = false;
+            }
+            if (trace && threadIdx.x % 4 == 0) ++traced;
+            if (trace && hit_root) own = (int)(hit_root[rr] % (uint32_t)nroots);
+        }
+        wide_roots<true, ORDERED>(roots, nroots, wbox, lds, coop, trace, p, dir, 0.01f, tmax, own);
+        if (valid && threadIdx.x % 4 == 0) set_shadow_bit(&flags[rr], l, lds.hit()[lane_id() >> 2] == 1u);
+        wide_sync();
     }
     if (shadow_count) {
         if (traced) atomicAdd(&s_cnt, traced);
@@ -3124,7 +3424,6 @@ int32_t rtx_trace_shadow_with(rtx_scene* s, rtx_bvh* b, rtx_rays* rays, rtx_hits
 }
 
 // ---------------------------------------------------------- instances --
-static_assert(sizeof(InstRoot) == 176, "InstRoot layout");
 static_assert(sizeof(RootChunk) + 16 <= 4096, "root chunk exceeds the kernel argument space");
 
 int32_t rtx_instances_create(rtx_ctx* ctx, rtx_scene* const* scenes, const float* tr, const float* tr_inv, int32_t n,
@@ -3261,7 +3560,7 @@ static int32_t refresh_roots(rtx_instances* in, hipStream_t st, int* var) {
     int32_t e = instance_bases(in, base);
     if (e) return e;
     in->table.resize(in->n);
-    bool deep = false;
+    bool deep = false, wide = true;
     for (int i = 0; i < in->n; ++i) {
         rtx_scene* s = in->scene[i];
         RTX_REQUIRE(s->built, RTX_ESTATE, "rtx_trace_instances: an instance's scene has no BVH");
@@ -3270,6 +3569,8 @@ static int32_t refresh_roots(rtx_instances* in, hipStream_t st, int* var) {
         R.node = sv.node;
         R.delta = sv.delta;
         R.tri = sv.tri;
+        R.wide = s->T <= WIDE_MAX_TRIS ? sv.wide : nullptr;
+        wide = wide && R.wide;
         R.nrm = sv.nrm;
         R.uv = s->uv.as<float2>();
         R.base = base[i];
@@ -3279,11 +3580,12 @@ static int32_t refresh_roots(rtx_instances* in, hipStream_t st, int* var) {
         deep = deep || s->depth >= STACK;
     }
     in->deep = deep;
+    // the default with culling: the wide walk where every tree has wide records;
     // the sibling-pair form cannot follow the MAX_LEVELS rule (32-level
     // trees) and the persistent form has no multi-root kernel: both use the
     // single-node form with its early delta load
     const int v = (int)in->ctx->tune.trace_variant;
-    *var = (v == 2 && !deep) ? 2 : (v == 0 ? 0 : 1);
+    *var = v == 2 && !deep ? 2 : v == 0 ? 0 : v == 1 && wide && in->ctx->tune.inst_lane_roots == 2 ? WIDE_GROUP : 1;
     if (in->shipped.size() != in->table.size()) in->shipped.assign(in->table.size(), InstRoot{});
     const bool fresh = in->shipped.empty() || in->shipped[0].node == nullptr;
     for (int c0 = 0; c0 < in->n; c0 += ROOT_CHUNK) {
@@ -3330,6 +3632,7 @@ int32_t rtx_trace_instances(rtx_instances* in, rtx_rays* rays, rtx_hits* hits, u
     ProfScope ps(in->ctx, st, "trace_instances");
     const int tb = (int)in->ctx->tune.trace_block;
     const bool lane_roots = var != 2 && in->ctx->tune.inst_lane_roots != 0;
+    const uint32_t coop = var == WIDE_GROUP ? rtx_wide_coop(in->ctx) : coop_threshold(in->ctx);
 #define RTX_TRACE_INST(V, B)                                                                                        \
     do {                                                                                                        \
         if (lane_roots) {                                                                                           \
@@ -3346,10 +3649,20 @@ int32_t rtx_trace_instances(rtx_instances* in, rtx_rays* rays, rtx_hits* hits, u
     in->roots.as<InstRoot>(), in->n, rays->ori4.as<float4>(), rays->dir4.as<float4>(), rays->count.as<uint32_t>(), \
         count, hits->flags.as<uint32_t>(), hits->t.as<float>(), hits->id.as<int32_t>(), hits->bary.as<float2>(),    \
         hits->n4.as<float4>(), hits->p4.as<float4>(), hits->uv2.as<float2>(), hits->list.as<uint32_t>(),            \
-        hits->list_count.as<uint32_t>(), in->hit_root.as<uint32_t>(), coop_threshold(in->ctx)
+        hits->list_count.as<uint32_t>(), in->hit_root.as<uint32_t>(), coop
     const RootBox* boxes = root_boxes(in, lane_roots, st);
     const bool chunks = boxes != nullptr && in->n > 64;  // culling over chunks of 64 roots
-    RTX_DISPATCH_TRAVERSAL(RTX_TRACE_INST, var, tb);
+#define RTX_TRACE_INST_W(B)                                                                                        \
+    hipLaunchKernelGGL((k_trace_inst_w<B>), dim3(walk_grid(in->ctx, var, count, rays->cap, B)), dim3(B), 0, st,    \
+                       TRACE_INST_ARGS, boxes, (uint32_t)in->ctx->tune.xcds)
+    if (var == WIDE_GROUP) {
+        if (tb == 64) RTX_TRACE_INST_W(64);
+        else if (tb == 256) RTX_TRACE_INST_W(256);
+        else RTX_TRACE_INST_W(128);
+    } else {
+        RTX_DISPATCH_TRAVERSAL(RTX_TRACE_INST, var, tb);
+    }
+#undef RTX_TRACE_INST_W
 #undef TRACE_INST_ARGS
 #undef RTX_TRACE_INST
     RTX_CHECK_HIP(hipGetLastError());
@@ -3380,6 +3693,7 @@ int32_t rtx_trace_shadow_instances_impl(rtx_instances* in, rtx_rays* rays, rtx_h
     const uint32_t* order = in->hit_root.bytes >= hits->cap * 4 ? in->hit_root.as<uint32_t>() : nullptr;
     const int tb = (int)in->ctx->tune.trace_block;
     const bool lane_roots = var != 2 && in->ctx->tune.inst_lane_roots != 0;
+    const uint32_t coop = var == WIDE_GROUP ? rtx_wide_coop(in->ctx) : coop_threshold(in->ctx);
 #define RTX_SHADOW_INST(V, B)                                                                                       \
     do {                                                                                                        \
         if (lane_roots) {                                                                                           \
@@ -3395,13 +3709,24 @@ int32_t rtx_trace_shadow_instances_impl(rtx_instances* in, rtx_rays* rays, rtx_h
 #define SHADOW_INST_ARGS                                                                                            \
     in->roots.as<InstRoot>(), in->n, in->lights, hits->list.as<uint32_t>(), hits->list_count.as<uint32_t>(),        \
         hits->flags.as<uint32_t>(), hits->p4.as<float4>(), order, (unsigned long long*)dev_shadow_count,            \
-        coop_threshold(in->ctx)
+        coop
     const RootBox* boxes = root_boxes(in, lane_roots, st);
     const bool chunks = boxes != nullptr && in->n > 64;  // culling over chunks of 64 roots
     // shadow rays in index order unless a root's tree has 32 levels (an OR
     // over the roots of order-free any-hit walks)
     const uint32_t ordered = (in->ctx->tune.shadow_order != 0 || in->deep) ? 1u : 0u;
-    RTX_DISPATCH_TRAVERSAL(RTX_SHADOW_INST, var, tb);
+#define RTX_SHADOW_INST_W(B)                                                                                       \
+    hipLaunchKernelGGL((ordered ? k_shadow_inst_w<true, B> : k_shadow_inst_w<false, B>),                           \
+                       dim3(walk_grid(in->ctx, var, items, items, B)), dim3(B), 0, st, SHADOW_INST_ARGS, boxes,     \
+                       (uint32_t)in->ctx->tune.xcds)
+    if (var == WIDE_GROUP) {
+        if (tb == 64) RTX_SHADOW_INST_W(64);
+        else if (tb == 256) RTX_SHADOW_INST_W(256);
+        else RTX_SHADOW_INST_W(128);
+    } else {
+        RTX_DISPATCH_TRAVERSAL(RTX_SHADOW_INST, var, tb);
+    }
+#undef RTX_SHADOW_INST_W
 #undef SHADOW_INST_ARGS
 #undef RTX_SHADOW_INST
     RTX_CHECK_HIP(hipGetLastError());

@@ -191,3 +191,47 @@ def test_wide_walk_full_stack(ctx):
     wf.destroy()
     R.destroy()
     s.destroy()
+
+
+def test_instances_left_to_the_exact_walk(ctx):
+    """Rays that leave the wide walk of an instance (a full stack, an infinite reciprocal with an
+    infinite tMax) and leaves of all sizes, over sets of one and two chunks of roots: the records of
+    the loop that walks a ray per lane over the same candidate roots."""
+    import rtx
+    pos, idx = _nested_scene()
+    a = load_scene(ctx, pos, idx)
+    pos, idx, nrm, uv, mm = random_scene(5, 300)
+    pos = np.round(pos).astype(np.float32) + np.float32(0.0)
+    idx = np.repeat(idx, np.arange(300) % 40 + 1, axis=0)
+    b = load_scene(ctx, pos, idx, nrm, uv, np.zeros(len(idx), np.int32))
+    for s in (a, b):
+        s.build(30, 1)
+    rng = np.random.default_rng(4)
+    ori4, dir4 = _odd_rays(rng, pos, 2048)
+    d = rng.uniform(0.5, 1.0, (512, 3)).astype(np.float32)
+    ori4[::4, :3], dir4[::4, :3] = 0.5 + rng.uniform(-0.01, 0.01, (512, 3)) - d, d
+    ori4[::4, 3], dir4[::4, 3] = 0.0, 1e36
+    r, h = rtx.Rays(ctx, 2048), rtx.Hits(ctx, 2048)
+    r.write(ori4, dir4)
+    old = ctx.tuned("trace_variant")
+    for n in (3, 70):
+        tr = np.tile(np.eye(4, dtype=np.float32), (n, 1, 1))
+        tr[1:, :3, 3] = rng.integers(-20, 20, (n - 1, 3))
+        tr[2::3, :3, :3] *= 2.0
+        inst = rtx.Instances(ctx, [(a, b)[i % 2] for i in range(n)], tr, np.linalg.inv(tr).astype(np.float32))
+        inst.set_lights(_lights())
+        want = None
+        for form in (0, 1):
+            ctx.tune("trace_variant", form)
+            inst.trace(r, h, 2048)
+            inst.trace_shadow(r, h, 2048)
+            got = h.read(2048)
+            want = want or got
+            for k in want:
+                if k != "list":
+                    assert np.array_equal(got[k], want[k], equal_nan=got[k].dtype.kind == "f"), (n, form, k)
+        assert (want["id"] >= 0).sum() > 300
+        inst.destroy()
+    ctx.tune("trace_variant", old)
+    for x in (r, h, a, b):
+        x.destroy()
