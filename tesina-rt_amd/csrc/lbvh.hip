@@ -45,7 +45,8 @@ __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t x, uint32_t lane) {
     return x;
 }
 
-// Exclusive scan of one value per thread over a 256-thread block.
+// Exclusive scan of one value per thread over a block of NT threads.
+template <int NT = BS>
 __device__ __forceinline__ uint32_t block_excl_scan(uint32_t x, uint32_t* s_w, uint32_t* total) {
     uint32_t lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     uint32_t inc = wave_incl_scan(x, lane);
@@ -53,7 +54,7 @@ __device__ __forceinline__ uint32_t block_excl_scan(uint32_t x, uint32_t* s_w, u
     __syncthreads();
     uint32_t base = 0, tot = 0;
 #pragma unroll
-    for (int i = 0; i < BS / RTX_WAVE; ++i) {
+    for (int i = 0; i < NT / RTX_WAVE; ++i) {
         uint32_t v = s_w[i];
         base += (i < (int)w) ? v : 0u;
         tot += v;
@@ -227,31 +228,36 @@ __global__ __launch_bounds__(BS) void k_morton(const float4* __restrict__ cen, c
 
 // One stable LSD pass over `bits` <= RB bits at `shift` (onesweep: in-tile
 // rank by wave64 ballot matching, per-digit decoupled look-back across tiles,
-// LDS-staged scatter) over tiles of BS * ITEMS pairs.  Replaces the bitonic
+// LDS-staged scatter) over tiles of NT * ITEMS pairs.  Replaces the bitonic
 // network of src/kernel/bvh-builder-sort.cl:26-232.  RB = 8: 256 digits a
 // pass; RB = 4: 16 digits, twice the passes, longer runs per digit in the
 // scatter (the reference's radix prototype, src/kernel/sort.cl:491-628, uses
 // 4-bit digits).  The look-back word of tile t, digit d is status[t * 2^RB + d].
-template <int RB, int ITEMS>
-__global__ __launch_bounds__(BS) void k_sort_pass(const uint32_t* __restrict__ kin, const uint32_t* __restrict__ vin,
+// A pass over few tiles is bound by one tile's latency (loads, ITEMS rank
+// rounds, scans, look-back), so such tiles are spread over 1024 threads of 4
+// pairs instead of 256 of 16: 13.1 to 9.9 us a pass over 65k pairs, 15.3 to
+// 11.8 over 300k, 20.8 to 17.7 over 1M.  Over 2000 tiles the fewer, larger
+// blocks per CU lose: 70 against 85 us at 8M.
+template <int RB, int ITEMS, int NT>
+__global__ __launch_bounds__(NT) void k_sort_pass(const uint32_t* __restrict__ kin, const uint32_t* __restrict__ vin,
                                                   uint32_t* __restrict__ kout, uint32_t* __restrict__ vout,
                                                   uint32_t n, int shift, int bits, const uint32_t* __restrict__ hist,
                                                   uint32_t* status, uint32_t* ticket) {
-    constexpr int TILE = BS * ITEMS;
+    constexpr int TILE = NT * ITEMS;
     constexpr uint32_t DIG = 1u << RB;
-    static_assert(DIG <= (uint32_t)BS, "one thread per digit");
+    static_assert(DIG <= (uint32_t)NT, "one thread per digit");
     __shared__ uint32_t s_keys[TILE];
     __shared__ uint32_t s_vals[TILE];
-    __shared__ uint32_t s_wcnt[BS / RTX_WAVE][DIG];
+    __shared__ uint32_t s_wcnt[NT / RTX_WAVE][DIG];
     __shared__ uint32_t s_tofs[DIG];
     __shared__ uint32_t s_gofs[DIG];
-    __shared__ uint32_t s_w[BS / RTX_WAVE];
+    __shared__ uint32_t s_w[NT / RTX_WAVE];
     __shared__ uint32_t s_tile;
     const uint32_t tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     if (tid == 0) s_tile = atomicAdd(ticket, 1u);
     if (tid < DIG) {
 #pragma unroll
-        for (int i = 0; i < BS / RTX_WAVE; ++i) s_wcnt[i][tid] = 0;
+        for (int i = 0; i < NT / RTX_WAVE; ++i) s_wcnt[i][tid] = 0;
     }
     __syncthreads();
     const uint32_t tile = s_tile;
@@ -266,6 +272,10 @@ __global__ __launch_bounds__(BS) void k_sort_pass(const uint32_t* __restrict__ k
         k[j] = ok ? kin[e] : 0xffffffffu;
         v[j] = ok ? vin[e] : 0u;
     }
+    // global start of each digit = exclusive scan of the pass histogram
+    uint32_t dummy;
+    const uint32_t hv = tid <= dmask ? hist[tid] : 0u;
+    const uint32_t dbase = block_excl_scan<NT>(hv, s_w, &dummy);
 #pragma unroll
     for (int j = 0; j < ITEMS; ++j) {
         uint32_t e = base + (w * ITEMS + j) * RTX_WAVE + lane;
@@ -290,21 +300,19 @@ __global__ __launch_bounds__(BS) void k_sort_pass(const uint32_t* __restrict__ k
     // per-digit tile totals, wave offsets (exclusive, in wave order)
     uint32_t tot = 0;
     if (tid < DIG) {
-        uint32_t c[BS / RTX_WAVE];
+        uint32_t c[NT / RTX_WAVE];
 #pragma unroll
-        for (int i = 0; i < BS / RTX_WAVE; ++i) c[i] = s_wcnt[i][tid];
+        for (int i = 0; i < NT / RTX_WAVE; ++i) c[i] = s_wcnt[i][tid];
 #pragma unroll
-        for (int i = 0; i < BS / RTX_WAVE; ++i) {
+        for (int i = 0; i < NT / RTX_WAVE; ++i) {
             s_wcnt[i][tid] = tot;
             tot += c[i];
         }
     }
-    uint32_t dummy;
-    uint32_t tofs = block_excl_scan(tot, s_w, &dummy);
+    // successors can go on with this tile's counts before the scan below
+    if (tid <= dmask) st_relaxed(&status[(size_t)tile * DIG + tid], (tile ? RTX_LB_AGG : RTX_LB_INC) | tot);
+    uint32_t tofs = block_excl_scan<NT>(tot, s_w, &dummy);
     if (tid < DIG) s_tofs[tid] = tofs;
-    // global start of each digit = exclusive scan of the pass histogram
-    uint32_t hv = tid <= dmask ? hist[tid] : 0u;
-    uint32_t dbase = block_excl_scan(hv, s_w, &dummy);
     if (tid <= dmask) {
         uint32_t prefix = lookback_thread(status + tid, tile, tot, DIG);
         s_gofs[tid] = dbase + prefix - tofs;  // dest = s_gofs[d] + local position
@@ -323,7 +331,7 @@ __global__ __launch_bounds__(BS) void k_sort_pass(const uint32_t* __restrict__ k
     }
     __syncthreads();
     uint32_t nvalid = n - base < (uint32_t)TILE ? n - base : (uint32_t)TILE;
-    for (uint32_t i = tid; i < nvalid; i += BS) {
+    for (uint32_t i = tid; i < nvalid; i += NT) {
         uint32_t key = s_keys[i];
         uint32_t dst = s_gofs[(key >> shift) & dmask] + i;
         kout[dst] = key;
@@ -1107,17 +1115,21 @@ static bool build_sort_phase(rtx_scene* s, int depth, hipStream_t st, const Buil
         const int bits = depth - shift < rb ? depth - shift : rb;
         uint32_t* const hist = W.sort_hist + ((size_t)pass << rb);
         uint32_t* const status = W.sort_status + ((size_t)pass * sort_tiles << rb);
-#define RTX_SORT_PASS(R, I)                                                                                    \
-    hipLaunchKernelGGL((k_sort_pass<R, I>), dim3(sort_tiles), dim3(BS), 0, st, kin, vin, kout, vout, T, shift, \
+#define RTX_SORT_PASS(R, I, N)                                                                                 \
+    hipLaunchKernelGGL((k_sort_pass<R, I, N>), dim3(sort_tiles), dim3(N), 0, st, kin, vin, kout, vout, T, shift, \
                        bits, hist, status, tickets + TK_SORT + pass)
         if (rb == 4 && items == 32)
-            RTX_SORT_PASS(4, 32);
+            RTX_SORT_PASS(4, 32, BS);
         else if (rb == 4)
-            RTX_SORT_PASS(4, 16);
+            RTX_SORT_PASS(4, 16, BS);
         else if (items == 32)
-            RTX_SORT_PASS(8, 32);
+            RTX_SORT_PASS(8, 32, BS);
+        else if (sort_tiles <= (uint32_t)s->ctx->cus)
+            // the tiles fit on the chip side by side (whole builds of 1.05M / 1.5M / 3M
+            // triangles: 290 / 391 / 699 us so, 302 / 388 / 689 with small blocks)
+            RTX_SORT_PASS(8, 4, 4 * BS);
         else
-            RTX_SORT_PASS(8, 16);
+            RTX_SORT_PASS(8, 16, BS);
 #undef RTX_SORT_PASS
         std::swap(kin, kout);
         std::swap(vin, vout);

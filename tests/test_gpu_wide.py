@@ -235,3 +235,25 @@ def test_instances_left_to_the_exact_walk(ctx):
     ctx.tune("trace_variant", old)
     for x in (r, h, a, b):
         x.destroy()
+
+
+@pytest.mark.parametrize("T", [1, 4095, 4096, 4097, 70001, 1 << 20, (1 << 20) + 1])
+def test_sort_tiles(ctx, T):
+    """Edges of the sort's tiles (4096 pairs) and of the count (a tile per CU) up to which a tile
+    takes 1024 threads: a stable order, the same as over tiles of 8192."""
+    rng = np.random.default_rng(T)
+    pos = rng.uniform(-5, 5, (max(3, T // 3), 3)).astype(np.float32)
+    idx = rng.integers(0, len(pos), (T, 3)).astype(np.uint32)
+    old, got = ctx.tuned("sort_items"), []
+    for items in (32, 16):
+        ctx.tune("sort_items", items)
+        s = load_scene(ctx, pos, idx, None, None, np.zeros(T, np.int32))
+        s.build()
+        got.append((s.codes(), s.perm()))
+        s.destroy()
+    ctx.tune("sort_items", old)
+    codes, perm = got[1]
+    unsorted = np.empty_like(codes)
+    unsorted[perm] = codes
+    assert np.array_equal(np.argsort(unsorted, kind="stable"), perm)
+    assert np.array_equal(got[0][0], codes) and np.array_equal(got[0][1], perm)
