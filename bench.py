@@ -276,7 +276,7 @@ def main():
 
     # the LBVH build's knobs, picked by back-to-back builds of this scene:
     # radix digit width and pairs per thread of the sort, persistent blocks
-    # per CU of the level launches (every setting builds the same tree)
+    # per CU of the pass over the child pairs (every setting builds the same tree)
     build_tune = lbvh_autotune(ctx, s)
     log("LBVH build tuning: " + ", ".join(
         f"bits {t['sort_bits']} items {t['sort_items']} grid {t['build_grid']}: {t['ms_per_build']:.3f} ms"
@@ -1197,7 +1197,7 @@ def bench_instances(ctx, frames: int = 50, reps: int = 3):
                              "loop (0)",
             "mrays_incl_shadow": round((n + shadow_rays) / dt_inst / 1e6, 2),
             "trace_instances_ms": trace_ms, "trace_shadow_instances_ms": shadow_ms,
-            "roofline": {"kernel": "k_trace_inst_lr (closest hit over 16 roots, culled by world boxes)", "bound": "hbm",
+            "roofline": {"kernel": "k_trace_inst_w (closest hit over 16 roots, culled by world boxes)", "bound": "hbm",
                          "achieved": round(48.0 * n / (trace_ms / 1e3) / 1e9, 2) if trace_ms else None,
                          "peak": HBM_PEAK_GBS, "unit": "GB/s",
                          "frac": round(48.0 * n / (trace_ms / 1e3) / 1e9 / HBM_PEAK_GBS, 5) if trace_ms else None,

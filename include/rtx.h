@@ -156,9 +156,11 @@ int32_t rtx_profile_reset(rtx_ctx* ctx);
 uint64_t rtx_mem_in_use(rtx_ctx* ctx);
 /* Tuning knobs, set by the autotuner (no reference counterpart: the
  * reference fixes its work-group sizes per device, src/gpu/function.cpp:322-385):
- *   "trace_variant": 0 single-node traversal, 1 single node with the near-child
- *                    delta loaded early, 2 sibling-pair traversal, 3 persistent
- *                    waves fed from a ray queue (single-node steps);
+ *   "trace_variant": 0 single-node traversal, 1 (default) four lanes per ray over
+ *                    records of four grandchildren, or, for trees without such
+ *                    records (over 2^25 triangles), single node with the
+ *                    near-child delta loaded early, 2 sibling-pair traversal, 3
+ *                    persistent waves fed from a ray queue (single-node steps);
  *   "refill":        variant 3: idle lanes of a wave that trigger a refill
  *                    from the queue (1..64);
  *   "trace_block":   64, 128 or 256 threads per traversal work-group;
@@ -167,12 +169,14 @@ uint64_t rtx_mem_in_use(rtx_ctx* ctx);
  *                    contiguous, screen-coherent chunk of the rays; 1 = plain
  *                    grid order);
  *   "coop_leaf":     leaves of at least this many triangles are tested by
- *                    the whole wave, 64 triangles per round (0 = never);
+ *                    the whole wave, 64 triangles per round (0 = never); the
+ *                    four-lane walk takes four times the value;
  *   "side_stream":   1: a renderer traces each bounce's shadow rays and shades
  *                    it on a second stream while the next bounce is generated
  *                    and traced (frames then capture as forked graphs); 0: all
  *                    stages on the caller's stream (linear graphs).
- *   "inst_lane_roots": instances under the single-node forms (0, 1): 1: each
+ *   "inst_lane_roots": instances under forms 0 and 1 (form 1 walks four lanes
+ *                    per ray only with value 2): 1: each
  *                    lane moves on to its next root as soon as its walk of the
  *                    last one ends, in one loop; 2 (default): the same over
  *                    only the roots whose world-space box (the root box under

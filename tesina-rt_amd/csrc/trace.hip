@@ -11,7 +11,9 @@
 // ids, distances and tie winners are those of the oracle.  The MI355X layout
 // is what differs: 32-byte nodes plus a 16-byte delta fetched only at
 // internal nodes, triangles stored contiguously in leaf order, the stack in
-// LDS ([level][thread], conflict-free), SoA rays and hits.
+// LDS ([level][thread], conflict-free), SoA rays and hits.  The default form
+// walks a ray on four lanes over records of four grandchildren (wide walk,
+// below) and shows why its results are those of the node-by-node forms.
 #include <algorithm>
 #include <atomic>
 #include <cstring>
