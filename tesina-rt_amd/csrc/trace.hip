@@ -2061,8 +2061,14 @@ __global__ __launch_bounds__(TB) void k_shadow_inst(const InstRoot* __restrict__
 // units of 6e-8, times the transforms' condition, times the magnitudes of
 // the origin and of the point, which lies within the box) stays far below
 // it, so a root whose widened box the ray misses holds no hit the walk
-// could find.  Roots under a projective transform (bottom rows other than
-// 0 0 0 1), or with a non-finite box, get k = -1: never culled.
+// could find, provided the walk tests every axis: an axis with |1/d| <= 1e-6
+// in the object's frame is left out (make_ray), and the walk then reaches
+// triangles outside the ray's path, which rounding can make hits of.  Those
+// components are at most |tr_inv| times the ray's largest one, and |tr_inv|
+// at most 1e4 k, so rays with k |d| >= 99 are never culled (at k >= 1 the
+// widened box holds the origin, so unit directions lose nothing by it).
+// Roots under a projective transform (bottom rows other than 0 0 0 1), or
+// with a non-finite box, get k = -1: never culled.
 __global__ void k_root_boxes(const InstRoot* __restrict__ roots, int n, RootBox* __restrict__ out) {
     const int k = (int)(blockIdx.x * blockDim.x + threadIdx.x);
     if (k >= n) return;
@@ -2100,7 +2106,7 @@ __global__ void k_root_boxes(const InstRoot* __restrict__ roots, int n, RootBox*
 }
 
 // Bit k set: the segment [tmin, tmax] of the ray (o, d) meets root k's
-// widened world box, or the root is never culled; k = first, first + STEP,
+// widened world box, or the root is not culled for it; k = first, first + STEP,
 // ... < n <= 64.  With first = 0 and STEP = 1 the loop is wave-uniform (the
 // boxes are read as scalars).
 template <int STEP = 1>
@@ -2110,11 +2116,12 @@ __device__ __forceinline__ uint64_t root_candidates(const RootBox* __restrict__ 
     float inv[3];
     for (int a = 0; a < 3; ++a) inv[a] = id[a] != 0.f ? 1.f / id[a] : 0.f;
     const float mo = fmaxf(fabsf(o.x), fmaxf(fabsf(o.y), fabsf(o.z)));
+    const float md = fmaxf(fabsf(d.x), fmaxf(fabsf(d.y), fabsf(d.z)));
     uint64_t m = 0;
     for (int k = first; k < n; k += STEP) {
         const RootBox b = wb[k];
         bool meet = true;
-        if (b.k >= 0.f) {
+        if (b.k >= 0.f && b.k * md < 99.f) {
             const float g = b.k * (2.f * mo + b.s);
             float t0 = tmin, t1 = tmax;
 #pragma unroll

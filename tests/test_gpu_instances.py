@@ -442,6 +442,54 @@ def test_culling_boundaries(ctx):
         s.destroy()
 
 
+def test_rays_with_skipped_axes(ctx):
+    """Directions of 1e5 to 1e8: bbox_hit leaves out the axes with |1/d| <= 1e-6
+    (src/kernel/trace-bvh.cl:247-273), so the walk reaches triangles whose boxes the
+    ray misses, and rays that start in a triangle's plane and run along it hit such
+    a triangle at t = 0 by rounding.  Root culling must keep the roots that hold
+    those hits: the oracle's records, in every form and schedule."""
+    import rtx
+    g = np.arange(-6, 7)
+    x, y = np.meshgrid(g, g, indexing="ij")
+    pos = np.stack([x, y, -x - y], -1).reshape(-1, 3).astype(np.float32)  # a piece of the plane x + y + z = 0
+    i = np.arange(169).reshape(13, 13)[:-1, :-1].ravel()
+    idx = np.concatenate([np.stack([i, i + 1, i + 13], 1), np.stack([i + 1, i + 14, i + 13], 1)]).astype(np.uint32)
+    meshes = [(pos, np.tile(np.float32([0.0, 1.0, 0.0]), (169, 1)), np.zeros((169, 2), np.float32), idx)]
+    lights = _lights()
+    scs = _load(ctx, meshes, lights)
+    builds = [O.Build(pos, idx, None, 30, 1)]
+    rng = np.random.default_rng(3)
+    n = 4096
+    o4, d4 = np.zeros((n, 4), np.float32), np.full((n, 4), np.inf, np.float32)
+    o4[:, :2] = rng.integers(-40, 41, (n, 2))
+    d = rng.normal(size=(n, 3))
+    d[:, 2] = -d[:, 0] - d[:, 1]
+    d4[:, :3] = d * 10.0 ** rng.uniform(5, 8, (n, 1))
+    o4[:, 2] = -o4[:, 0] - o4[:, 1]
+    r = rtx.Rays(ctx, n)
+    r.write(o4, d4)
+    hb = rtx.Hits(ctx, n)
+    for count in (4, 70):  # one and two chunks of roots
+        insts = []
+        for k in range(count):
+            t = rng.integers(-70, 71, 2)
+            insts.append((0, *xform(np.eye(3), (1.0, 2.0, 0.5)[k % 3], (t[0], t[1], -t[0] - t[1]))))
+        o, _ = _oracle(meshes, builds, insts, lights, o4, d4)
+        missed = np.ones(n, bool)  # rays that miss every instance's box by more than 1
+        for (lo, hi) in _world_boxes(meshes, insts):
+            with np.errstate(all="ignore"):
+                a, b = (lo - 1 - o4[:, :3]) / d4[:, :3], (hi + 1 - o4[:, :3]) / d4[:, :3]
+            missed &= np.maximum(np.minimum(a, b).max(1), 0) > np.maximum(a, b).min(1)
+        assert (missed & (o["id"] >= 0)).sum() > (500 if count == 4 else 5)
+        inst = rtx.Instances(ctx, [scs[0]] * count, [t for _, t, _ in insts], [ti for _, _, ti in insts])
+        inst.set_lights(lights)
+        _check_all_forms(ctx, inst, r, hb, n, o, f"skipped axes, {count} roots")
+        inst.destroy()
+    r.destroy()
+    hb.destroy()
+    scs[0].destroy()
+
+
 def test_many_instances_culled_in_chunks(ctx):
     """100 instances (a 10 x 10 grid of the two meshes under rotations and
     scales): root culling runs over two chunks of roots (64 + 36); closest
