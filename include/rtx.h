@@ -296,7 +296,9 @@ int32_t rtx_lbvh_build(rtx_scene* s, const rtx_lbvh_params* p, void* stream);
 #define RTX_LBVH_NOALLOC_SCRATCH_BYTES 43549184u
 int32_t rtx_lbvh_build_noalloc(rtx_scene* s, const rtx_lbvh_params* p, void* stream);
 /* BVHBuilder::refit_lbvh (src/rt/bvh-builder.cpp:743-850): AABBs from the
- * current (already permuted) vertices, topology kept.  Asynchronous. */
+ * current (already permuted) vertices, topology kept.  Asynchronous.  Uses
+ * the scene's build scratch; allocates it (3 B a triangle) only where the tree
+ * came from rtx_lbvh_build_noalloc and no rtx_lbvh_build got that far. */
 int32_t rtx_lbvh_refit(rtx_scene* s, void* stream);
 /* Node count and per-iteration output counts OC[0..63] (scene.bvh_node_count,
  * bvh_level_node_count; src/rt/bvh-builder.cpp:614-625, 733-736).  Synchronizes. */

@@ -80,13 +80,14 @@ def build(verbose: bool = False) -> Path:
 TOOLS = {"stage_render": ROOT / "tests" / "cpp" / "stage_render.cpp",
          "stage_objects": ROOT / "tests" / "cpp" / "stage_objects.cpp",
          "stage_boat": ROOT / "tests" / "cpp" / "stage_boat.cpp",
-         "stage_tracer": ROOT / "tests" / "cpp" / "stage_tracer.cpp"}
+         "stage_tracer": ROOT / "tests" / "cpp" / "stage_tracer.cpp",
+         "refit_reserve": ROOT / "tests" / "cpp" / "refit_reserve.cpp"}
 BIN = PKG / "bin"
 
 
 def build_tools() -> None:
-    """C++ programs that drive the library through include/rt/stages.hpp
-    (host code only: plain g++ against librtx.so)."""
+    """C++ programs that drive the library through include/rt/stages.hpp or its
+    C ABI (host code only: plain g++ against librtx.so)."""
     BIN.mkdir(exist_ok=True)
     for name, src in TOOLS.items():
         if not src.exists():

@@ -1416,6 +1416,10 @@ int32_t rtx_lbvh_refit(rtx_scene* s, void* stream) {
     RTX_REQUIRE(s->built, RTX_ESTATE, "rtx_lbvh_refit: no BVH built");
     RTX_REQUIRE(!s->sah, RTX_ESTATE, "rtx_lbvh_refit: the tree is an SAH tree (refit follows LBVH levels)");
     hipStream_t st = s->ctx->pick(stream);
+    // held already unless the tree came from rtx_lbvh_build_noalloc after an
+    // rtx_lbvh_build that ran out of memory at its scratch
+    int32_t e = s->b().tree_tiles.reserve(s->ctx, rtx_div_up(s->T, TREE_TILE) * TILE_BYTES);
+    if (e) return e;
     tree_boxes<true>(s, st, scratch_of(s->b()), s->ctx);
     RTX_CHECK_HIP(hipGetLastError());
     return RTX_OK;

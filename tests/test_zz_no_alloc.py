@@ -6,6 +6,9 @@ triangles, so the shared scratch array holds the first call's contents), on
 a chained rebuild, at an odd sort-pass count, and with the size and state
 errors the entry point documents.
 """
+import subprocess
+from pathlib import Path
+
 import numpy as np
 import pytest
 
@@ -126,3 +129,14 @@ def test_noalloc_errors(ctx):
             s.build_noalloc(30, 1)
     finally:
         s.destroy()
+
+
+def test_refit_after_builds_out_of_memory():
+    """tests/cpp/refit_reserve.cpp: every allocation of a growing scene's build refused in turn;
+    where the allocation-free build then accepts the scene, a refit has the scratch it writes."""
+    exe = Path(__file__).resolve().parent.parent / "tesina-rt_amd" / "bin" / "refit_reserve"
+    assert exe.exists(), "refit_reserve not built (run __graft_entry__.build())"
+    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stdout + r.stderr
+    words = r.stdout.splitlines()[-1].split()
+    assert int(words[1]) > 10 and int(words[3]) > 5, r.stdout
