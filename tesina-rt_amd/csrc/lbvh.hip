@@ -34,7 +34,7 @@ constexpr int TK_COUNT = 80;
 
 // Layout of scene->levels (uint32): [d] = first node of level d,
 // [64 + d] = node count of level d, [128] = total node count.
-constexpr int LV_OFF = 0, LV_CNT = 64, LV_TOTAL = 128, LV_WORDS = 192;
+constexpr int LV_OFF = 0, LV_CNT = 64, LV_TOTAL = BuildSet::NODE_COUNT, LV_WORDS = 192;
 
 // ------------------------------------------------------------- helpers --
 __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t x, uint32_t lane) {

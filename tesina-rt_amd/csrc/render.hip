@@ -10,22 +10,31 @@
 #include <chrono>
 
 #include "rtx_impl.hpp"
+#include "wide.hpp"
 
 namespace {
 // Device counters of a frame (uint64): [0] secondary rays, [1] shadow rays.
 __global__ void k_zero_u64(unsigned long long* p, int n) {
     if (threadIdx.x < (unsigned)n) p[threadIdx.x] = 0ull;
 }
-// Device copy of up to 5 u32 arrays (the render copy of a scene), grid-stride.
+// Device copy of up to 6 u32 arrays (the render copy of a scene), grid-stride.
+// Array k has n[k] words, or, where per[k] is set, those that a tree of N nodes
+// fills: base[k] + per[k] N.  N is on the device, so that a captured copy
+// follows each replay's tree.  A tree fills about half of what its buffers have
+// to hold (nodes and differences 2T, wide records T): a copy of 1M triangles
+// takes 38 us so, 99 over the whole buffers.
 struct CopySegs {
     uint32_t* dst[6];
     const uint32_t* src[6];
     uint64_t n[6];
+    int32_t per[6], base[6];
+    const uint32_t* nodes;  // N
     int count;
 };
 __global__ __launch_bounds__(256) void k_copy_segs(CopySegs c) {
+    const int64_t N = c.count > 2 ? *c.nodes : 0;
     for (int k = 0; k < c.count; ++k) {
-        const uint64_t n = c.n[k];
+        const uint64_t n = c.per[k] ? (uint64_t)(c.base[k] + c.per[k] * N) : c.n[k];
         uint32_t* __restrict__ d = c.dst[k];
         const uint32_t* __restrict__ sp = c.src[k];
         if ((n & 3) == 0) {  // 16-byte moves (every buffer is 256-byte aligned)
@@ -37,20 +46,32 @@ __global__ __launch_bounds__(256) void k_copy_segs(CopySegs c) {
         }
     }
 }
+
+// The arrays of a render copy and their bytes, from the scene's sizes alone (a
+// build buffer may be larger, from an earlier scene); the first two are the
+// shading's.  Trees of more than WIDE_MAX_TRIS triangles have no wide records.
+struct CopyArrays {
+    DevBuf *src[6], *dst[6];
+    uint64_t bytes[6];
+    int count;
+};
+CopyArrays copy_arrays(rtx_scene* s, rtx_scene::RenderCopy& rc, bool shading_only) {
+    BuildSet& b = s->b();
+    const uint64_t T = s->T;
+    return CopyArrays{{&s->nrm, &s->matmap, &b.tri, &b.node, &b.delta, &b.wide},
+                      {&rc.nrm, &rc.matmap, &rc.tri, &rc.node, &rc.delta, &rc.wide},
+                      {(uint64_t)s->V * 16, T * 4, T * 48, T * 64 + 64, T * 32, T * 128},
+                      shading_only ? 2 : T <= WIDE_MAX_TRIS ? 6 : 5};
+}
 }  // namespace
 
 // Allocates render copy k (host-side; do it before frames run concurrently).
 int32_t rtx_reserve_render_copy(rtx_scene* s, int k, bool shading_only) {
     RTX_REQUIRE(k >= 0 && k < rtx_scene::COPIES, RTX_EINVAL, "render copy: bad copy index");
-    rtx_scene::RenderCopy& rc = s->rc[k];
+    const CopyArrays a = copy_arrays(s, s->rc[k], shading_only);
     int32_t e;
-    if ((e = rc.nrm.reserve(s->ctx, (uint64_t)s->V * 16)) || (e = rc.matmap.reserve(s->ctx, (uint64_t)s->T * 4)))
-        return e;
-    if (shading_only) return RTX_OK;
-    if ((e = rc.node.reserve(s->ctx, s->b().node.bytes)) || (e = rc.delta.reserve(s->ctx, s->b().delta.bytes)) ||
-        (e = rc.tri.reserve(s->ctx, (uint64_t)s->T * 48)) ||
-        (s->b().wide.p && (e = rc.wide.reserve(s->ctx, s->b().wide.bytes))))
-        return e;
+    for (int j = 0; j < a.count; ++j)
+        if ((e = a.dst[j]->reserve(s->ctx, a.bytes[j]))) return e;
     return RTX_OK;
 }
 
@@ -65,21 +86,17 @@ int32_t rtx_refresh_render_copy(rtx_scene* s, int k, hipStream_t st, bool shadin
 // material ids) into rc, on `st`.
 int32_t rtx_copy_render_state(rtx_scene* s, rtx_scene::RenderCopy& rc, hipStream_t st, bool shading_only) {
     int32_t e;
-    DevBuf* src[6] = {&s->nrm, &s->matmap, &s->b().node, &s->b().delta, &s->b().tri, &s->b().wide};
-    DevBuf* dst[6] = {&rc.nrm, &rc.matmap, &rc.node, &rc.delta, &rc.tri, &rc.wide};
-    const uint64_t bytes[6] = {(uint64_t)s->V * 16, (uint64_t)s->T * 4, s->b().node.bytes, s->b().delta.bytes,
-                               (uint64_t)s->T * 48, s->b().wide.bytes};
-    const int n = shading_only ? 2 : s->b().wide.p ? 6 : 5;
-    if (!shading_only && n < 6) rc.wide.release();
-    CopySegs c{};
-    for (int j = 0; j < n; ++j) {
-        RTX_REQUIRE(src[j]->p && src[j]->bytes >= bytes[j], RTX_ESTATE, "render copy: scene not built");
-        if ((e = dst[j]->reserve(s->ctx, bytes[j]))) return e;
-        c.dst[j] = dst[j]->as<uint32_t>();
-        c.src[j] = src[j]->as<uint32_t>();
-        c.n[j] = bytes[j] / 4;
+    const CopyArrays a = copy_arrays(s, rc, shading_only);
+    // nodes from byte 32 on, near-child differences, a wide record per child pair
+    CopySegs c{{}, {}, {}, {0, 0, 0, 8, 4, 16}, {0, 0, 0, 8, 0, -16},
+               s->b().levels.as<uint32_t>() + BuildSet::NODE_COUNT, a.count};
+    for (int j = 0; j < a.count; ++j) {
+        RTX_REQUIRE(a.src[j]->p && a.src[j]->bytes >= a.bytes[j], RTX_ESTATE, "render copy: scene not built");
+        if ((e = a.dst[j]->reserve(s->ctx, a.bytes[j]))) return e;
+        c.dst[j] = a.dst[j]->as<uint32_t>();
+        c.src[j] = a.src[j]->as<uint32_t>();
+        c.n[j] = a.bytes[j] / 4;
     }
-    c.count = n;
     ProfScope ps(s->ctx, st, "render_copy");
     hipLaunchKernelGGL(k_copy_segs, dim3(s->ctx->cus * 4), dim3(256), 0, st, c);
     RTX_CHECK_HIP(hipGetLastError());

@@ -122,7 +122,8 @@ struct BuildSet {
     DevBuf node, delta, parent, tri, codes, perm;
     DevBuf wide;        // wide records (wide.hpp); none for trees of more than WIDE_MAX_TRIS triangles
     DevBuf gbox;        // 6 x int32 ordered-float keys
-    DevBuf levels;      // uint32: [0..64) level offsets, [64..128) level counts, [128] node count
+    DevBuf levels;      // uint32: [0..64) level offsets, [64..128) level counts, [NODE_COUNT] node count
+    static constexpr int NODE_COUNT = 128;
     // build scratch
     DevBuf span;                  // per split: its node's range, number and children (kept for refit)
     DevBuf keys_alt, vals_alt;    // radix ping-pong

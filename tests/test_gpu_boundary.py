@@ -76,6 +76,45 @@ def _primary(rtx, ctx, cam, w, h):
     return r, oo, od
 
 
+def test_accelerator_copy_is_sized_by_its_scene(ctx):
+    """A copy holds what its scene's triangles need, also where the scene's own buffers are those of
+    an earlier, larger mesh, and it holds the whole tree: one leaf, and trees of all node counts."""
+    import rtx
+    from test_gpu_parity import load_scene, random_scene
+    s = load_scene(ctx, *random_scene(1, 60000)[:2])
+    s.build(30, 1)
+    for T, min_leaf in ((5000, 1), (5001, 8), (3, 1)):
+        pos, idx, nrm, uv, mm = random_scene(T, T)
+        if T == 3:  # one leaf, of triangles that are none's neighbours
+            pos, idx = random_scene(9, 9)[0], np.arange(9, dtype=np.uint32).reshape(3, 3)
+            nrm, uv = np.tile(np.float32([0, 0, 1]), (9, 1)), np.zeros((9, 2), np.float32)
+        s.set_geometry(pos, idx, nrm, uv, mm)
+        s.build(30, min_leaf)
+        bvh = rtx.BVHCopy(ctx)
+        before = ctx.mem_in_use()
+        bvh.copy(s)
+        # nodes 64 (+ 64 in all), differences 32, wide records 128, triangles 48, material ids 4, normals 16 a vertex
+        assert ctx.mem_in_use() - before <= T * (64 + 32 + 128 + 48 + 4) + 64 + 16 * len(pos)
+        b = O.Build(pos, idx, mm, 30, min_leaf)
+        rng = np.random.default_rng(T)
+        n = 2048
+        o4, d4 = np.zeros((n, 4), np.float32), np.full((n, 4), 1e36, np.float32)
+        o4[:, :3] = rng.uniform(-12, 12, (n, 3))
+        d4[:, :3] = pos[idx[rng.integers(0, T, n)]].mean(1) - o4[:, :3]
+        r, hb = rtx.Rays(ctx, n), rtx.Hits(ctx, n)
+        r.write(o4, d4)
+        s.update_positions(pos * np.float32(0.5))  # the scene's own buffers move on
+        s.build(30, min_leaf)
+        rtx.trace(s, r, hb, n, bvh=bvh)
+        g, want = hb.read(n), O.trace(b, nrm, uv, o4, d4)
+        assert (want["id"] >= 0).sum() > n // 4
+        for k in ("id", "t", "bary", "n4", "p4"):
+            assert np.array_equal(g[k], want[k]), (T, k)
+        for x in (r, hb, bvh):
+            x.destroy()
+    s.destroy()
+
+
 def test_trace_with_accelerator_copy(ctx):
     import rtx
     from rtx import scenes
