@@ -158,9 +158,12 @@ uint64_t rtx_mem_in_use(rtx_ctx* ctx);
  * reference fixes its work-group sizes per device, src/gpu/function.cpp:322-385):
  *   "trace_variant": 0 single-node traversal, 1 (default) four lanes per ray over
  *                    records of four grandchildren, or, for trees without such
- *                    records (over 2^25 triangles), single node with the
- *                    near-child delta loaded early, 2 sibling-pair traversal, 3
- *                    persistent waves fed from a ray queue (single-node steps);
+ *                    records (over 2^25 triangles) and with "wide_walk" 0,
+ *                    single node with the near-child delta loaded early, 2
+ *                    sibling-pair traversal, 3 persistent waves fed from a ray
+ *                    queue (single-node steps);
+ *   "wide_walk":     variant 1: 1 (default) the four-lane walk where it can be
+ *                    taken, 0 the single-node walk;
  *   "refill":        variant 3: idle lanes of a wave that trigger a refill
  *                    from the queue (1..64);
  *   "trace_block":   64, 128 or 256 threads per traversal work-group;
@@ -210,7 +213,8 @@ uint64_t rtx_mem_in_use(rtx_ctx* ctx);
  *                    everywhere;
  *   "stack_lds":     traversal stack entries per lane kept in LDS by the
  *                    single-node and sibling-pair forms (scene and wavefront
- *                    launches): 32 (the whole MAX_LEVELS stack), 16 or 8 (a
+ *                    launches; the four-lane walk, the default, has a stack of
+ *                    its own and ignores it): 32 (the whole MAX_LEVELS stack), 16 or 8 (a
  *                    ring of the top levels; deeper levels spill to the
  *                    lane's private memory), trading LDS for resident waves.
  *   "sort_bits":     LBVH radix sort digit width: 8 (default, 4 passes of

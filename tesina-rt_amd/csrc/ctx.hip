@@ -262,6 +262,9 @@ int32_t rtx_tune_set(rtx_ctx* ctx, const char* key, int64_t value) {
     if (k == "trace_variant") {
         RTX_REQUIRE(value >= 0 && value <= 4, RTX_EINVAL, "rtx_tune_set: trace_variant must be 0 to 4");
         ctx->tune.trace_variant = value;
+    } else if (k == "wide_walk") {
+        RTX_REQUIRE(value == 0 || value == 1, RTX_EINVAL, "rtx_tune_set: wide_walk must be 0 or 1");
+        ctx->tune.wide_walk = value;
     } else if (k == "trace_block") {
         RTX_REQUIRE(value == 64 || value == 128 || value == 256, RTX_EINVAL,
                     "rtx_tune_set: trace_block must be 64, 128 or 256");
@@ -319,6 +322,7 @@ int64_t rtx_tune_get(rtx_ctx* ctx, const char* key) {
     if (!ctx || !key) return -1;
     std::string k(key);
     if (k == "trace_variant") return ctx->tune.trace_variant;
+    if (k == "wide_walk") return ctx->tune.wide_walk;
     if (k == "trace_block") return ctx->tune.trace_block;
     if (k == "xcds") return ctx->tune.xcds;
     if (k == "coop_leaf") return ctx->tune.coop_leaf;

@@ -66,6 +66,8 @@ struct KernelTiming {
 struct rtx_tuning {
     int64_t trace_variant = 1;  // 0 single node, 1 + early delta load, 2 sibling pairs, 3 persistent + ray queue,
                                 // 4 stackless walk by parent pointers
+    int64_t wide_walk = 1;      // trace_variant 1: four lanes per ray where the tree has wide records; 0: a lane per
+                                // ray, as over trees without them
     int64_t trace_block = 128;  // 64, 128 or 256 threads per traversal block
     int64_t xcds = 1;           // ray chunks = L2 domains (MI355X: 8 XCDs); 1 = plain grid order
     int64_t sort_bits = 8;      // LBVH radix sort digit width: 8 or 4 bits a pass

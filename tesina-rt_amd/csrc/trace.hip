@@ -3246,7 +3246,7 @@ static int traversal_variant(const rtx_scene* s, const SceneView& sv) {
     if (var == 4 && !sv.parent) var = 1;
     const int depth = s->ext ? s->ext->depth : s->depth;
     if (var == 2 && depth >= STACK) return 1;
-    return var == 1 && sv.wide && s->T <= WIDE_MAX_TRIS ? WIDE_GROUP : var;
+    return var == 1 && s->ctx->tune.wide_walk && sv.wide && s->T <= WIDE_MAX_TRIS ? WIDE_GROUP : var;
 }
 
 // Grid of a scene walk: four lanes per item for WIDE_GROUP.
@@ -3597,7 +3597,7 @@ static int32_t refresh_roots(rtx_instances* in, hipStream_t st, int* var) {
     int32_t e = instance_bases(in, base);
     if (e) return e;
     in->table.resize(in->n);
-    bool deep = false, wide = true;
+    bool deep = false, wide = in->ctx->tune.wide_walk != 0;
     for (int i = 0; i < in->n; ++i) {
         rtx_scene* s = in->scene[i];
         RTX_REQUIRE(s->built, RTX_ESTATE, "rtx_trace_instances: an instance's scene has no BVH");

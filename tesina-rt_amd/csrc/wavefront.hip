@@ -313,7 +313,7 @@ int32_t rtx_wavefront_step_impl(rtx_wavefront* wf, hipStream_t st, int32_t* pend
     // persistent and stackless forms have no segmented kernels
     int var = (int)c->tune.trace_variant;
     if (var > 2 || (var == 2 && deep)) var = 1;
-    if (var == 1 && wide) var = WF_WIDE;
+    if (var == 1 && wide && c->tune.wide_walk) var = WF_WIDE;
     const int tb = (int)c->tune.trace_block;
     uint32_t coop = c->tune.coop_leaf > 0 ? (uint32_t)c->tune.coop_leaf : 0xffffffffu;
     if (var == WF_WIDE) coop = rtx_wide_coop(c);

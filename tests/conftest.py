@@ -1,4 +1,5 @@
 """Shared pytest setup: markers, import paths, GPU gating."""
+import contextlib
 import sys
 from pathlib import Path
 
@@ -20,6 +21,23 @@ def gpu_available() -> bool:
         return torch.cuda.device_count() > 0
     except Exception:
         return False
+
+
+@contextlib.contextmanager
+def tuned(ctx, **knobs):
+    """The context's tuning knobs set for a block, and set back however it ends."""
+    old = {k: ctx.tuned(k) for k in knobs}
+    try:
+        for k, v in knobs.items():
+            ctx.tune(k, v)
+        yield
+    finally:
+        for k, v in old.items():
+            ctx.tune(k, v)
+
+
+# trace_variant, wide_walk: the traversal forms with a multi-lane and a single-lane form 1
+FORMS = [(0, 1), (1, 1), (1, 0), (2, 1), (3, 1)]
 
 
 @pytest.fixture(scope="session")

@@ -201,6 +201,7 @@ def test_stage_tracer_overloads_and_builder_log(tmp_path):
 
 TUNE_KEYS = {  # key: (values accepted, values refused)
     "trace_variant": ([0, 4], [-1, 5]),
+    "wide_walk": ([0, 1], [-1, 2]),
     "trace_block": ([64, 128, 256], [32, 512]),
     "xcds": ([1, 64], [0, 65]),
     "refill": ([1, 64], [0, 65]),

@@ -18,6 +18,7 @@ import numpy as np
 import pytest
 
 import oracle as O
+from conftest import tuned
 
 pytestmark = pytest.mark.gpu
 
@@ -103,8 +104,8 @@ CAMS = {
 
 @pytest.mark.parametrize("cam_name", list(CAMS))
 @pytest.mark.parametrize("coop", [0, 1, 2, 8, 64])
-@pytest.mark.parametrize("variant", [0, 1, 3])
-def test_coop_leaf_thresholds_identical(ctx, poles, cam_name, coop, variant):
+@pytest.mark.parametrize("variant,wide", [(0, 1), (1, 1), (1, 0), (3, 1)])
+def test_coop_leaf_thresholds_identical(ctx, poles, cam_name, coop, variant, wide):
     rtx = _rtx()
     s, b = poles["s"], poles["b"]
     p, at, up, w, h = CAMS[cam_name]
@@ -112,10 +113,7 @@ def test_coop_leaf_thresholds_identical(ctx, poles, cam_name, coop, variant):
     n = w * h
     r, r2 = rtx.Rays(ctx, 2 * n + 2), rtx.Rays(ctx, 2 * n + 2)
     hb = rtx.Hits(ctx, 2 * n + 2)
-    old = (ctx.tuned("coop_leaf"), ctx.tuned("trace_variant"))
-    ctx.tune("coop_leaf", coop)
-    ctx.tune("trace_variant", variant)
-    try:
+    with tuned(ctx, coop_leaf=coop, trace_variant=variant, wide_walk=wide):
         r.primary(cam, w, h)
         rtx.trace(s, r, hb, n)
         rtx.trace_shadow(s, r, hb, n)
@@ -124,9 +122,6 @@ def test_coop_leaf_thresholds_identical(ctx, poles, cam_name, coop, variant):
         rtx.trace(s, r2, hb, m)
         rtx.trace_shadow(s, r2, hb, m)
         g2 = hb.read(m)
-    finally:
-        ctx.tune("coop_leaf", old[0])
-        ctx.tune("trace_variant", old[1])
     lights = O.lights_from(poles["lights"])
     oo, od, op, oc = O.raygen_primary(O.camera_from(cam), w, h)
     o = O.trace(b, poles["nrm"], poles["uv"], oo, od)

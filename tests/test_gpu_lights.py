@@ -9,6 +9,7 @@ import numpy as np
 import pytest
 
 import oracle as O
+from conftest import FORMS, tuned
 
 pytestmark = pytest.mark.gpu
 
@@ -52,22 +53,20 @@ def _primary_hits(rtx, ctx, s, cam, w, h):
     return r, hb
 
 
-@pytest.mark.parametrize("variant", [0, 1, 2, 3, 4])
+@pytest.mark.parametrize("variant,wide", [*FORMS, (4, 1)])
 @pytest.mark.parametrize("which", ["spot", "dir", "point", "mixed"])
-def test_shadow_flags_per_light_type(ctx, c1s, which, variant):
+def test_shadow_flags_per_light_type(ctx, c1s, which, variant, wide):
     import rtx
     sd, s, b, cam = c1s
     w, h = 256, 256
     L = rtx.make_lights((0.1, 0.1, 0.1), LIGHT_SETS[which])
     s.set_lights(L)
-    old = ctx.tuned("trace_variant")
-    ctx.tune("trace_variant", variant)
     try:
-        r, hb = _primary_hits(rtx, ctx, s, cam, w, h)
-        rtx.trace_shadow(s, r, hb, w * h)
-        g = hb.read(w * h)
+        with tuned(ctx, trace_variant=variant, wide_walk=wide):
+            r, hb = _primary_hits(rtx, ctx, s, cam, w, h)
+            rtx.trace_shadow(s, r, hb, w * h)
+            g = hb.read(w * h)
     finally:
-        ctx.tune("trace_variant", old)
         s.set_lights(sd.lights)
     oo, od, _, _ = O.raygen_primary(O.camera_from(cam), w, h)
     o = O.trace(b, sd.nrm, sd.uv, oo, od)

@@ -15,6 +15,7 @@ import numpy as np
 import pytest
 
 import oracle as O
+from conftest import FORMS, tuned
 
 pytestmark = pytest.mark.gpu
 
@@ -411,9 +412,9 @@ def test_frame_rebuild_c1(ctx, c1):
     s.destroy()
 
 
-@pytest.mark.parametrize("variant", [0, 1, 2, 3])
+@pytest.mark.parametrize("variant,wide", FORMS)
 @pytest.mark.parametrize("block", [64, 128, 256])
-def test_traversal_variants_identical(ctx, c1, variant, block):
+def test_traversal_variants_identical(ctx, c1, variant, wide, block):
     # every tuned traversal form reproduces the oracle's hits and shadow flags
     rtx = _rtx()
     sd, s, b, cam = c1
@@ -422,10 +423,7 @@ def test_traversal_variants_identical(ctx, c1, variant, block):
     r = rtx.Rays(ctx, 2 * n)
     r2 = rtx.Rays(ctx, 2 * n)
     hb = rtx.Hits(ctx, 2 * n)
-    old = (ctx.tuned("trace_variant"), ctx.tuned("trace_block"))
-    ctx.tune("trace_variant", variant)
-    ctx.tune("trace_block", block)
-    try:
+    with tuned(ctx, trace_variant=variant, wide_walk=wide, trace_block=block):
         r.primary(cam, w, h)
         rtx.trace(s, r, hb, n)
         rtx.trace_shadow(s, r, hb, n)
@@ -434,9 +432,6 @@ def test_traversal_variants_identical(ctx, c1, variant, block):
         rtx.trace(s, r2, hb, m)
         rtx.trace_shadow(s, r2, hb, m)
         g2 = hb.read(m)
-    finally:
-        ctx.tune("trace_variant", old[0])
-        ctx.tune("trace_block", old[1])
     lights = O.lights_from(sd.lights)
     oo, od, op, oc = O.raygen_primary(O.camera_from(cam), w, h)
     o = O.trace(b, sd.nrm, sd.uv, oo, od)

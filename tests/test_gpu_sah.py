@@ -14,6 +14,7 @@ import numpy as np
 import pytest
 
 import oracle as O
+from conftest import FORMS, tuned
 from sah_cases import terrain_scene
 from test_gpu_parity import load_scene
 
@@ -91,16 +92,13 @@ def test_sah_tree_traversal(ctx, case):
     r.write(ori4, dir4)
     hb = rtx.Hits(ctx, n)
     old = ctx.tuned("trace_variant")
-    try:
-        for variant in (0, 1, 2, 3):
-            ctx.tune("trace_variant", variant)
+    for variant, wide in FORMS:
+        with tuned(ctx, trace_variant=variant, wide_walk=wide):
             rtx.trace(s, r, hb, n)
             rtx.trace_shadow(s, r, hb, n)
             got = hb.read(n)
-            for k in ("flags", "id", "t", "bary", "n4", "p4", "uv2"):
-                assert np.array_equal(got[k], o[k]), f"{case}: {k} differs (variant {variant})"
-    finally:
-        ctx.tune("trace_variant", old)
+        for k in ("flags", "id", "t", "bary", "n4", "p4", "uv2"):
+            assert np.array_equal(got[k], o[k]), f"{case}: {k} differs (variant {variant}, wide {wide})"
     # the stackless walk (form 4) against the oracle's stackless walk: on the
     # 36-level tree it does not end rays at MAX_LEVELS
     with O.stackless():

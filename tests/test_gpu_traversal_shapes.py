@@ -7,7 +7,7 @@ leaves, tested by the whole wave) and a flat axis.  Random rays from inside
 and around the scene give long, incoherent traversals.  Hits and shadow
 flags of each form must equal the oracle's bit for bit, with the whole
 traversal stack in LDS and with ring stacks of 16 and 8 LDS entries (the
-deeper levels in private memory), with shadow rays in the reference's child
+deeper levels in private memory), form 1 with four lanes per ray and with one, with shadow rays in the reference's child
 order and in index order.
 """
 import numpy as np
@@ -15,6 +15,7 @@ import pytest
 
 import oracle as O
 from chain import chain_scene
+from conftest import tuned
 from test_gpu_parity import load_scene, random_scene
 
 pytestmark = pytest.mark.gpu
@@ -71,43 +72,36 @@ def test_traversal_forms_match_oracle(ctx, T, depth, min_leaf, seed, kind):
     o["flags"] = O.trace_shadow(b, O.lights_from(lights), o["flags"], o["p4"])
     if T >= 300:
         assert (o["id"] >= 0).sum() > n // 8, "the rays should hit the scene"
-    old = (ctx.tuned("trace_variant"), ctx.tuned("stack_lds"), ctx.tuned("shadow_order"))
-    try:
-        for variant, sl, so in ((0, 32, 0), (0, 16, 0), (0, 8, 0), (1, 32, 0), (1, 16, 0), (1, 8, 0), (2, 32, 0),
-                                (2, 16, 0), (2, 8, 0), (0, 32, 1), (1, 32, 1), (1, 16, 1)):
-            # so: shadow rays in the reference's child order (1) or in index order (0)
-            ctx.tune("trace_variant", variant)
-            ctx.tune("stack_lds", sl)
-            ctx.tune("shadow_order", so)
+    # wide: form 1 with four lanes per ray (a stack of its own) or one (1, 0);
+    # so: shadow rays in the reference's child order (1) or in index order (0)
+    for variant, wide, sl, so in ((0, 1, 32, 0), (0, 1, 16, 0), (0, 1, 8, 0), (1, 1, 32, 0), (1, 0, 32, 0),
+                                  (1, 0, 16, 0), (1, 0, 8, 0), (2, 1, 32, 0), (2, 1, 16, 0), (2, 1, 8, 0),
+                                  (0, 1, 32, 1), (1, 1, 32, 1), (1, 0, 32, 1), (1, 0, 16, 1)):
+        with tuned(ctx, trace_variant=variant, wide_walk=wide, stack_lds=sl, shadow_order=so):
             rtx.trace(s, r, hb, n)
             rtx.trace_shadow(s, r, hb, n)
             g = hb.read(n)
-            for k in ("flags", "id", "t", "bary", "n4", "p4"):
-                assert np.array_equal(g[k], o[k]), \
-                    f"{k} differs (variant {variant}, stack_lds {sl}, shadow_order {so}, T {T}, depth {depth})"
-        # the stackless walk (parent pointers of the LBVH) against the oracle's
-        with O.stackless():
-            ons = O.trace(b, nrm, uv, ori4, dir4)
-            ons["flags"] = O.trace_shadow(b, O.lights_from(lights), ons["flags"], ons["p4"])
-        ctx.tune("trace_variant", 4)
-        ctx.tune("stack_lds", 32)
+        for k in ("flags", "id", "t", "bary", "n4", "p4"):
+            assert np.array_equal(g[k], o[k]), f"{k} differs (variant {variant}, wide {wide}, stack_lds {sl}, " \
+                                               f"shadow_order {so}, T {T}, depth {depth})"
+    # the stackless walk (parent pointers of the LBVH) against the oracle's
+    with O.stackless():
+        ons = O.trace(b, nrm, uv, ori4, dir4)
+        ons["flags"] = O.trace_shadow(b, O.lights_from(lights), ons["flags"], ons["p4"])
+    with tuned(ctx, trace_variant=4, stack_lds=32):
         rtx.trace(s, r, hb, n)
         rtx.trace_shadow(s, r, hb, n)
         g = hb.read(n)
-        for k in ("flags", "id", "t", "bary", "n4", "p4"):
-            assert np.array_equal(g[k], ons[k]), f"{k} differs (stackless, T {T}, depth {depth})"
-    finally:
-        ctx.tune("trace_variant", old[0])
-        ctx.tune("stack_lds", old[1])
-        ctx.tune("shadow_order", old[2])
+    for k in ("flags", "id", "t", "bary", "n4", "p4"):
+        assert np.array_equal(g[k], ons[k]), f"{k} differs (stackless, T {T}, depth {depth})"
     r.destroy()
     hb.destroy()
     s.destroy()
 
 
-@pytest.mark.parametrize("variant,stack_lds", [(0, 32), (1, 32), (2, 32), (3, 32), (4, 32), (0, 16), (1, 16),
-                                               (1, 8), (2, 8)])
-def test_max_levels_rule(ctx, variant, stack_lds):
+@pytest.mark.parametrize("variant,wide,stack_lds", [(0, 1, 32), (1, 1, 32), (1, 0, 32), (2, 1, 32), (3, 1, 32),
+                                                    (4, 1, 32), (0, 1, 16), (1, 0, 16), (1, 0, 8), (2, 1, 8)])
+def test_max_levels_rule(ctx, variant, wide, stack_lds):
     # A ray whose near children all lie on the chain has 32 entries on its
     # stack at the bottom leaf; the reference then ends the ray instead of
     # popping (src/kernel/trace-bvh.cl:361-367, shadow-trace-bvh.cl alike).
@@ -151,18 +145,12 @@ def test_max_levels_rule(ctx, variant, stack_lds):
     r = rtx.Rays(ctx, n)
     r.write(ori4, dir4)
     hb = rtx.Hits(ctx, n)
-    old = (ctx.tuned("trace_variant"), ctx.tuned("stack_lds"))
-    try:
-        ctx.tune("trace_variant", variant)
-        ctx.tune("stack_lds", stack_lds)
+    with tuned(ctx, trace_variant=variant, wide_walk=wide, stack_lds=stack_lds):
         rtx.trace(s, r, hb, n)
         rtx.trace_shadow(s, r, hb, n)
         g = hb.read(n)
-    finally:
-        ctx.tune("trace_variant", old[0])
-        ctx.tune("stack_lds", old[1])
     for k in ("flags", "id", "t", "bary", "n4", "p4"):
-        assert np.array_equal(g[k], o[k]), f"{k} differs (variant {variant}, stack_lds {stack_lds})"
+        assert np.array_equal(g[k], o[k]), f"{k} differs (variant {variant}, wide {wide}, stack_lds {stack_lds})"
     r.destroy()
     hb.destroy()
     s.destroy()

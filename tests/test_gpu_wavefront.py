@@ -13,6 +13,7 @@ import numpy as np
 import pytest
 
 import oracle as O
+from conftest import tuned
 
 pytestmark = pytest.mark.gpu
 
@@ -129,14 +130,16 @@ def test_frames_together_equal_stand_alone(ctx, wf_scenes, expected):
         wf.destroy()
 
 
-@pytest.mark.parametrize("variant,block,sched,stack_lds,shadow_order,share", [
-    (0, 64, 0, 32, 0, 0), (1, 128, 0, 32, 0, 0), (1, 128, 1, 32, 0, 0), (2, 256, 0, 32, 0, 0), (2, 128, 1, 32, 0, 0),
-    (3, 128, 0, 32, 0, 0), (4, 64, 1, 32, 0, 0), (1, 128, 1, 16, 0, 0), (1, 128, 0, 16, 0, 0), (2, 256, 1, 16, 0, 0),
-    (0, 64, 1, 8, 0, 0), (1, 256, 0, 8, 0, 0), (1, 128, 1, 32, 1, 0), (0, 128, 0, 32, 1, 0), (1, 128, 1, 32, 0, 65),
-    (1, 64, 1, 16, 0, 1)])
-def test_every_traversal_form(ctx, wf_scenes, expected, variant, block, sched, stack_lds, shadow_order, share):
+@pytest.mark.parametrize("variant,wide,block,sched,stack_lds,shadow_order,share", [
+    (0, 1, 64, 0, 32, 0, 0), (1, 1, 128, 0, 32, 0, 0), (1, 1, 128, 1, 32, 0, 0), (2, 1, 256, 0, 32, 0, 0),
+    (2, 1, 128, 1, 32, 0, 0), (3, 1, 128, 0, 32, 0, 0), (4, 1, 64, 1, 32, 0, 0), (1, 0, 128, 1, 16, 0, 0),
+    (1, 0, 128, 0, 16, 0, 0), (2, 1, 256, 1, 16, 0, 0), (0, 1, 64, 1, 8, 0, 0), (1, 0, 256, 0, 8, 0, 0),
+    (1, 1, 128, 1, 32, 1, 0), (0, 1, 128, 0, 32, 1, 0), (1, 1, 128, 1, 32, 0, 65), (1, 0, 64, 1, 16, 0, 1),
+    (1, 1, 64, 1, 32, 0, 1), (1, 1, 256, 0, 32, 0, 0), (1, 0, 128, 0, 32, 0, 0), (1, 0, 128, 1, 32, 1, 65)])
+def test_every_traversal_form(ctx, wf_scenes, expected, variant, wide, block, sched, stack_lds, shadow_order, share):
     # the sibling-pair form falls back to the single-node form when a scene
-    # has 32 levels (the chain); the persistent and stackless forms map to it;
+    # has 32 levels (the chain); the persistent and stackless forms map to form 1;
+    # wide: form 1 with four lanes per ray (which ignores stack_lds) or one;
     # sched: closest hit in launch order (0) or by persistent waves (1);
     # stack_lds: traversal stack entries in LDS (the rest in private memory);
     # shadow_order: shadow rays in the reference's child order (1) or in index
@@ -144,31 +147,19 @@ def test_every_traversal_form(ctx, wf_scenes, expected, variant, block, sched, s
     # share: percent of the resident blocks a persistent launch takes (1: one
     # block per CU)
     rtx = _rtx()
-    old = (ctx.tuned("trace_variant"), ctx.tuned("trace_block"), ctx.tuned("wf_sched"), ctx.tuned("stack_lds"),
-           ctx.tuned("shadow_order"), ctx.tuned("wf_share"))
-    ctx.tune("trace_variant", variant)
-    ctx.tune("trace_block", block)
-    ctx.tune("wf_sched", sched)
-    ctx.tune("stack_lds", stack_lds)
-    ctx.tune("shadow_order", shadow_order)
-    ctx.tune("wf_share", share)
-    wf = rtx.Wavefront(ctx, arena_bytes=2 << 30, max_frames=32)
-    try:
-        ids = []
-        for name, w, h, b, cap in FRAMES:
-            s, cam, _ = wf_scenes[name]
-            ids.append(wf.add(s, cam, w, h, b, ray_capacity=cap))
-        wf.run()
-        for k, fid in enumerate(ids):
-            _check(wf, fid, expected[k], f"variant {variant} block {block} frame {k}")
-    finally:
-        wf.destroy()
-        ctx.tune("trace_variant", old[0])
-        ctx.tune("trace_block", old[1])
-        ctx.tune("wf_sched", old[2])
-        ctx.tune("stack_lds", old[3])
-        ctx.tune("shadow_order", old[4])
-        ctx.tune("wf_share", old[5])
+    with tuned(ctx, trace_variant=variant, wide_walk=wide, trace_block=block, wf_sched=sched, stack_lds=stack_lds,
+               shadow_order=shadow_order, wf_share=share):
+        wf = rtx.Wavefront(ctx, arena_bytes=2 << 30, max_frames=32)
+        try:
+            ids = []
+            for name, w, h, b, cap in FRAMES:
+                s, cam, _ = wf_scenes[name]
+                ids.append(wf.add(s, cam, w, h, b, ray_capacity=cap))
+            wf.run()
+            for k, fid in enumerate(ids):
+                _check(wf, fid, expected[k], f"variant {variant} wide {wide} block {block} frame {k}")
+        finally:
+            wf.destroy()
 
 
 def test_frames_joining_at_different_steps(ctx, wf_scenes, expected):

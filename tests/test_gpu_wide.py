@@ -13,6 +13,7 @@ import numpy as np
 import pytest
 
 import oracle as O
+from conftest import tuned
 from test_gpu_parity import check_build, load_scene, random_scene
 
 pytestmark = pytest.mark.gpu
@@ -257,3 +258,142 @@ def test_sort_tiles(ctx, T):
     unsorted[perm] = codes
     assert np.array_equal(np.argsort(unsorted, kind="stable"), perm)
     assert np.array_equal(got[0][0], codes) and np.array_equal(got[0][1], perm)
+
+
+def test_frames_without_the_wide_walk(ctx):
+    """Every way of rendering the same frames with one lane per ray (wide_walk 0, as over trees without
+    wide records) gives the images of the four-lane walk."""
+    import rtx
+    from rtx import scenes
+    sd = scenes.config_c1()
+    s = scenes.load(rtx.Scene(ctx), sd)
+    w, h = 160, 120
+    cam = rtx.camera_set(sd.camera["pos"], sd.camera["look_at"], sd.camera["up"], sd.camera["fov"], w / h)
+
+    def frames():
+        out = {}
+        R = rtx.Renderer(ctx, w, h, 3)
+        for mode in ("plain", "async", "pipelined", "graph"):
+            R.set_pipelined(mode == "pipelined")
+            if mode == "plain":
+                R.frame(s, cam)
+            elif mode == "graph":
+                R.capture(s, cam)
+                for _ in range(2):
+                    R.replay()
+            else:
+                for _ in range(2):
+                    R.frame_async(s, cam)
+            ctx.sync()
+            out[mode] = R.fb.accum()
+        R.destroy()
+        pl = rtx.Pipeline(ctx, s, w, h, 3, depth=2)
+        for _ in range(3):
+            last = pl.frame(cam)
+        pl.wait(last)
+        out["pipeline"] = pl.fb(last).accum()
+        pl.destroy()
+        return out
+
+    want = frames()
+    assert (want["plain"] > 0).any(1).mean() > 0.2
+    with tuned(ctx, wide_walk=0):
+        got = frames()
+    for mode in want:
+        assert np.array_equal(got[mode], want[mode]), mode
+        assert np.array_equal(got[mode], want["plain"]), mode
+    s.destroy()
+
+
+def test_tree_without_wide_records(ctx):
+    """A scene that had wide records, then a mesh of more than 2^25 triangles, which gets none (the
+    earlier tree's are still in the buffer): scene, accelerator-copy, wavefront and instance launches
+    of the default form give the records of form 0, before and after a refit, and rays straight down
+    end on the surface."""
+    import rtx
+    n, m = 4098, 4098  # 2 * 4097 * 4097 triangles
+    x = np.arange(n, dtype=np.float32)
+
+    def mesh(phase):
+        y = np.round(8 * np.sin(0.01 * x[:, None] + phase) * np.cos(0.013 * x[None, :])).astype(np.float32)
+        pos = np.empty((n, m, 3), np.float32)
+        pos[..., 0], pos[..., 1], pos[..., 2] = x[:, None], y, x[None, :]
+        return pos.reshape(-1, 3)
+
+    pos = mesh(0.0)
+    v = np.arange(n * m, dtype=np.uint32).reshape(n, m)[:-1, :-1].ravel()
+    idx = np.empty((2 * len(v), 3), np.uint32)
+    for k, o in enumerate((0, m, m + 1)):
+        np.add(v, np.uint32(o), out=idx[0::2, k])
+    for k, o in enumerate((0, m + 1, 1)):
+        np.add(v, np.uint32(o), out=idx[1::2, k])
+    T = len(idx)
+    assert T > 1 << 25
+    mats = rtx.make_materials([(0.8, 0.3, 0.2, 0.5, 0.5, 0.0)])
+    lights = rtx.make_lights((0.1, 0.1, 0.1), [dict(type=rtx.LIGHT_POINT, pos=(2000.0, 300.0, 2000.0))])
+    p, i, nr, _, _ = random_scene(3, 5000)
+    s = load_scene(ctx, p, i, nr, mats=mats, lights=lights)
+    s.build()
+    # with normals: bounce rays of zero normals are NaN, which pass every box of the tree
+    s.set_geometry(pos, idx, np.tile(np.float32([0, 1, 0]), (len(pos), 1)))
+    s.build()
+    small = load_scene(ctx, p, i, nr, lights=lights)
+    small.build()
+    rng = np.random.default_rng(8)
+    count = 8192
+    ori4, dir4 = np.zeros((count, 4), np.float32), np.full((count, 4), 1e36, np.float32)
+    ori4[:, 0], ori4[:, 2] = rng.uniform(0, n - 1, (2, count))
+    ori4[:, 1] = 50
+    dir4[:, :3] = rng.normal(size=(count, 3))
+    dir4[:, 1] = -np.abs(dir4[:, 1]) * 0.2
+    dir4[: count // 2, :3] = (0, -1, 0)
+    r, h = rtx.Rays(ctx, count), rtx.Hits(ctx, count)
+    r.write(ori4, dir4)
+    inst = rtx.Instances(ctx, [s, small], np.tile(np.eye(4, dtype=np.float32), (2, 1, 1)),
+                         np.tile(np.eye(4, dtype=np.float32), (2, 1, 1)))
+    inst.set_lights(lights)
+    cam = rtx.camera_set((100.0, 60.0, -50.0), (800.0, 0.0, 800.0), (0, 1, 0), np.pi / 4, 1.0)
+    bvh = rtx.BVHCopy(ctx)
+
+    def records(trace, shadow):
+        trace()
+        shadow()
+        return h.read(count)
+
+    def everything():
+        out = {"scene": records(lambda: rtx.trace(s, r, h, count), lambda: rtx.trace_shadow(s, r, h, count)),
+               "copy": records(lambda: rtx.trace(s, r, h, count, bvh=bvh),
+                               lambda: rtx.trace_shadow(s, r, h, count, bvh=bvh)),
+               "instances": records(lambda: inst.trace(r, h, count), lambda: inst.trace_shadow(r, h, count))}
+        wf = rtx.Wavefront(ctx, arena_bytes=1 << 28, max_frames=1)
+        fid = wf.add(s, cam, 128, 128, 1)
+        wf.run()
+        out["wavefront"] = {"accum": wf.accum(fid)}
+        wf.destroy()
+        return out
+
+    for phase in (0.0, 0.7):
+        if phase:
+            pos = mesh(phase)
+            s.update_positions(pos)
+            s.refit()
+        bvh.copy(s)
+        got = everything()
+        with tuned(ctx, trace_variant=0):
+            want = everything()
+        for what in want:
+            for k in want[what]:
+                assert np.array_equal(got[what][k], want[what][k], equal_nan=True), (phase, what, k)
+        assert np.array_equal(got["copy"]["id"], got["scene"]["id"])
+        assert got["wavefront"]["accum"].any()
+        down = got["scene"]["t"][: count // 2]
+        c = ori4[: count // 2].astype(np.float64)
+        ix, iz = np.floor(c[:, 0]).astype(int), np.floor(c[:, 2]).astype(int)
+        fx, fz = c[:, 0] - ix, c[:, 2] - iz
+        y = pos.reshape(n, m, 3)[..., 1].astype(np.float64)
+        y00, y10, y01, y11 = y[ix, iz], y[ix + 1, iz], y[ix, iz + 1], y[ix + 1, iz + 1]
+        at = np.where(fx >= fz, y00 + fx * (y10 - y00) + fz * (y11 - y10), y00 + fz * (y01 - y00) + fx * (y11 - y01))
+        # t is near 50; its rounding, and that of the vertex differences, are a few units of 4e-6
+        assert np.abs(50 - down - at).max() < 1e-3
+    for z in (inst, bvh, r, h, s, small):
+        z.destroy()
