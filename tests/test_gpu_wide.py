@@ -196,17 +196,18 @@ def test_wide_walk_full_stack(ctx):
 
 def test_instances_left_to_the_exact_walk(ctx):
     """Rays that leave the wide walk of an instance (a full stack, an infinite reciprocal with an
-    infinite tMax) and leaves of all sizes, over sets of one and two chunks of roots: the records of
-    the loop that walks a ray per lane over the same candidate roots."""
+    infinite tMax) and leaves of all sizes, over sets of one and two chunks of roots: the oracle's
+    records, and so those of the loops that walk a ray per lane over the same roots."""
     import rtx
     pos, idx = _nested_scene()
-    a = load_scene(ctx, pos, idx)
-    pos, idx, nrm, uv, mm = random_scene(5, 300)
+    meshes = [(pos, np.tile(np.float32([0, 0, 1]), (len(pos), 1)), np.zeros((len(pos), 2), np.float32), idx)]
+    pos, idx, nrm, uv, _ = random_scene(5, 300)
     pos = np.round(pos).astype(np.float32) + np.float32(0.0)
-    idx = np.repeat(idx, np.arange(300) % 40 + 1, axis=0)
-    b = load_scene(ctx, pos, idx, nrm, uv, np.zeros(len(idx), np.int32))
-    for s in (a, b):
+    meshes.append((pos, nrm, uv, np.repeat(idx, np.arange(300) % 40 + 1, axis=0)))
+    scs = [load_scene(ctx, p, i, n, t, np.zeros(len(i), np.int32)) for p, n, t, i in meshes]
+    for s in scs:
         s.build(30, 1)
+    builds = [O.Build(p, i, None, 30, 1) for p, _, _, i in meshes]
     rng = np.random.default_rng(4)
     ori4, dir4 = _odd_rays(rng, pos, 2048)
     d = rng.uniform(0.5, 1.0, (512, 3)).astype(np.float32)
@@ -214,27 +215,27 @@ def test_instances_left_to_the_exact_walk(ctx):
     ori4[::4, 3], dir4[::4, 3] = 0.0, 1e36
     r, h = rtx.Rays(ctx, 2048), rtx.Hits(ctx, 2048)
     r.write(ori4, dir4)
-    old = ctx.tuned("trace_variant")
     for n in (3, 70):
         tr = np.tile(np.eye(4, dtype=np.float32), (n, 1, 1))
         tr[1:, :3, 3] = rng.integers(-20, 20, (n - 1, 3))
         tr[2::3, :3, :3] *= 2.0
-        inst = rtx.Instances(ctx, [(a, b)[i % 2] for i in range(n)], tr, np.linalg.inv(tr).astype(np.float32))
+        inv = np.linalg.inv(tr).astype(np.float32)
+        inst = rtx.Instances(ctx, [scs[i % 2] for i in range(n)], tr, inv)
         inst.set_lights(_lights())
-        want = None
-        for form in (0, 1):
-            ctx.tune("trace_variant", form)
-            inst.trace(r, h, 2048)
-            inst.trace_shadow(r, h, 2048)
-            got = h.read(2048)
-            want = want or got
-            for k in want:
-                if k != "list":
-                    assert np.array_equal(got[k], want[k], equal_nan=got[k].dtype.kind == "f"), (n, form, k)
+        ms = O.MultiScene(builds, [m[1] for m in meshes], [m[2] for m in meshes],
+                          [(i % 2, tr[i], inv[i]) for i in range(n)])
+        want = O.trace_multi(ms, ori4, dir4)
+        want["flags"] = O.trace_shadow_multi(ms, O.lights_from(_lights()), want["flags"], want["p4"])
         assert (want["id"] >= 0).sum() > 300
+        for form, wide in ((0, 1), (1, 1), (1, 0)):
+            with tuned(ctx, trace_variant=form, wide_walk=wide):
+                inst.trace(r, h, 2048)
+                inst.trace_shadow(r, h, 2048)
+                got = h.read(2048)
+            for k in ("flags", "t", "id", "bary", "n4", "p4", "uv2"):
+                assert np.array_equal(got[k], want[k], equal_nan=got[k].dtype.kind == "f"), (n, form, wide, k)
         inst.destroy()
-    ctx.tune("trace_variant", old)
-    for x in (r, h, a, b):
+    for x in (r, h, *scs):
         x.destroy()
 
 
@@ -245,14 +246,13 @@ def test_sort_tiles(ctx, T):
     rng = np.random.default_rng(T)
     pos = rng.uniform(-5, 5, (max(3, T // 3), 3)).astype(np.float32)
     idx = rng.integers(0, len(pos), (T, 3)).astype(np.uint32)
-    old, got = ctx.tuned("sort_items"), []
+    got = []
     for items in (32, 16):
-        ctx.tune("sort_items", items)
-        s = load_scene(ctx, pos, idx, None, None, np.zeros(T, np.int32))
-        s.build()
-        got.append((s.codes(), s.perm()))
-        s.destroy()
-    ctx.tune("sort_items", old)
+        with tuned(ctx, sort_items=items):
+            s = load_scene(ctx, pos, idx, None, None, np.zeros(T, np.int32))
+            s.build()
+            got.append((s.codes(), s.perm()))
+            s.destroy()
     codes, perm = got[1]
     unsorted = np.empty_like(codes)
     unsorted[perm] = codes
