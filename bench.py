@@ -20,7 +20,7 @@ traversal) and of the build's HBM-bound radix-sort pass, with HBM traffic
 per launch when recorded under profiles/, and the CPU oracle timed on this
 host on the same frame (one core, median of 3 frames).
 
-    python bench.py [--gpus 1] [--steps K] [--warmup W] [--no-cpu]
+    python bench.py [--gpus 1] [--steps K] [--warmup W] [--no-cpu] [--details FILE]
     python bench.py --copy-calibration 256   # device copy for counter scaling
     python bench.py --c3-only --c3-frames 20 # the dynamic-scene leg alone
 """
@@ -195,12 +195,33 @@ def copy_calibration(mib: int, reps: int = 3):
                       "reps": reps}))
 
 
+def result_line(out):
+    """The printed line: the headline with its configuration, the rooflines and the CPU baseline whole, of
+    every other section the plain figures (tables, sweeps, texts and per-kernel times are in --details)."""
+    whole = ("config", "env", "roofline", "roofline_sort_pass", "cpu_baseline")
+    line = {}
+    for k, v in out.items():
+        if k in whole or not isinstance(v, (dict, list)):
+            line[k] = v
+        elif isinstance(v, dict) and k != "kernels":
+            figures = {kk: vv for kk, vv in v.items() if isinstance(vv, (int, float))}
+            if figures:
+                line[k] = figures
+    for leg, part in (("c4_batched", "wavefront"), ("instances", "whole_frame"), ("c5_serving", "p99_within_50ms")):
+        section = out.get(leg, {}).get(part)
+        if section:
+            line[leg][part] = {kk: vv for kk, vv in section.items() if isinstance(vv, (int, float))}
+    return line
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
     ap.add_argument("--steps", type=int, default=20)
     ap.add_argument("--warmup", type=int, default=3)
     ap.add_argument("--no-cpu", action="store_true", help="skip the CPU oracle baseline")
+    ap.add_argument("--details", type=str, default="", metavar="FILE",
+                    help="also write the whole result (sweeps, per-kernel times, per-rate tables) to FILE")
     ap.add_argument("--profile-frames", type=int, default=3)
     ap.add_argument("--cpu-frames", type=int, default=3, help="oracle frames timed for the CPU baseline (median)")
     ap.add_argument("--c3-frames", type=int, default=300, help="frames of the dynamic-scene leg (0 = skip)")
@@ -576,7 +597,9 @@ def main():
         R.destroy()
         s.destroy()
     ctx.close()
-    print(json.dumps(out))
+    if args.details:
+        Path(args.details).write_text(json.dumps(out, indent=1) + "\n")
+    print(json.dumps(result_line(out)))
 
 
 def build_stage_rooflines(kernels, T, nodes):
