@@ -288,7 +288,7 @@ struct InstRoot {
 static_assert(sizeof(InstRoot) == 192, "InstRoot rows must be 16-byte aligned");
 
 // World-space box of a root for the lane-roots kernels' culling: the root
-// node's box under tr, inflated at use by k * (2 |o| + s) (k < 0: never
+// node's box under tr, inflated at use by k * (2 |o| + s) (k infinite: never
 // culled).
 struct RootBox {
     float lo[3];

@@ -2068,7 +2068,7 @@ __global__ __launch_bounds__(TB) void k_shadow_inst(const InstRoot* __restrict__
 // at most 1e4 k, so rays with k |d| >= 99 are never culled (at k >= 1 the
 // widened box holds the origin, so unit directions lose nothing by it).
 // Roots under a projective transform (bottom rows other than 0 0 0 1), or
-// with a non-finite box, get k = -1: never culled.
+// with a non-finite box, get k = inf: never culled.
 __global__ void k_root_boxes(const InstRoot* __restrict__ roots, int n, RootBox* __restrict__ out) {
     const int k = (int)(blockIdx.x * blockDim.x + threadIdx.x);
     if (k >= n) return;
@@ -2101,7 +2101,7 @@ __global__ void k_root_boxes(const InstRoot* __restrict__ roots, int n, RootBox*
         finite = finite && isfinite(b.lo[r]) && isfinite(b.hi[r]);
     }
     b.k = 1e-4f * nm * nmi;
-    if (!affine || !finite || !isfinite(b.k) || !isfinite(b.s)) b.k = -1.f;
+    if (!affine || !finite || !isfinite(b.k) || !isfinite(b.s)) b.k = INFINITY;
     out[k] = b;
 }
 
@@ -2121,23 +2121,20 @@ __device__ __forceinline__ uint64_t root_candidates(const RootBox* __restrict__ 
     for (int k = first; k < n; k += STEP) {
         const RootBox b = wb[k];
         bool meet = true;
-        if (b.k >= 0.f && b.k * md < 99.f) {
-            const float g = b.k * (2.f * mo + b.s);
-            float t0 = tmin, t1 = tmax;
+        const float g = b.k * (2.f * mo + b.s);
+        float t0 = tmin, t1 = tmax;
 #pragma unroll
-            for (int a = 0; a < 3; ++a) {
-                const float l = b.lo[a] - g, h = b.hi[a] + g;
-                if (id[a] == 0.f) {
-                    meet = meet && io[a] >= l && io[a] <= h;
-                } else {
-                    const float ta = (l - io[a]) * inv[a], tb = (h - io[a]) * inv[a];
-                    t0 = fmaxf(t0, fminf(ta, tb));
-                    t1 = fminf(t1, fmaxf(ta, tb));
-                }
+        for (int a = 0; a < 3; ++a) {
+            const float l = b.lo[a] - g, h = b.hi[a] + g;
+            if (id[a] == 0.f) {
+                meet = meet && io[a] >= l && io[a] <= h;
+            } else {
+                const float ta = (l - io[a]) * inv[a], tb = (h - io[a]) * inv[a];
+                t0 = fmaxf(t0, fminf(ta, tb));
+                t1 = fminf(t1, fmaxf(ta, tb));
             }
-            meet = meet && t0 <= t1;
         }
-        if (meet) m |= 1ull << k;
+        if ((meet && t0 <= t1) || !(b.k * md < 99.f)) m |= 1ull << k;
     }
     return m;
 }
