@@ -1,6 +1,7 @@
 // LBVH build on gfx950: prim AABB + global AABB, Morton codes, onesweep
-// radix sort, permutation of the scene buffers, level-ordered hierarchy
-// emission, bottom-up AABB refit.
+// radix sort, permutation of the scene buffers, every node of the level-ordered
+// hierarchy from its split, boxes by unions over the sorted positions, and the
+// child pairs' differences and wide records.
 //
 // Reference: BVHBuilder::build_lbvh / refit_lbvh (src/rt/bvh-builder.cpp:201-850)
 // with the kernels of src/kernel/bvh-builder.cl and bvh-builder-sort.cl.
@@ -411,10 +412,10 @@ __global__ __launch_bounds__(BS) void k_tri_records(const uint32_t* __restrict__
 //   the box of a node is the union of the triangle boxes of its range, in
 //     any order (k_boxes, k_cross).
 // A build was bound by its launches (55, a few microseconds each) and, when
-// large, by the chains of dependent reads in each level's tiles; now it has 16
-// launches and no chain longer than one search.  Whole builds, back to back,
-// before and now: 65k triangles 258 and 116 us, 8M triangles 2197 and 1601 us;
-// refit of 1M 145 and 111 us.
+// large, by the chains of dependent reads in each level's tiles; now it has 15
+// launches (of 30-bit codes) and no chain longer than one search.  Whole builds,
+// back to back, before and now, the wide records included: 65k triangles 259
+// and 103 us, 8M triangles 2198 and 1684 us; refit of 1M 145 and 123 us.
 
 // Split s of the nodes: {l, r, flags | level << 2, -}, then (k_boxes) {l, r,
 // node, children}.  Flags: bit 0 the left child is a leaf, bit 1 the right.
@@ -917,8 +918,8 @@ __global__ __launch_bounds__(BS) void k_cross(float4* __restrict__ node, TreeTil
 // the parent is at an even level, its wide record (wide.hpp), number k, one
 // slot per lane.  by_level: the tree is level-ordered and its level table gives
 // a node's level; else the level is the length of its parent chain.  Reads and
-// writes run through the arrays in order (HBM bound: 1M triangles 25 us for
-// 110 MB, 13 of them the differences alone).
+// writes run through the arrays in order (memory bound: 12 to 19 us at 1M
+// triangles, by the node count, 163 at 8M).
 __global__ __launch_bounds__(BS) void k_pairs(const float4* __restrict__ node, const uint32_t* __restrict__ parent,
                                               float4* __restrict__ delta, float4* __restrict__ wide,
                                               const uint32_t* __restrict__ levels, int by_level) {
@@ -1230,8 +1231,9 @@ int32_t rtx_lbvh_reserve(rtx_scene* s, int depth) { return lbvh_alloc(s, s->T, d
 // build scratch carved from `scratch`, a fixed array that every GPU holds for
 // the life of the process, so that it calls no allocator.  Sized for
 // RTX_LBVH_NOALLOC_MAX_TRIS triangles at any depth <= 32 (4 sort passes of
-// 8-bit digits or 8 of 4-bit digits, whose look-back words fit the same space; 33
-// levels).
+// 8-bit digits or 8 of 4-bit digits, whose look-back words fit the same space).
+// The size is the header's constant, which a program may have compiled in; the
+// parts take NA_USED of it.
 namespace {
 constexpr size_t al256(size_t b) { return (b + 255) & ~(size_t)255; }
 constexpr size_t NA_T = RTX_LBVH_NOALLOC_MAX_TRIS;

@@ -271,7 +271,7 @@ struct rtx_hits {
 // One root of a multi-root traversal: a built scene's buffers as the
 // traversal reads them, where its triangles start in the shared numbering,
 // and the object-to-world transform with its inverse (row-major 4x4, the
-// BVHRoot of include/rt/multi-bvh.hpp:9-14).  176 bytes.
+// BVHRoot of include/rt/multi-bvh.hpp:9-14).  192 bytes.
 struct InstRoot {
     const float4* node;
     const float4* delta;

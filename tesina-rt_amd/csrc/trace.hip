@@ -673,7 +673,8 @@ __device__ bool traverse_any_ns(const float4* __restrict__ node, const float4* _
 //     chunks are 64 rays).
 // Measured, WIDE_GROUP against WIDE: 720p frame over a 200k SAH tree 463
 // against 549 us, 131k scattered rays 196 against 214; batch of 12 frames 8.1
-// against 6.5 ms.
+// against 6.5 ms.  The waiting rays also cost the closest-hit form two of its 7
+// waves per SIMD, so the figures hold for the pair of both.
 //
 // Equality with the node-by-node walk.  The reference visits leaves in a
 // fixed depth-first order of the ray (near child first by
@@ -1191,7 +1192,9 @@ constexpr bool is_wide() {
 }
 // LDS of a block's walks, the type that hands it to them, and the waves per
 // SIMD that the kernel's registers have to allow (the wide walk is bound by
-// VALU issue and fetch latency: 5 and 7 waves gave 5681 and 5013 us on water).
+// VALU issue and fetch latency: 5 and 7 waves gave 5681 and 5013 us on water,
+// with WIDE_GROUP).  Of the WIDE forms, closest hit comes to 5 waves by its LDS
+// and the persistent any-hit launch keeps 7 by spilling two registers.
 template <int VAR, int TB, int SR, bool ANY>
 constexpr int walk_words() {
     return is_wide<VAR>() ? TB / RTX_WAVE * WideLds<ANY, VAR == WIDE_GROUP ? GROUP_FEED : RAY_FEED>::WORDS : (VAR == 4 ? 1 : SR * TB);
