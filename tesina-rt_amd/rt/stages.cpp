@@ -638,7 +638,7 @@ int32_t BVHBuilder::log_stages(const char* title) {
     // the reference's stage names where a kernel is that stage
     static const std::pair<const char*, const char*> named[] = {
         {"lbvh_prim_bounds", "BBox builder time"}, {"lbvh_morton", "Morton encoder time"},
-        {"lbvh_sort_pass", "Morton sorter"}, {"lbvh_refit_level", "Node bbox compute time"}};
+        {"lbvh_sort_pass", "Morton sorter"}, {"lbvh_boxes", "Node bbox compute time"}};
     Log& log = *m_log;
     log << title << "\n";
     double total = 0;
@@ -650,6 +650,12 @@ int32_t BVHBuilder::log_stages(const char* title) {
         if (kv.second.first == (b == before.end() ? 0ull : b->second.first)) continue;  // not launched
         ms[kv.first] = d;
         total += d;
+    }
+    // the boxes inside the tiles and those across them are one stage
+    const auto cross = ms.find("lbvh_cross");
+    if (cross != ms.end()) {
+        ms["lbvh_boxes"] += cross->second;
+        ms.erase(cross);
     }
     for (const auto& n : named) {
         auto it = ms.find(n.first);

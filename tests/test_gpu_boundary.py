@@ -177,7 +177,7 @@ def test_stage_tracer_overloads_and_builder_log(tmp_path):
     assert r.returncode == 0, r.stdout + r.stderr
     log = (out / "bvh.log").read_text()
     assert log.count("-----BVH construction times:") == 2, log
-    for line in ("BBox builder time:", "Morton encoder time:", "Morton sorter:", "Total:"):
+    for line in ("BBox builder time:", "Morton encoder time:", "Morton sorter:", "Node bbox compute time:", "Total:"):
         assert line in log, f"{line} missing from the builder's log:\n{log}"
     rd = {k: np.fromfile(out / f"{k}.bin", dt) for k, dt in
           (("first_t", np.float32), ("first_id", np.int32), ("copy_t", np.float32), ("copy_id", np.int32),
