@@ -185,7 +185,8 @@ uint64_t rtx_mem_in_use(rtx_ctx* ctx);
  *                    only the roots whose world-space box (the root box under
  *                    the transform, widened far beyond rounding) the ray
  *                    meets, affine roots only, 64 roots per wave-uniform
- *                    chunk; 0: the wave
+ *                    chunk (all of them for a ray so long that its walk leaves
+ *                    out an axis); 0: the wave
  *                    walks the roots one after the other, every lane waiting
  *                    for the wave's slowest walk of each root.
  *   "wf_grain":      wavefront renderer: consecutive 64-ray chunks a

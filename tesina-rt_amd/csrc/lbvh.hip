@@ -633,7 +633,7 @@ __global__ __launch_bounds__(BS) void k_ranks(uint32_t* __restrict__ rel, uint32
 
 // Triangles from which the ranks use tiles of 4096 splits instead of 1024: the
 // look-back over many tiles then costs more than a tile's longer ranking (8M
-// splits 55 against 113 us; at 65k the short tiles take 6.3 us).
+// splits 55 against 113 us; at 65k the short tiles take 6.8 us).
 constexpr uint32_t RANK_WIDE = 1u << 19;
 
 struct Box {
